@@ -18,10 +18,10 @@ from .fxkernel import num_rows, station_bytes
 class Batch:
     """Batch(nant, [(nchan, numffts, lo, bw), ...]) over gxc_batch_*.
 
-    fstage_mfma: 0 (False) keeps every subband in the multi-subband F launch;
-    1 (True) gives the subbands of 2048 points and more a launch each on the
-    matrix-core F-stage where it covers them, else the register F-stage; 2
-    gives them a launch each on the register F-stage.  autotune() chooses.
+    The subbands of 2048 points and more have an F-stage launch each:
+    fstage_mfma 1 (True) on the matrix-core F-stage (f16 operands) where it
+    covers the length, 0 (False) and 2 on a handle's default F-stage.
+    autotune() chooses.
     """
 
     def __init__(self, nant, subbands, *, precision="fp32", autos=False, exact_phase=False,

@@ -1,13 +1,59 @@
-// Per-subband F-stage launch: one workgroup per group of items (station,
-// FFT).  FFT lengths 64..8192 run fstage_item (fstage_item.hpp) at the
-// default workgroup size here, at half or double that size in
-// fstage_half.hip / fstage_double.hip; longer FFTs go to fstage_big.hip.
-#include "fstage_launch.hpp"
+// Per-subband F-stage launch.  FFT lengths 64..1024 run fstage16_item
+// (fstage16.hpp), a workgroup of 256 threads per group of items (station,
+// FFT); longer FFTs go to fstage_big.hip.
+#include "fstage16.hpp"
 
 namespace gxc {
+namespace {
 
-hipError_t launch_fstage_half(const FParams &p, int L, bool cplx, hipStream_t s);
-hipError_t launch_fstage_double(const FParams &p, int L, bool cplx, hipStream_t s);
+using namespace fs;
+
+// The workgroup sizes gxc_config.fblock names (0: not one for this length):
+// FFT blocks of L/16 threads, the default (256 threads or one block) times
+// mult / 2, as far as 1024 threads and a transform of both polarisations in
+// 160 KiB of LDS went.
+constexpr int fblock_for(int L, bool cplx, int mult) {
+  const int T = L / 16, def = T >= 256 ? T : 256, b = def * mult / 2;
+  if (b < T || b < 64 || b > 1024 || b % T) return 0;
+  const int nchan = cplx ? L : L / 2, sq = 1 << (ilog2c(nchan) / 2), s2 = cplx ? sq : 2 * sq;
+  const int slots = (b / T) * (2 * (L + L / 16) + s2 + L / s2 + sq + nchan / sq) + 16;
+  return slots * 8 > 160 * 1024 ? 0 : b;
+}
+
+// Items per workgroup of 256 threads.
+constexpr int f_ipw(int L) { return 2048 / L; }
+
+template <int L, bool CPLX, int OUT>
+__global__ void __launch_bounds__((2 * (L / 16) * f_ipw(L))) __attribute__((amdgpu_waves_per_eu(8)))
+fstage_kernel(FParams p) {
+  __shared__ __align__(16) unsigned char smem[QLds<L, CPLX, f_ipw(L)>::BYTES];
+  fstage16_item<L, CPLX, OUT, f_ipw(L)>(p, (int)xcd_order(blockIdx.x, gridDim.x), smem);
+}
+
+template <int L, bool CPLX, int OUT>
+hipError_t launch_out(const FParams &p, int items, hipStream_t s) {
+  constexpr int IPW = f_ipw(L);
+  hipLaunchKernelGGL((fstage_kernel<L, CPLX, OUT>), dim3((unsigned)((items + IPW - 1) / IPW)),
+                     dim3(2 * (L / 16) * IPW), 0, s, p);
+  return hipGetLastError();
+}
+
+template <int L, bool CPLX>
+hipError_t launch_one(const FParams &p, hipStream_t s) {
+  const long long items = (long long)p.nant * p.nt;
+  if (items <= 0) return hipSuccess;
+  if (items > 0x3fffffffLL) return hipErrorInvalidValue;
+  switch (p.out_mode) {
+    case OUT_F32: return launch_out<L, CPLX, OUT_F32>(p, (int)items, s);
+    case OUT_F16: return launch_out<L, CPLX, OUT_F16>(p, (int)items, s);
+    case OUT_BF16: return launch_out<L, CPLX, OUT_BF16>(p, (int)items, s);
+    case OUT_FP8: return launch_out<L, CPLX, OUT_FP8>(p, (int)items, s);
+    case OUT_POWER: return launch_out<L, CPLX, OUT_POWER>(p, (int)items, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace
 
 bool fstage_supported(int L, bool cplx) {
   (void)cplx;
@@ -21,10 +67,9 @@ int fstage_blocks(int L, bool cplx, int *out) {
   }
   int n = 0;
   for (int mult : {2, 1, 4}) {  // default first
-    const int b = fs::fblock_for(L, cplx, mult);
+    const int b = fblock_for(L, cplx, mult);
     if (b) out[n++] = b;
   }
-  // the register kernel of the long FFTs (fstage_big), L/32 threads
   if (L >= 2048) out[n++] = L / 32;
   return n;
 }
@@ -32,11 +77,18 @@ int fstage_blocks(int L, bool cplx, int *out) {
 hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s) {
   if (block == kFBlockMfma)
     return fstage_mfma_supported(L, cplx, p.out_mode == OUT_F32) ? launch_fstage_mfma(p, L, s) : hipErrorInvalidValue;
-  if (L > 8192 || (L >= 2048 && block == L / 32)) return launch_fstage_big(p, L, cplx, s);
-  if (block == 0 || block == fs::fblock_for(L, cplx, 2)) return fs::launch_fstage_mult<2>(p, L, cplx, s);
-  if (block == fs::fblock_for(L, cplx, 1)) return launch_fstage_half(p, L, cplx, s);
-  if (block == fs::fblock_for(L, cplx, 4)) return launch_fstage_double(p, L, cplx, s);
-  return hipErrorInvalidValue;
+  if (f_matrix(L)) return launch_fstage_big(p, L, cplx, s);
+#define GXC_F_CASE(LL) \
+  case LL: return cplx ? launch_one<LL, true>(p, s) : launch_one<LL, false>(p, s);
+  switch (L) {
+    GXC_F_CASE(64)
+    GXC_F_CASE(128)
+    GXC_F_CASE(256)
+    GXC_F_CASE(512)
+    GXC_F_CASE(1024)
+    default: return hipErrorInvalidValue;
+  }
+#undef GXC_F_CASE
 }
 
 }  // namespace gxc

@@ -1,8 +1,6 @@
-// Per-subband launch of the register/plane F-stage (fstage_big.hpp): one
-// workgroup of L/32 threads per (station, FFT) for real input up to 8192
-// points, per (station, FFT, pol) otherwise.  The only F-stage for
-// L = 16384, 32768; at L = 2048..8192 an alternative to fstage_item that the
-// autotuner weighs.
+// Per-subband launch of the F-stage of 2048 points and more (fstage_big.hpp):
+// one workgroup of L/32 threads per (station, FFT) for real input up to 8192
+// points, per (station, FFT, pol) otherwise.
 #include "fstage_big.hpp"
 
 namespace gxc {
@@ -11,18 +9,17 @@ namespace {
 using namespace fs;
 
 // For real input up to 8192 points a workgroup takes both polarisations of
-// one (station, FFT) in turn, so the delay split and the rotator tables are
-// built once for two FFTs; the two FFTs fit 128 registers (4 waves per
-// SIMD).  At 16384 and 32768 points (512 and 1024 threads), and for complex
-// input, whose two copies hold full 32-bit sample words, the second copy
-// spills, and a workgroup takes one polarisation.
+// one (station, FFT) in turn, so the delay split, the rotator tables and the
+// pass-0 matrix are built once for two FFTs.  Above, one polarisation is
+// already 512 and 1024 threads, and complex input would hold 32 registers of
+// M's operands over the first FFT.
 template <int L, bool CPLX>
 constexpr bool big_both() { return !CPLX && L <= 8192; }
 
 template <int L, bool CPLX, int OUT>
 __global__ void __launch_bounds__((BG<L, CPLX>::T)) __attribute__((amdgpu_waves_per_eu(4)))
 fstage_big_kernel(FParams p) {
-  __shared__ float2 smem[BLds<L, CPLX>::N];
+  __shared__ __align__(16) unsigned char smem[BLds<L, CPLX>::BYTES];
   // grid = nant * nt (both polarisations per workgroup) or 2 * nant * nt
   // exactly; in the second form the two polarisations of one (station,
   // FFT) are consecutive units on one XCD, so the second finds the input

@@ -1,224 +1,180 @@
-// The register/plane F-stage as a device function over one (station, FFT,
-// polarisation), shared by the per-subband launch (fstage_big.hip) and the
-// multi-subband launch (fstage_multi.hip).
-//   - L/32 threads, 32 points per thread in registers, radix-32 Stockham
-//     passes (then one smaller pass when log2 L is not a multiple of 5);
-//   - between passes the points go through LDS one component plane at a
-//     time (real parts, then imaginary parts): L floats plus one pad per 32;
-//   - the two polarisations of one (station, FFT) are neighbouring units, so
-//     the second reads the shared input words from L2.
+// The F-stage for FFT lengths 2048..32768 as a device function over one
+// (station, FFT) with its polarisations in turn (real input up to 8192
+// points) or one (station, FFT, polarisation):
+//   - L/32 threads, 32 points per thread: pass 0 (radix 32) on the matrix cores
+//     (fstage_pass0.hpp), pass 1 (radix 32) and the last pass on the VALU;
+//   - between passes the points go through LDS one component plane at a time
+//     (L words, no padding), which the samples and the matrix operands use
+//     before.
+// Small workgroups with a plane each keep four waves per SIMD from four and
+// more independent workgroups: forms with 16 points per thread and twice the
+// waves, with both polarisations side by side, and with a pipeline over items
+// in a persistent workgroup all measured 3-15 % slower at 8192 points (their
+// waves met at barriers more often and wrote as much LDS).
+// What bounds it: VALU issue and LDS writes (~80 bytes per clock and CU), each
+// about half of the time.  16 stations x 4096 channels x 4096 FFTs (FP32, 4.3
+// GB of spectra): 6.7 ms with the first pass on the VALU and both
+// polarisations in registers, 6.1 ms now; 6 stations x 1024 channels 3.3 ->
+// 2.3 ms, 10 stations x 2048 channels (BF16) 1.05 -> 0.54 ms.
 #pragma once
 
-#include "fstage_common.hpp"
+#include "fstage_pass0.hpp"
 
 namespace gxc {
 namespace fs {
 
-template <int L, bool CPLX>
+// CON_: most neighbouring butterflies of the last pass per thread
+template <int L, bool CPLX, int CON_ = 2>
 struct BG {
   using TG = TabGeom<L, CPLX>;
-  static constexpr int LG = ilog2c(L);
-  static constexpr int PT = 32;     // points per thread
-  static constexpr int T = L / PT;  // threads per item = workgroup size
-  static constexpr int N32 = LG / 5;
-  static constexpr int REM = 1 << (LG % 5);
-  static constexpr int NPASS = N32 + (REM > 1 ? 1 : 0);
-  static constexpr int radix(int p) { return p < N32 ? 32 : REM; }
-  static constexpr int ns(int p) {
-    int n = 1;
-    for (int i = 0; i < p; i++) n *= radix(i);
-    return n;
-  }
-  static constexpr int PADL = L + L / 32;
-  static_assert(L >= 2048 && L <= 32768, "register/plane F-stage covers L = 2048 .. 32768");
-  static_assert(T <= 1024, "one workgroup per FFT");
+  static constexpr int T = L / 32;  // threads, 32 points each
+  static constexpr int RL = L / 1024;            // radix of the last pass
+  static constexpr int NB = 32 / RL;             // its butterflies per thread,
+  static constexpr int CON = NB < CON_ ? NB : CON_;  // CON neighbouring ones
+  static constexpr int GRP = NB / CON;           // in each of GRP groups
+  static constexpr int KEEP = CPLX ? RL : RL / 2;  // outputs kept per butterfly
+  static_assert(f_radix(L, 0) == 32 && f_radix(L, 1) == 32 && RL >= 2, "radices 32, 32, L/1024");
+  static_assert(T >= 64 && T <= 1024 && T % TG::S2 == 0, "whole waves, one sub-rotator entry per pass-0 column");
 };
 
-__device__ __forceinline__ int padb(int i) { return i + (i >> 5); }
-
-// padb(i + k*STRIDE) - padb(i) for STRIDE a multiple of 32 (any i), or for
-// STRIDE == 1 when i is a multiple of 32 and k < 32: a compile-time offset.
-template <int STRIDE>
-__device__ __forceinline__ constexpr int padb_step(int k) {
-  return STRIDE == 1 ? k : k * (STRIDE / 32) * 33;
-}
-
-// Store one component of the outputs of pass P (Stockham order).
-template <int L, bool CPLX, int P, int COMP>
-__device__ __forceinline__ void put_plane(const float2 (&v)[32], float *s, int j) {
-  using G = BG<L, CPLX>;
-  constexpr int R = G::radix(P), NS = G::ns(P), NB = 32 / R, T = G::T;
-#pragma unroll
-  for (int bf = 0; bf < NB; bf++) {
-    const int jj = j + bf * T;
-    const int base = (jj / NS) * NS * R + (jj % NS);
-    static_assert(NS % 32 == 0 || (NS == 1 && R == 32), "compile-time padded offsets");
-    float *d = s + padb(base);
-#pragma unroll
-    for (int k = 0; k < R; k++) d[padb_step<NS>(k)] = COMP ? v[bf * R + k].y : v[bf * R + k].x;
-  }
-}
-
-// Load one component of the inputs of pass P.
-template <int L, bool CPLX, int P, int COMP>
-__device__ __forceinline__ void get_plane(float2 (&v)[32], const float *s, int j) {
-  using G = BG<L, CPLX>;
-  constexpr int R = G::radix(P), NB = 32 / R, T = G::T, STR = L / R;
-#pragma unroll
-  for (int bf = 0; bf < NB; bf++) {
-    const int jj = j + bf * T;
-    static_assert(STR % 32 == 0, "compile-time padded offsets");
-    const float *d = s + padb(jj);
-#pragma unroll
-    for (int k = 0; k < R; k++) {
-      const float x = d[padb_step<STR>(k)];
-      if (COMP)
-        v[bf * R + k].y = x;
-      else
-        v[bf * R + k].x = x;
-    }
-  }
-}
-
-// v[k] *= w^k for k = 1 .. R-1, w = W_L^m, table entry m of the byte
-// offset mb (entries m*k < L).  Only w^1 .. w^3 and w^(4 * 2^i) come from
-// the table (in L2: at 8192 points the whole table is 64 KiB, and loading
-// every twiddle cost a third of the F-stage); w^(4a) is the product of the
-// loaded powers of the bits of a and w^(4a + b) = w^(4a) w^b, at most three
-// FP32 products (a few ulps) from table entries.
-template <int R>
-__device__ __forceinline__ void twiddle_powers(float2 *v, const unsigned char *twb, unsigned mb) {
-  auto ld = [&](unsigned k) { return *reinterpret_cast<const float2 *>(twb + mb * k); };
-  float2 p[4];
-#pragma unroll
-  for (int b = 1; b < 4 && b < R; b++) {
-    p[b] = ld((unsigned)b);
-    v[b] = cmul(v[b], p[b]);
-  }
-  if constexpr (R > 4) {
-    constexpr int NQ = ilog2c(R) - 2;  // w^4, w^8, .., w^(R/2)
-    float2 q[NQ];
-#pragma unroll
-    for (int i = 0; i < NQ; i++) q[i] = ld(4u << i);
-#pragma unroll
-    for (int a = 1; 4 * a < R; a++) {
-      float2 w4 = make_float2(1.f, 0.f);
-      bool first = true;
-#pragma unroll
-      for (int i = 0; i < NQ; i++)
-        if (a & (1 << i)) {
-          w4 = first ? q[i] : cmul(w4, q[i]);
-          first = false;
-        }
-      v[4 * a] = cmul(v[4 * a], w4);
-#pragma unroll
-      for (int b = 1; b < 4; b++)
-        if (4 * a + b < R) v[4 * a + b] = cmul(v[4 * a + b], cmul(w4, p[b]));
-    }
-  }
-}
-
-// Twiddles and butterflies of pass P >= 1.
-template <int L, bool CPLX, int P>
-__device__ __forceinline__ void butterflies(float2 (&v)[32], int j, const float2 *__restrict__ tw) {
-  using G = BG<L, CPLX>;
-  constexpr int R = G::radix(P), NS = G::ns(P), NB = 32 / R, T = G::T;
-#pragma unroll
-  for (int bf = 0; bf < NB; bf++) {
-    const int jj = j + bf * T;
-    // table entry m as a 32-bit byte offset from the table's uniform base
-    const unsigned mb = (unsigned)(jj % NS) * (unsigned)(L / (NS * R)) * (unsigned)sizeof(float2);
-    twiddle_powers<R>(&v[bf * R], reinterpret_cast<const unsigned char *>(tw), mb);
-    dft<R>(&v[bf * R]);
-  }
-}
-
-// Passes P .. NPASS-1: exchange through LDS, then butterflies.
-template <int L, bool CPLX, int P>
-__device__ __forceinline__ void later_passes(float2 (&v)[32], float *s, int j, const float2 *__restrict__ tw) {
-  using G = BG<L, CPLX>;
-  if constexpr (P < G::NPASS) {
-    put_plane<L, CPLX, P - 1, 0>(v, s, j);
-    __syncthreads();
-    get_plane<L, CPLX, P, 0>(v, s, j);
-    __syncthreads();
-    put_plane<L, CPLX, P - 1, 1>(v, s, j);
-    __syncthreads();
-    get_plane<L, CPLX, P, 1>(v, s, j);
-    __syncthreads();
-    butterflies<L, CPLX, P>(v, j, tw);
-    later_passes<L, CPLX, P + 1>(v, s, j, tw);
-  }
-}
-
-// LDS of one unit: one component plane of L points (+1 pad per 32) and
-// the rotator tables, in float2 slots.
+// LDS of one unit, in bytes: a component plane of L points (and, before the
+// first exchange, the delay split, then the operands of M), the rotator
+// tables, the 2-bit level pairs and the packed samples.  At 8192 real points
+// 39.6 KB: four workgroups per CU.
 template <int L, bool CPLX>
 struct BLds {
-  static constexpr int PLANE2 = (BG<L, CPLX>::PADL + 1) / 2;  // plane, in float2 slots
-  static constexpr int N = PLANE2 + TabGeom<L, CPLX>::NTAB + 2;  // + 4-float 2-bit LUT
+  static constexpr int TAB = 4 * L;
+  static constexpr int LUT = TAB + TabGeom<L, CPLX>::NTAB * 8;
+  static constexpr int STAGE = LUT + (CPLX ? 0 : 128);
+  static constexpr int BYTES = STAGE + (CPLX ? 0 : L / 2);
+  static_assert(MatLds<CPLX>::BYTES <= 4 * L, "M's operands fit the plane");
 };
 
-// Unit u = 2 * (station + nant * FFT) + pol of one launch (BOTH false), or
-// u = station + nant * FFT with the two polarisations in turn (BOTH true:
-// the delay split, the rotator tables and the input words, which hold both
-// polarisations' samples, then serve two FFTs), on a workgroup of exactly
-// BG::T threads (every thread calls it with the same u: it contains
-// __syncthreads).  smem holds BLds::N float2 slots.
-template <int L, bool CPLX, int OUT, bool BOTH = false>
-__device__ __forceinline__ void fstage_big_item(const FParams &p, int u, float2 *smem) {
-  using G = BG<L, CPLX>;
-  using TG = typename G::TG;
-  constexpr int T = G::T, S = TG::S, S2 = TG::S2, NSTEPS = TG::NSTEPS;
-  static_assert(T % S2 == 0, "pass-0 points of one thread share one sub-rotator entry");
-  float *splane = reinterpret_cast<float *>(smem);
-  float2 *stab = smem + BLds<L, CPLX>::PLANE2;
+// One component of the points between pass 1 and the last pass.
+template <int L, bool CPLX, int COMP>
+__device__ __forceinline__ void put_plane(const float2 (&v)[32], float *s, int j) {
+  float *d = s + (j >> 5) * 1024 + (j & 31);
+#pragma unroll
+  for (int k = 0; k < 32; k++) d[32 * k] = COMP ? v[k].y : v[k].x;
+}
+// Butterfly CON j + bf of group g sits at v[(g CON + bf) RL ..]: its inputs are
+// words CON (j + g T) + bf + k L/RL, CON neighbours in one LDS read.
+template <int L, bool CPLX, int CON_, int COMP>
+__device__ __forceinline__ void get_plane(float2 (&v)[32], const float *s, int j) {
+  using G = BG<L, CPLX, CON_>;
+  constexpr int CON = G::CON, RL = G::RL;
+  typedef float row __attribute__((ext_vector_type(CON)));
+#pragma unroll
+  for (int g = 0; g < G::GRP; g++)
+#pragma unroll
+    for (int k = 0; k < RL; k++) {
+      const row x = *reinterpret_cast<const row *>(s + CON * (j + g * G::T) + k * (L / RL));
+#pragma unroll
+      for (int bf = 0; bf < CON; bf++) {
+        float2 &d = v[(g * CON + bf) * RL + k];
+        if (COMP)
+          d.y = x[bf];
+        else
+          d.x = x[bf];
+      }
+    }
+}
 
-  const int j = threadIdx.x;
+// Last pass, butterflies I ..: twiddles, DFT, fractional-sample rotation of the
+// kept outputs, which replace the butterfly's first ones.  w holds the powers
+// of W_L^(CON j); butterfly CON j + bf + CON T g takes them times a constant.
+template <int L, bool CPLX, int CON_, int I = 0>
+__device__ __forceinline__ void last_butterflies(float2 (&v)[32], const Powers &w) {
+  using G = BG<L, CPLX, CON_>;
+  constexpr int CON = G::CON, RL = G::RL;
+  if constexpr (I < G::NB) {
+    constexpr int M = I % CON + CON * G::T * (I / CON);
+    float2 *x = &v[I * RL];
+    if constexpr (RL == 2) {
+      x[1] = cmul(x[1], twc<L, M % L>(w.p1));
+    } else {
+      Powers u;
+      u.p1 = twc<L, M % L>(w.p1);
+      u.p2 = twc<L, 2 * M % L>(w.p2);
+      u.p3 = twc<L, 3 * M % L>(w.p3);
+      u.q0 = twc<L, 4 * M % L>(w.q0);
+      u.q1 = twc<L, 8 * M % L>(w.q1);
+      u.q2 = twc<L, 16 * M % L>(w.q2);
+      times_powers<RL, 0>(x, u);
+    }
+    dft<RL>(x);
+    last_butterflies<L, CPLX, CON_, I + 1>(v, w);
+  }
+}
+
+// Unit u = station + nant * FFT (BOTH) or 2 * that + pol, on a workgroup of
+// exactly BG::T threads (every thread calls it with the same u: it contains
+// __syncthreads).  smem holds BLds::BYTES bytes, 16-byte aligned.
+template <int L, bool CPLX, int OUT, bool BOTH>
+__device__ __forceinline__ void fstage_big_item(const FParams &p, int u, unsigned char *smem) {
+  // Neighbouring bins of a thread: 16 bytes, so that a wave's store covers whole
+  // lines (four FP32 bins as two stores of 16 bytes, 32 apart per lane, took
+  // 6.8 ms instead of 6.1 at 8192 points; 16-bit bins gain 5 % from two to four).
+  constexpr int CON_ = out_bytes(OUT) == 8 ? 2 : 4;
+  using G = BG<L, CPLX, CON_>;
+  using TG = typename G::TG;
+  using LD = BLds<L, CPLX>;
+  constexpr int T = G::T, S = TG::S, S2 = TG::S2, NSTEPS = TG::NSTEPS, NCHAN = TG::NCHAN, TR = T / 32;
+  constexpr int CON = G::CON, RL = G::RL;
+  static_assert(!BOTH || !CPLX, "both polarisations in turn: 2-bit samples");
+  float *splane = reinterpret_cast<float *>(smem);
+  float2 *stab = reinterpret_cast<float2 *>(smem + LD::TAB);
+  uint2 *slut = reinterpret_cast<uint2 *>(smem + LD::LUT);
+  uint32_t *stage = reinterpret_cast<uint32_t *>(smem + LD::STAGE);
+
+  const int tid = threadIdx.x;
   const int pol0 = BOTH ? 0 : u & 1;
   const int item = BOTH ? u : u >> 1;
   const int tl = item / p.nant;
   const int st = item % p.nant;
   const int t = p.t0 + tl * p.tstride;
-  const size_t row0 = ((size_t)tl * p.nant + st) * 2;  // output row of pol 0
+  constexpr unsigned EB = out_bytes(OUT);
+  unsigned char *out = out_base<OUT>(p) + ((size_t)item * 2 + pol0) * (NCHAN * EB);
 
-  int offset = 0;
-  double frac = 0.0, a = 0.0, b = 0.0;
+  // The delay split (two FP64 divisions) on one wave; the others wait for it
+  // at the barrier and leave the VALU to the other workgroups of the CU.
+  struct Split {
+    double frac, a, b;
+    int offset, valid;
+  };
+  Split *ssplit = reinterpret_cast<Split *>(smem);
+  if (T <= 64 || tid < 64) {
+    Split w{0.0, 0.0, 0.0, 0, 0};
+    w.valid = split_offset<L>(p, st, t, w.offset, w.frac, w.a, w.b) ? 1 : 0;
+    if (tid == 0) {
+      *ssplit = w;
+      if (pol0 == 0 && OUT != OUT_POWER) p.valid[(size_t)st * p.numffts + t] = w.valid;
+    }
+  }
+  __syncthreads();
   // The same for every thread of the workgroup: the branches below that
   // depend on it are uniform, so every __syncthreads is reached by all.
-  const bool valid = split_offset<L>(p, st, t, offset, frac, a, b);
-  if (j == 0 && pol0 == 0 && OUT != OUT_POWER) p.valid[(size_t)st * p.numffts + t] = valid ? 1 : 0;
+  const int offset = __builtin_amdgcn_readfirstlane(ssplit->offset);
+  const bool valid = __builtin_amdgcn_readfirstlane(ssplit->valid) != 0;
+  const double frac = ssplit->frac, a = ssplit->a, b = ssplit->b;
   if (!valid) {
-    for (int pol = pol0; pol < (BOTH ? 2 : pol0 + 1); pol++)
-      for (int q = j; q < TG::NCHAN; q += T)
-        store_bin<OUT, TG::NCHAN>(p, row0 + pol, 2 * st + pol, q, make_float2(0.f, 0.f));
+    for (unsigned q = tid; q < (BOTH ? 2 : 1) * NCHAN; q += T) store_val<OUT>(out + q * EB, make_float2(0.f, 0.f), 1.f);
     return;
   }
-  // This thread's pass-0 input words, requested before the table build so
-  // that their latency overlaps it: complex 8-bit [Are, Aim, Bre, Bim] as
-  // one 32-bit word per sample; 2-bit as the aligned word that holds the
-  // sample's byte (byte layout [A_t, B_t, A_t+1, B_t+1], fxkernel.cpp:443-476).  Pass-0 point k
-  // of thread j is window sample n = j + k*T, packed sample offset + n.
-  gbyte *src = (gbyte *)p.station[st];
-  const int s0 = offset + j;
-  int rawin[32];
-  // T is even, so every k shares the nibble parity of s0.  Each byte comes
-  // in its aligned 32-bit word (never past the page of a valid byte): the
-  // field extract below then needs no byte mask, one VALU less per sample.
-  gint *wsrc = CPLX ? reinterpret_cast<gint *>(src + 4 * (size_t)s0)
-                    : (gint *)((uintptr_t)(src + (s0 >> 1)) & ~(uintptr_t)3);
-  constexpr int WSTRIDE = CPLX ? T : T / 8;  // words between points k and k+1
-  auto load_words = [&]() {
-#pragma unroll
-    for (int k = 0; k < 32; k++) rawin[k] = wsrc[(size_t)k * WSTRIDE];
-  };
-  load_words();
-  fill_tables<L, CPLX>(p, frac, a, b, stab, j, T);
-  // 2-bit levels by code (fxkernel.cpp:15-28): an LDS read replaces the
-  // compare/select chain that would otherwise cost ~6 VALU per sample
-  float *lut = reinterpret_cast<float *>(stab + TabGeom<L, CPLX>::NTAB);
-  if (!CPLX && j < 4) lut[j] = j == 0 ? -kHiMag : j == 1 ? -1.0f : j == 2 ? 1.0f : kHiMag;
+  Pass0In<L, CPLX, true, 4> in;
+  in.template load<T>((gbyte *)p.station[st], offset, tid, tid);
+  fill_tables<L, CPLX>(p, frac, a, b, stab, tid, T, pass0_unscale<CPLX>());
+  if (!CPLX && tid < 16) slut[tid] = level_pair(tid);
+  in.template put<T>(stage, tid);
   __syncthreads();
+  build_matrix<CPLX, T>(smem, stab + S2, T / S2, p.twiddle, tid);
+  __syncthreads();
+  // M's operands for both polarisations (2-bit input: 16 registers)
+  uint4 am[2][2];
+  if constexpr (BOTH) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) am[i >> 1][i & 1] = reinterpret_cast<const uint4 *>(smem)[64 * i + (tid & 63)];
+  }
 
   auto one_pol = [&](const int pol) {
     // An opaque copy of the thread index (and an opaque zero offset) in
@@ -234,64 +190,81 @@ __device__ __forceinline__ void fstage_big_item(const FParams &p, int u, float2 
     const float2 *fstep = fsub + S;
     const float2 *__restrict__ tw = p.twiddle + z;
 
-    // Pass-0 point k of thread j is window sample n = j + k*T: its rotator
-    // is sub[n % S2] * step[n / S2] (fxkernel.cpp:553-558) = sub[j % S2] *
-    // step[j / S2 + k*T/S2].
-    const float2 rsub = sub[j % S2];
-    const size_t row = row0 + pol;
+    // ---- pass 0: columns j0 + tile of lane (c, g) ----
+    const int c = j & 15, g = (j >> 4) & 3, j0 = (j & ~63) + 4 * c;
+    floatx4 acc[4][2][2];
+    in.fetch(stage + z, j);
+    if constexpr (BOTH)
+      in.matmul(acc, am, slut + z, pol);
+    else
+      in.matmul(acc, smem, slut + z, pol);
+    finish_columns<L, CPLX, 4>(acc, sub, step, tw, j0, g);
+    __syncthreads();  // M's operands (the last polarisation's points) are read
+    // Exchange to pass 1, one component at a time: point 32 jj + r, in rows
+    // of 8 chunks of 4 points at chunk position (r / 4) ^ (jj / 4 mod 8).
+    // Eight neighbouring lanes of a 16-byte store then cover the 32 banks
+    // once, and so do 32 lanes of a pass-1 load.
     float2 v[32];
-    if constexpr (CPLX) {
-      const int sh = 16 * pol;
+    {
+      const int r = j & 31, jr = j >> 5;
+      const int b0 = 32 * jr + 4 * ((r >> 2) ^ ((jr >> 2) & 7)) + (r & 3);
 #pragma unroll
-      for (int k = 0; k < 32; k++) {
-        const int wv = rawin[k];
-        const float re = (float)(int8_t)((wv >> sh) & 0xff), im = (float)(int8_t)((wv >> (sh + 8)) & 0xff);
-        v[k] = cmul(cmul(rsub, step[j / S2 + k * (T / S2)]), make_float2(re, im));
-      }
-    } else {
-      // sample s is nibble s&1 of its byte, the byte (address & 3) of its
-      // word; pol A in the nibble's low 2 bits
-      const int sh = 8 * (int)((uintptr_t)(src + (s0 >> 1)) & 3) + (s0 & 1) * 4 + 2 * pol;
+      for (int comp = 0; comp < 2; comp++) {
 #pragma unroll
-      for (int k = 0; k < 32; k++) {
-        const int code = (int)__builtin_amdgcn_ubfe((unsigned)rawin[k], (unsigned)sh, 2u);
-        const float x = lut[code];
-        const float2 r = cmul(rsub, step[j / S2 + k * (T / S2)]);
-        v[k] = make_float2(x * r.x, x * r.y);
+        for (int e = 0; e < 4; e++)
+#pragma unroll
+          for (int rh = 0; rh < 2; rh++)
+            *reinterpret_cast<floatx4 *>(splane + 32 * (j0 + e) + 4 * ((g ^ (c & 7)) ^ (4 * rh))) = acc[e][rh][comp];
+        __syncthreads();
+#pragma unroll
+        for (int k = 0; k < 32; k++) {
+          const float x = splane[(b0 ^ (4 * (((k * TR) >> 2) & 7))) + k * T];
+          if (comp)
+            v[k].y = x;
+          else
+            v[k].x = x;
+        }
+        __syncthreads();
       }
     }
-#pragma unroll
-    for (int bf = 0; bf < 32 / G::radix(0); bf++) dft<G::radix(0)>(&v[bf * G::radix(0)]);
-    later_passes<L, CPLX, 1>(v, splane, j, tw);
+    // ---- pass 1 and the last pass ----
+    dft<32>(v);
+    put_plane<L, CPLX, 0>(v, splane, j);
+    __syncthreads();
+    get_plane<L, CPLX, CON_, 0>(v, splane, j);
+    __syncthreads();
+    put_plane<L, CPLX, 1>(v, splane, j);
+    __syncthreads();
+    get_plane<L, CPLX, CON_, 1>(v, splane, j);
+    constexpr int TWS = f_tw_step(L, 2);
+    static_assert(CON % TWS == 0 || CON == 1, "the first butterfly's powers are in the table");
+    last_butterflies<L, CPLX, CON_>(v, load_powers<RL, f_tw_entries(L, 2), f_tw_off(L, 2)>(tw, (unsigned)j * (CON / TWS)));
 
-    // last pass outputs: bins q = jj + k*(L/R), keep q < nchan
-    constexpr int PL = G::NPASS - 1;
-    constexpr int R = G::radix(PL), NB = 32 / R;
-    constexpr int KEEP = CPLX ? R : R / 2;
+    // outputs: bins q = CON (j + g T) + bf + k L/RL, q < nchan, CON neighbours
+    // of a thread in one store
 #pragma unroll
-    for (int bf = 0; bf < NB; bf++) {
-      const int jj = j + bf * T;
+    for (int gr = 0; gr < G::GRP; gr++)
 #pragma unroll
-      for (int k = 0; k < KEEP; k++) {
-        const int q = jj + k * (L / R);
-        // q % S = j % S and q / S = j / S + a compile-time step when S
-        // divides T and L/R, which keeps the table offsets out of the VALU
-        const float2 fr = (T % S == 0 && (L / R) % S == 0)
-                              ? cmul(fsub[j % S], fstep[j / S + (bf * T + k * (L / R)) / S])
-                              : cmul(fsub[q % S], fstep[q / S]);  // fracsamprotator, fxkernel.cpp:614-625
-        store_bin<OUT, TG::NCHAN>(p, row, 2 * st + pol, q, cmul(fr, v[bf * R + k]));
+      for (int k = 0; k < G::KEEP; k++) {
+        // q / S = CON j / S + a compile-time step: S divides CON T and L/RL,
+        // CON divides S
+        static_assert((CON * T) % S == 0 && (L / RL) % S == 0 && S % CON == 0, "table offsets");
+        const int step0 = (CON * T * gr + k * (L / RL)) / S;
+        const float2 fs = fstep[CON * j / S + step0];
+        const unsigned q = (unsigned)(CON * j) + CON * T * gr + k * (L / RL);
+        float2 y[CON];
+        float sc[CON];
+#pragma unroll
+        for (int bf = 0; bf < CON; bf++) {
+          const float2 fr = cmul(fsub[(CON * j) % S + bf], fs);  // fracsamprotator, fxkernel.cpp:614-625
+          y[bf] = cmul(fr, v[(gr * CON + bf) * RL + k]);
+          sc[bf] = bin_scale<OUT, NCHAN>(p, 2 * st + pol, q + bf);
+        }
+        store_row<OUT, CON>(out + ((unsigned)(BOTH ? pol : 0) * (NCHAN * EB) + q * EB), y, sc);
       }
-    }
   };
   one_pol(pol0);
-  if constexpr (BOTH) {
-    // the second polarisation reads its words again (from L2): keeping
-    // them in registers over the first FFT would cost occupancy.  The last
-    // pass of the first FFT read the plane before a barrier, so this FFT's
-    // first plane store is safe.
-    load_words();
-    one_pol(1);
-  }
+  if constexpr (BOTH) one_pol(1);
 }
 
 }  // namespace fs

@@ -1,6 +1,6 @@
-// Device helpers shared by the F-stage kernels: fstage_item.hpp (FFT held in
-// LDS with both polarisations, L <= 8192) and fstage_big.hpp (one
-// polarisation per workgroup, L = 2048..32768).
+// Device helpers shared by the F-stage kernels: fstage16.hpp (16 points per
+// thread, L = 64..1024), fstage_big.hpp (32 points per thread, L =
+// 2048..32768) and fstage_mfma.hip (all passes on the matrix cores).
 #pragma once
 
 #include "gxc_internal.hpp"
@@ -240,50 +240,49 @@ __device__ __forceinline__ bool split_offset(const FParams &p, int st, int t, in
 
 // Entries e = e0, e0+estep, ... of one item's rotator tables: sub, step
 // (fringe rotation, fxkernel.cpp:498-567) and fsub, fstep (fractional-sample
-// correction, fxkernel.cpp:595-634).  Phases in FP64, reduced, rounded to
-// FP32, then the hardware sine/cosine (v_sin_f32/v_cos_f32 via __sincosf).
-// Every argument is already reduced: the fringe phases to (-2 pi, 0], the
-// fractional-sample phases to |2 pi c bw/nchan * frac| < 2 pi (|frac| is at
-// most a sample), where the hardware result is within ~5e-7 of libm
-// sincosf (the 2^-24 rounding of x/2 pi times 2 pi, plus the unit's own
-// error); IPP's ippsSinCos_32f_A11, which fxkernel uses, is itself only
-// ~11-bit accurate.
+// correction, fxkernel.cpp:595-634), the fsub entries multiplied by fscale (a
+// power of two).  Phases in FP64 turns, reduced to half a turn, rounded to
+// FP32 (at most 9e-8 rad), then sincospif.  (Phases rounded to FP32 in
+// radians and the hardware sine and cosine, within ~5e-7, had been the largest
+// part of the FP32 path's error: against FP64, 16 stations x 4096 channels,
+// 6.2e-7 -> 3.8e-7 with 1 % more time in the F-stage.)
+// Entry e of one item's tables.
 template <int L, bool CPLX>
-__device__ __forceinline__ void fill_tables(const FParams &p, double frac, double a, double b, float2 *tab,
-                                            int e0, int estep) {
+__device__ __forceinline__ float2 table_entry(const FParams &p, double frac, double a, double b, int e, float fscale) {
 #pragma clang fp contract(off)
   using TG = TabGeom<L, CPLX>;
   constexpr int S = TG::S, S2 = TG::S2, NSTEPS = TG::NSTEPS;
-  // fxkernel.cpp:503-505: remove whole seconds of delay.
-  const double intdelay = trunc(b);
-  const double bf = b - intdelay;
-  const float ffrac = (float)frac;  // ippsMulC_32f takes an Ipp32f (fxkernel.cpp:600)
-  for (int e = e0; e < TG::NTAB; e += estep) {
-    float sn, cs;
-    if (e < S2) {
-      // subphase, fxkernel.cpp:107,508,514,519,525-530,535
-      double ph = ((double)e / (double)L) * a;
-      ph = ph + bf;
-      ph = ph * p.lo;
-      if (p.fraclo) ph = ph + p.lofrac * intdelay;
-      const double arg = (-2.0 * kPi) * (ph - trunc(ph));
-      __sincosf((float)arg, &sn, &cs);
-    } else if (e < S2 + NSTEPS) {
-      // stepphase, fxkernel.cpp:112,511,522,539
-      const int i = e - S2;
-      double ph = ((double)(i * p.stepmul) / (double)L) * a;
-      ph = ph * p.lo;
-      const double arg = (-2.0 * kPi) * (ph - trunc(ph));
-      __sincosf((float)arg, &sn, &cs);
-    } else if (e < S2 + NSTEPS + S) {
-      // fxkernel.cpp:600,608
-      __sincosf(p.subchanfreq[e - S2 - NSTEPS] * ffrac, &sn, &cs);
-    } else {
-      // fxkernel.cpp:603,611
-      __sincosf(p.stepchanfreq[e - S2 - NSTEPS - S] * ffrac, &sn, &cs);
-    }
-    tab[e] = make_float2(cs, sn);
+  double ph;
+  if (e < S2) {
+    // subphase, fxkernel.cpp:107,508,514,519,525-530,535; whole seconds of
+    // delay removed (fxkernel.cpp:503-505)
+    const double intdelay = trunc(b);
+    ph = ((double)e / (double)L) * a;
+    ph = ph + (b - intdelay);
+    ph = ph * p.lo;
+    if (p.fraclo) ph = ph + p.lofrac * intdelay;
+    ph = -ph;
+  } else if (e < S2 + NSTEPS) {
+    // stepphase, fxkernel.cpp:112,511,522,539
+    const int i = e - S2;
+    ph = ((double)(i * p.stepmul) / (double)L) * a;
+    ph = -(ph * p.lo);
+  } else {
+    // channel c turns by c bw/nchan frac (fxkernel.cpp:600-611): in samples,
+    // frac / (sampletime L) per channel
+    const int i = e - S2 - NSTEPS;
+    ph = (frac * p.samplerate) * (1.0 / (double)L) * (double)(i < S ? i : (i - S) * S);
   }
+  float sn, cs;
+  sincospif((float)(2.0 * (ph - rint(ph))), &sn, &cs);
+  const float sc = e >= S2 + NSTEPS && e < S2 + NSTEPS + S ? fscale : 1.f;
+  return make_float2(cs * sc, sn * sc);
+}
+
+template <int L, bool CPLX>
+__device__ __forceinline__ void fill_tables(const FParams &p, double frac, double a, double b, float2 *tab,
+                                            int e0, int estep, float fscale = 1.f) {
+  for (int e = e0; e < TabGeom<L, CPLX>::NTAB; e += estep) tab[e] = table_entry<L, CPLX>(p, frac, a, b, e, fscale);
 }
 
 __device__ __forceinline__ uint32_t pack_f16(float re, float im) {
@@ -314,12 +313,25 @@ __device__ __forceinline__ float bin_scale(const FParams &p, int srow, int q) {
   if constexpr (OUT == OUT_F32 || OUT == OUT_POWER) {
     return 1.f;
   } else {
-    return p.scales[(size_t)srow * NCHAN + q];
+    return *reinterpret_cast<const float *>(reinterpret_cast<const unsigned char *>(p.scales + (size_t)srow * NCHAN) +
+                                            (unsigned)q * 4u);
   }
 }
 
-// Store bin q of output row `row` (= 2*station + pol within FFT row block)
-// in the spectra format OUT, with its scale sc = bin_scale(...) already read.
+// Bytes of one stored bin, and where the launch's output starts.
+constexpr unsigned out_bytes(int out) {
+  return out == OUT_F32 ? 8 : out == OUT_FP8 ? 2 : 4;
+}
+template <int OUT>
+__device__ __forceinline__ unsigned char *out_base(const FParams &p) {
+  return static_cast<unsigned char *>(OUT == OUT_F32     ? static_cast<void *>(p.spectra)
+                                      : OUT == OUT_POWER ? static_cast<void *>(p.power)
+                                                         : p.out);
+}
+
+// Store one bin at d in the spectra format OUT, with its scale sc =
+// bin_scale(...) already read.  (Callers form d as a uniform base plus a 32-bit
+// byte offset: the store then takes the base from scalar registers.)
 // The spectra are written once and read once, by the X-stage after the
 // whole F-stage: streaming (nontemporal) stores of the 4- and 8-byte
 // values, so that the X-stage no longer meets the write-back of dirty
@@ -327,23 +339,62 @@ __device__ __forceinline__ float bin_scale(const FParams &p, int srow, int q) {
 // -> 2.78 ms, FP32 F-stage -0.8 %).  The 2-byte FP8 values keep ordinary
 // stores, which the caches combine (as streaming stores the 16-station FP8
 // F-stage measured 2-5 % slower).
-template <int OUT, int NCHAN>
-__device__ __forceinline__ void store_bin_sc(const FParams &p, size_t row, int q, float2 y, float sc) {
+template <int OUT>
+__device__ __forceinline__ void store_val(unsigned char *d, float2 y, float sc) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
   if constexpr (OUT == OUT_F32) {
     const f32x2 v = {y.x, y.y};
-    __builtin_nontemporal_store(v, reinterpret_cast<f32x2 *>(p.spectra + row * NCHAN + q));
+    __builtin_nontemporal_store(v, reinterpret_cast<f32x2 *>(d));
   } else if constexpr (OUT == OUT_POWER) {
     // one row per sampled FFT; the scale kernel sums rows in a fixed order,
     // so the scales do not depend on scheduling
-    p.power[row * NCHAN + q] = y.x * y.x + y.y * y.y;
+    *reinterpret_cast<float *>(d) = y.x * y.x + y.y * y.y;
   } else if constexpr (OUT == OUT_FP8) {
-    static_cast<uint16_t *>(p.out)[row * NCHAN + q] = pack_fp8(y.x * sc, y.y * sc);
+    *reinterpret_cast<uint16_t *>(d) = pack_fp8(y.x * sc, y.y * sc);
   } else if constexpr (OUT == OUT_F16) {
-    __builtin_nontemporal_store(pack_f16(y.x * sc, y.y * sc), static_cast<uint32_t *>(p.out) + row * NCHAN + q);
+    __builtin_nontemporal_store(pack_f16(y.x * sc, y.y * sc), reinterpret_cast<uint32_t *>(d));
   } else {
-    __builtin_nontemporal_store(pack_bf16(y.x * sc, y.y * sc), static_cast<uint32_t *>(p.out) + row * NCHAN + q);
+    __builtin_nontemporal_store(pack_bf16(y.x * sc, y.y * sc), reinterpret_cast<uint32_t *>(d));
   }
+}
+
+// Store CON neighbouring bins at d (CON * the bin's bytes aligned) in one store
+// (FP32: one per two bins).
+template <int OUT, int CON>
+__device__ __forceinline__ void store_row(unsigned char *d, const float2 (&y)[CON], const float (&sc)[CON]) {
+  typedef float f32x4 __attribute__((ext_vector_type(4)));
+  if constexpr (CON == 1) {
+    store_val<OUT>(d, y[0], sc[0]);
+  } else if constexpr (OUT == OUT_F32) {
+#pragma unroll
+    for (int i = 0; i < CON; i += 2)
+      __builtin_nontemporal_store((f32x4){y[i].x, y[i].y, y[i + 1].x, y[i + 1].y}, reinterpret_cast<f32x4 *>(d + 8 * i));
+  } else if constexpr (OUT == OUT_POWER) {
+    typedef float row __attribute__((ext_vector_type(CON)));
+    row r;
+#pragma unroll
+    for (int i = 0; i < CON; i++) r[i] = y[i].x * y[i].x + y[i].y * y[i].y;
+    *reinterpret_cast<row *>(d) = r;
+  } else if constexpr (OUT == OUT_FP8) {
+    typedef uint16_t row __attribute__((ext_vector_type(CON)));
+    row r;
+#pragma unroll
+    for (int i = 0; i < CON; i++) r[i] = pack_fp8(y[i].x * sc[i], y[i].y * sc[i]);
+    *reinterpret_cast<row *>(d) = r;
+  } else {
+    typedef uint32_t row __attribute__((ext_vector_type(CON)));
+    row r;
+#pragma unroll
+    for (int i = 0; i < CON; i++)
+      r[i] = OUT == OUT_F16 ? pack_f16(y[i].x * sc[i], y[i].y * sc[i]) : pack_bf16(y[i].x * sc[i], y[i].y * sc[i]);
+    __builtin_nontemporal_store(r, reinterpret_cast<row *>(d));
+  }
+}
+
+// Store bin q of output row `row` (= 2*station + pol within FFT row block).
+template <int OUT, int NCHAN>
+__device__ __forceinline__ void store_bin_sc(const FParams &p, size_t row, int q, float2 y, float sc) {
+  store_val<OUT>(out_base<OUT>(p) + row * (NCHAN * out_bytes(OUT)) + (unsigned)q * out_bytes(OUT), y, sc);
 }
 
 // Store bin q of output row `row`; `srow` is the input index 2*station+pol.

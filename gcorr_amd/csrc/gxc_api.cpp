@@ -96,6 +96,7 @@ gxc_status run_fstage(gxc_handle *h, int t0, int nt, int mode, void *out, int ts
   p.lofrac = lo - std::trunc(lo);
   p.fraclo = (lo - std::trunc(lo)) > 0.00000000001 ? 1 : 0;  // TINY, fxkernel.cpp:66-71
   p.sampletime = h->d.sampletime;
+  p.samplerate = 1.0 / p.sampletime;
   GXC_HIP(h, gxc::launch_fstage(p, h->d.L, h->cfg.is_complex != 0, h->fblock, s));
   return GXC_OK;
 }

@@ -6,7 +6,8 @@
 //   [reduced precision: power pass over 64 sampled FFTs of every subband
 //    (one launch), power-of-two scales (one launch)]
 //   for each chunk c (1/chunks of every subband's FFTs):
-//     F-stage of all subbands (one launch) -> spectra buffer c % 2
+//     F-stage of the subbands below 2048 points (one launch) and of each
+//     longer one -> spectra buffer c % 2
 //     X-stage of all subbands (one launch), accumulating split partials
 //   row counts (one launch), finalise (one launch)
 // The launches read segment tables built once at gxc_batch_create: one
@@ -70,7 +71,7 @@ struct gxc_batch {
   gxc_batch_config cfg{};
   std::vector<Sub> sub;
   std::string err;
-  int device = 0, out_mode = 0, M = 0, nrows = 0, nchunks = 1, nbuf = 1, fblock = 256;
+  int device = 0, out_mode = 0, M = 0, nrows = 0, nchunks = 1, nbuf = 1;
   int maxL = 0, xunits = 2048;  // longest FFT; X units per launch the splits aim at
   hipStream_t stream = nullptr, xstream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_f[2] = {nullptr, nullptr}, ev_x[2] = {nullptr, nullptr};
@@ -80,7 +81,8 @@ struct gxc_batch {
   // segment tables and unit totals
   gxc::FSeg *d_fseg = nullptr;  // [nchunks][nmulti]: subbands of the multi-subband F launch
   int nmulti = 0;
-  std::vector<std::vector<gxc::FSeg>> mseg;  // [nchunks]: subbands on the matrix-core F-stage
+  std::vector<std::vector<gxc::FSeg>> mseg;  // [nchunks]: subbands with launches of their own
+  std::vector<gxc::FSeg> mpow;               // the same subbands' power pass
   gxc::XSeg *d_xseg = nullptr;  // [nchunks][nsub]
   gxc::FSeg *d_powseg = nullptr;
   gxc::ScaleSeg *d_scaleseg = nullptr;
@@ -174,6 +176,7 @@ gxc::FParams fparams(const gxc_batch *b, const Sub &u, int t0, int nt, int tstri
   p.lofrac = lo - std::trunc(lo);
   p.fraclo = (lo - std::trunc(lo)) > 0.00000000001 ? 1 : 0;  // TINY, fxkernel.cpp:66-71
   p.sampletime = u.d.sampletime;
+  p.samplerate = 1.0 / p.sampletime;
   p.frame_ok = u.vdif ? u.vs.d_flag_ptrs : nullptr;
   p.frame_samples = u.vs.d_spf;
   return p;
@@ -197,12 +200,15 @@ gxc_status build_tables(gxc_batch *b) {
   b->d_scaleseg = nullptr;
   const int ns = (int)b->sub.size(), C = b->nchunks;
   const int ct = gxc::xm_channels_per_group(b->M, b->out_mode);
-  // with fstage_mfma, the subbands of 2048 points and more get launches of
-  // their own: on the matrix cores where those cover them, else on the
-  // register kernel (fstage_mfma 1), or all on the register kernel (2)
-  auto on_mfma = [&](const Sub &u) { return b->cfg.fstage_mfma != 0 && u.d.L >= 2048; };
+  // The subbands of 2048 points and more get launches of their own: their
+  // kernel holds 32 points per thread and one length's LDS per workgroup, and
+  // in one persistent launch with the shorter lengths every workgroup would
+  // take the largest length's (8 subbands of 512..8192 points, FP32, 0.25 s:
+  // F-stage 12.4 -> 6.6 ms).  fstage_mfma 1 runs them with f16 operands in
+  // every pass where that form covers the length.
+  auto own_launch = [&](const Sub &u) { return u.d.L >= 2048; };
   b->nmulti = 0;
-  for (const Sub &u : b->sub) b->nmulti += on_mfma(u) ? 0 : 1;
+  for (const Sub &u : b->sub) b->nmulti += own_launch(u) ? 0 : 1;
   b->mseg.assign(C, {});
   std::vector<gxc::FSeg> fseg((size_t)C * std::max(1, b->nmulti));
   std::vector<gxc::XSeg> xseg((size_t)C * ns);
@@ -219,12 +225,12 @@ gxc_status build_tables(gxc_batch *b) {
       gxc::FSeg f;
       f.p = fparams(b, u, t0, nt, 1, b->out_mode, spec);
       f.L = u.d.L;
-      if (on_mfma(u)) {
+      if (own_launch(u)) {
         f.unit0 = 0;
         b->mseg[c].push_back(f);
       } else {
         f.unit0 = fu;
-        fu += gxc::fstage_multi_units(u.d.L, b->fblock, (long long)b->cfg.nant * nt);
+        fu += gxc::fstage_multi_units(u.d.L, (long long)b->cfg.nant * nt);
         fseg[(size_t)c * b->nmulti + m++] = f;
       }
       gxc::XSeg &x = xseg[(size_t)c * ns + s];
@@ -277,15 +283,23 @@ gxc_status build_tables(gxc_batch *b) {
   GXB_TRY(upload(b, &b->d_finseg, finseg));
 
   if (b->out_mode != gxc::OUT_F32) {
-    std::vector<gxc::FSeg> pseg(ns);
+    std::vector<gxc::FSeg> pseg;
     std::vector<gxc::ScaleSeg> sseg(ns);
     long long pu = 0, su = 0;
+    b->mpow.clear();
     for (int s = 0; s < ns; s++) {
       const Sub &u = b->sub[s];
-      pseg[s].p = fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr);
-      pseg[s].L = u.d.L;
-      pseg[s].unit0 = pu;
-      pu += gxc::fstage_multi_units(u.d.L, b->fblock, (long long)b->cfg.nant * u.npow);
+      gxc::FSeg f;
+      f.p = fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr);
+      f.L = u.d.L;
+      f.unit0 = 0;
+      if (own_launch(u)) {
+        b->mpow.push_back(f);
+      } else {
+        f.unit0 = pu;
+        pu += gxc::fstage_multi_units(u.d.L, (long long)b->cfg.nant * u.npow);
+        pseg.push_back(f);
+      }
       sseg[s].scales = u.d_scales;
       sseg[s].power = u.d_power;
       sseg[s].n = b->M * u.cfg.nchan;
@@ -335,7 +349,9 @@ gxc_status enqueue_device_work(gxc_batch *b) {
   const bool overlap = b->nbuf == 2;
   hipStream_t fs = b->stream, xs = overlap ? b->xstream : b->stream;
   if (b->out_mode != gxc::OUT_F32) {
-    GXB_HIP(b, gxc::launch_fstage_multi(b->d_powseg, ns, b->powtotal, gxc::OUT_POWER, b->fblock, fs));
+    GXB_HIP(b, gxc::launch_fstage_multi(b->d_powseg, b->nmulti, b->powtotal, gxc::OUT_POWER, fs));
+    for (const gxc::FSeg &f : b->mpow)
+      GXB_HIP(b, gxc::launch_fstage(f.p, f.L, b->cfg.is_complex != 0, 0, fs));
     GXB_HIP(b, gxc::launch_scales_multi(b->d_scaleseg, ns, b->scaletotal, fs));
   }
   if (overlap) {
@@ -347,13 +363,12 @@ gxc_status enqueue_device_work(gxc_batch *b) {
     if (overlap && c >= 2) GXB_HIP(b, hipStreamWaitEvent(fs, b->ev_x[buf], 0));
     mark(b, 0, fs);
     if (b->nmulti > 0 && b->ftotal[c] > 0)
-      GXB_HIP(b, gxc::launch_fstage_multi(b->d_fseg + (size_t)c * b->nmulti, b->nmulti, b->ftotal[c], b->out_mode,
-                                          b->fblock, fs));
+      GXB_HIP(b, gxc::launch_fstage_multi(b->d_fseg + (size_t)c * b->nmulti, b->nmulti, b->ftotal[c], b->out_mode, fs));
     for (const gxc::FSeg &f : b->mseg[c])
       GXB_HIP(b, b->cfg.fstage_mfma == 1 &&
                          gxc::fstage_mfma_supported(f.L, b->cfg.is_complex != 0, b->out_mode == gxc::OUT_F32)
                      ? gxc::launch_fstage_mfma(f.p, f.L, fs)
-                     : gxc::launch_fstage_big(f.p, f.L, b->cfg.is_complex != 0, fs));
+                     : gxc::launch_fstage(f.p, f.L, b->cfg.is_complex != 0, 0, fs));
     mark(b, 1, fs);
     if (overlap) {
       GXB_HIP(b, hipEventRecord(b->ev_f[buf], fs));
@@ -520,7 +535,7 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
     std::string why;
     gxc_status st = gxc::host::derive(&c, &subs[s].d, &why);
     if (st != GXC_OK) return set_err(nullptr, st, "subband " + std::to_string(s) + ": " + why);
-    if (!gxc::fstage_multi_supported(subs[s].d.L, false))
+    if (subs[s].d.L < 256 || subs[s].d.L > 8192)
       return set_err(nullptr, GXC_ERR_UNSUPPORTED,
                      "subband " + std::to_string(s) + ": FFT length must be 256..8192 in a batch");
     const int ct = gxc::xm_channels_per_group(subs[s].d.M, out_mode);
@@ -545,7 +560,6 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
   b->out_mode = out_mode;
   b->M = 2 * cfg->nant;
   b->nrows = b->sub[0].d.nrows;
-  b->fblock = gxc::fstage_multi_block(maxL);
   auto fail = [&](gxc_status st) {
     g_batch_error = b->err;
     gxc_batch_destroy(b);
@@ -852,28 +866,24 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   double def_ms = 0, best = 1e30;
   gxc_status st = time_process(b, &def_ms);
   cand++;
-  int best_fb = b->fblock, best_units = b->xunits, best_mfma = b->cfg.fstage_mfma;
-  bool any_mfma = false;  // a subband that fstage_mfma would give its own launch
-  for (const Sub &u : b->sub) any_mfma = any_mfma || u.d.L >= 2048;
-  for (int mf = 0; mf <= (any_mfma ? 2 : 0); mf++)
-    for (int fb : {256, 512}) {
+  int best_units = b->xunits, best_mfma = b->cfg.fstage_mfma;
+  bool any_mfma = false;  // a subband that the matrix-core F-stage covers
+  for (const Sub &u : b->sub)
+    any_mfma = any_mfma || gxc::fstage_mfma_supported(u.d.L, false, b->out_mode == gxc::OUT_F32);
+  for (int mf = 0; mf <= (any_mfma ? 1 : 0); mf++)
+    for (int units : {1024, 2048, 4096, 8192}) {
       if (st != GXC_OK) continue;
-      for (int units : {1024, 2048, 4096, 8192}) {
-        b->cfg.fstage_mfma = mf;
-        b->fblock = fb;
-        b->xunits = units;
-        st = assign_splits(b);
-        if (st == GXC_OK) st = build_tables(b);
-        double ms = 0;
-        if (st == GXC_OK) st = time_process(b, &ms);
-        cand++;
-        if (st != GXC_OK) break;
-        if (ms < best) best = ms, best_fb = fb, best_units = units, best_mfma = mf;
-      }
+      b->cfg.fstage_mfma = mf;
+      b->xunits = units;
+      st = assign_splits(b);
+      if (st == GXC_OK) st = build_tables(b);
+      double ms = 0;
+      if (st == GXC_OK) st = time_process(b, &ms);
+      cand++;
+      if (st == GXC_OK && ms < best) best = ms, best_units = units, best_mfma = mf;
     }
   if (st == GXC_OK) {
     b->cfg.fstage_mfma = best_mfma;
-    b->fblock = best_fb;
     b->xunits = best_units;
     st = assign_splits(b);
     if (st == GXC_OK) st = build_tables(b);
@@ -889,7 +899,7 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   b->graph_exec = nullptr;
   b->profiling = prof;
   if (st != GXC_OK) return st;
-  t.fblock = b->cfg.fstage_mfma == 1 ? gxc::kFBlockMfma : b->cfg.fstage_mfma == 2 ? GXC_FBLOCK_ONEPOL : b->fblock;
+  t.fblock = b->cfg.fstage_mfma == 1 ? gxc::kFBlockMfma : gxc::fstage_multi_block();
   t.xtile = gxc::xm_channels_per_group(b->M, b->out_mode);
   t.xsplits = b->xunits;  // for a batch: the X units per launch the splits aim at
   t.graph = b->cfg.graph;

@@ -104,10 +104,22 @@ gxc_status check_device(int *dev, std::string *why) {
 gxc_status upload_tables(const Derived &d, double bw, int nchan, float2 **twiddle, float **subfreq,
                          float **stepfreq, std::string *why) {
   const int L = d.L, s = d.g.s, nsf = d.g.fracsteps;
-  std::vector<float2> tw(L);
-  for (int m = 0; m < L; m++) {
-    const double ang = -2.0 * kPi * (double)m / (double)L;
-    tw[m] = make_float2((float)std::cos(ang), (float)std::sin(ang));
+  std::vector<float2> tw(f_tw_size(L));
+  auto w = [](long long m, int n) {  // exp(-2 pi i m / n)
+    const double ang = -2.0 * kPi * (double)(m % n) / (double)n;
+    return make_float2((float)std::cos(ang), (float)std::sin(ang));
+  };
+  for (int m = 0; m < 32; m++) tw[m] = w(m, 32);
+  if (f_matrix(L))
+    for (int k1 = 0; k1 < f_radix(L, 1); k1++)
+      for (int r = 0; r < 32; r++)
+        tw[32 + 2 * (((2 * (r / 16) + r / 2 % 2) * 4 + r / 4 % 4) * f_radix(L, 1) + k1) + r % 2] =
+            w((long long)k1 * r, 32 * f_radix(L, 1));
+  for (int p = f_tw_first(L); p < f_npass(L); p++) {
+    const int R = f_radix(L, p), ns = f_ns(L, p), n = f_tw_entries(L, p);
+    for (int i = 0; i < f_npowers(R); i++)
+      for (int m = 0; m < n; m++)
+        tw[f_tw_off(L, p) + i * n + m] = w((long long)f_power(i) * f_tw_step(L, p) * m, ns * R);
   }
   // fxkernel.cpp:171-175 channel-frequency tables, identical expressions.
   std::vector<float> subf(s), stepf(nsf);
@@ -115,13 +127,13 @@ gxc_status upload_tables(const Derived &d, double bw, int nchan, float2 **twiddl
   for (int i = 0; i < nsf; i++) stepf[i] = (float)((2 * kPi * i * s * bw) / (double)nchan);
   *twiddle = nullptr;
   *subfreq = *stepfreq = nullptr;
-  if (hipMalloc((void **)twiddle, L * sizeof(float2)) != hipSuccess ||
+  if (hipMalloc((void **)twiddle, tw.size() * sizeof(float2)) != hipSuccess ||
       hipMalloc((void **)subfreq, s * sizeof(float)) != hipSuccess ||
       hipMalloc((void **)stepfreq, nsf * sizeof(float)) != hipSuccess) {
     *why = "hipMalloc of the FFT tables failed";
     return GXC_ERR_OUT_OF_MEMORY;
   }
-  if (hipMemcpy(*twiddle, tw.data(), L * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
+  if (hipMemcpy(*twiddle, tw.data(), tw.size() * sizeof(float2), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(*subfreq, subf.data(), s * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
       hipMemcpy(*stepfreq, stepf.data(), nsf * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
     *why = "upload of the FFT tables failed";

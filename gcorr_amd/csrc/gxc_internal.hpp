@@ -30,6 +30,40 @@ struct Geometry {
   }
 };
 
+// FFT passes of the F-stage at length L: radix of pass p (1: no such pass),
+// product of the radices before it, number of passes.  From 2048 points on
+// pass 0 is a radix-32 pass on the matrix cores and a thread holds 32 points
+// (fstage_big.hpp), below 16 (fstage16.hpp).
+constexpr bool f_matrix(int L) { return L >= 2048; }
+constexpr int f_radix(int L, int p) {
+  return p == 0   ? (f_matrix(L) ? 32 : 16)
+         : p == 1 ? (f_matrix(L) ? 32 : L == 256 ? 16 : L == 64 ? 4 : 8)
+                  : L / (f_radix(L, 0) * f_radix(L, 1));
+}
+constexpr int f_ns(int L, int p) { return p == 0 ? 1 : f_ns(L, p - 1) * f_radix(L, p - 1); }
+constexpr int f_npass(int L) { return f_radix(L, 2) == 1 ? 2 : 3; }
+// Twiddle tables of one FFT length, in float2 entries:
+//   W_32^m (m < 32);
+//   matrix pass 0: W_1024^(k1 r), applied to its outputs r < 32 for pass-1
+//   input k1 < 32: [r / 16][r / 2 % 2][r / 4 % 4][k1][r % 2]; and for the last
+//   pass of radix R, [power][m] W_L^(power m) of every second m < 1024 (every
+//   m at radix 32): a thread loads its first butterfly's powers and takes
+//   constants on top for the others;
+//   VALU passes of radix R after NS points: [power][m < NS] W_(NS R)^(power m);
+// for the powers 1, 2, 3, 4, 8, .. R/2.  Neighbouring lanes read neighbouring
+// entries: gathers from one table of W_L, up to a 128-byte line per lane, kept
+// the vector L1 busy 64 % of the F-stage (16 stations x 4096 channels).
+constexpr int f_npowers(int R) { return R == 2 ? 1 : R == 4 ? 3 : 2 + ilog2c(R) - 1; }
+constexpr int f_power(int i) { return i < 3 ? i + 1 : 4 << (i - 3); }
+constexpr int f_tw_first(int L) { return f_matrix(L) ? 2 : 1; }  // first pass with a power table
+constexpr int f_tw_step(int L, int p) { return !f_matrix(L) || f_radix(L, p) >= 32 ? 1 : 2; }
+constexpr int f_tw_entries(int L, int p) { return f_ns(L, p) / f_tw_step(L, p); }
+constexpr int f_tw_off(int L, int p) {
+  return p == f_tw_first(L) ? 32 + (f_matrix(L) ? 1024 : 0)
+                            : f_tw_off(L, p - 1) + f_npowers(f_radix(L, p - 1)) * f_tw_entries(L, p - 1);
+}
+constexpr int f_tw_size(int L) { return f_tw_off(L, f_npass(L)); }
+
 // What the F-stage writes per (station, FFT): FP32 spectra, scaled
 // reduced-precision spectra (complex: 2 x 16 bits or 2 x 8 bits), or |X|^2
 // accumulated per (input, channel) for the scale estimate.
@@ -42,7 +76,7 @@ struct FParams {
   const double *delays;           // [nant][4]: d0, d1, d2, file offset (s)
   const float *subchanfreq;       // [s]          fxkernel.cpp:173
   const float *stepchanfreq;      // [fracsteps]  fxkernel.cpp:174
-  const float2 *twiddle;          // [L] exp(-2 pi i m / L)
+  const float2 *twiddle;          // [f_tw_size(L)]
   float2 *spectra;                // OUT_F32: [nt][nant*2][nchan]
   void *out;                      // OUT_F16/BF16/FP8: [nt][nant*2][nchan] packed complex
   const float *scales;            // [nant*2][nchan] multipliers before rounding
@@ -59,6 +93,7 @@ struct FParams {
   int stepmul;                    // s (stride law) or S2 (exact phase)
   int fraclo;                     // LO has a fractional part
   double lo, lofrac, sampletime;
+  double samplerate;              // 1 / sampletime
 };
 
 // Row counts: for each output row (station pair; autos have j == k) the
@@ -92,11 +127,13 @@ hipError_t allow_dynamic_lds(const void *kernel, int bytes);
 
 // Launchers (defined in the .hip files).  Return hipSuccess or the launch error.
 bool fstage_supported(int L, bool cplx);
-// F-stage workgroup sizes available at FFT length L (default first).
+// F-stage workgroup sizes that gxc_config.fblock may name at FFT length L
+// (default first).
 int fstage_blocks(int L, bool cplx, int *out /* [4] */);
-// block: one of fstage_blocks (0 = default); ignored for L > 8192
+// block: kFBlockMfma, else one of fstage_blocks (0 = default), which all run
+// the length's one kernel
 hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s);
-hipError_t launch_fstage_big(const FParams &p, int L, bool cplx, hipStream_t s);  // L = 16384, 32768
+hipError_t launch_fstage_big(const FParams &p, int L, bool cplx, hipStream_t s);  // L = 2048..32768
 // F-stage with the FFT passes on the matrix cores (fstage_mfma.hip): real
 // input; reduced-precision outputs (and the power pass) at L = 2048..8192,
 // FP32 spectra (operands as f16 hi + lo) at L = 2048..4096.
@@ -104,14 +141,11 @@ constexpr int kFBlockMfma = -1;
 bool fstage_mfma_supported(int L, bool cplx, bool fp32);
 hipError_t launch_fstage_mfma(const FParams &p, int L, hipStream_t s);
 hipError_t launch_counts(const CountParams &p, hipStream_t s);
-// Multi-subband F-stage: real 2-bit input, FFT lengths 256..8192, workgroups
-// of `block` threads (256, the default, or 512); units of a subband =
-// ceil(nant * nt / (block / (L/16))), or 2 * nant * nt at L = 8192 and 256.
-bool fstage_multi_supported(int L, bool cplx);
-int fstage_multi_block(int maxL);
-long long fstage_multi_units(int L, int block, long long items);
-hipError_t launch_fstage_multi(const FSeg *segs, int nseg, long long total, int out_mode, int block,
-                               hipStream_t s);
+// Multi-subband F-stage: real 2-bit input, FFT lengths 256..1024, workgroups
+// of fstage_multi_block() threads; units of a subband of `items` = nant * nt.
+int fstage_multi_block();
+long long fstage_multi_units(int L, long long items);
+hipError_t launch_fstage_multi(const FSeg *segs, int nseg, long long total, int out_mode, hipStream_t s);
 hipError_t launch_counts_multi(const CountSeg *segs, int nseg, long long total, hipStream_t s);
 
 }  // namespace gxc

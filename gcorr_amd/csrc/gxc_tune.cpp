@@ -64,10 +64,12 @@ gxc_status gxc_autotune(gxc_handle *h, gxc_tuning *out) {
   gxc_status st = time_ms(h, process, 3, &def_ms);
   cand++;
 
-  // F-stage: FFT blocks per workgroup
+  // F-stage: the kernel of this length, and the one with f16 operands in
+  // every pass where it covers the length
   double best_f = 1e30;
   int best_fb = h->fblock;
-  int fb[5], nfb = gxc::fstage_blocks(h->d.L, h->cfg.is_complex != 0, fb);
+  int fb[5], nfb = 1;
+  gxc::fstage_blocks(h->d.L, h->cfg.is_complex != 0, fb);
   if (gxc::fstage_mfma_supported(h->d.L, h->cfg.is_complex != 0, h->out_mode == gxc::OUT_F32))
     fb[nfb++] = gxc::kFBlockMfma;
   for (int i = 0; i < nfb && st == GXC_OK; i++) {

@@ -90,8 +90,10 @@ typedef struct {
   int graph;       /* 1: capture the device work of one subintegration as a
                       hipGraph on first use and replay it afterwards */
   /* Launch shapes (0 = default; gxc_autotune measures and sets them): */
-  int fblock;      /* F-stage workgroup size, i.e. FFT blocks per workgroup
-                      = fblock / (fftchannels/16); or GXC_FBLOCK_MFMA */
+  int fblock;      /* F-stage kernel: GXC_FBLOCK_MFMA, or 0 or a workgroup
+                      size (fftchannels/16 times a power of two, or
+                      fftchannels/32), which all name the one kernel of the
+                      length */
   int xtile;       /* X-stage channel tile (channels per workgroup) */
   int xsplits;     /* X-stage FFT splits (workgroups per channel tile) */
   int reserved[1];
@@ -102,11 +104,8 @@ typedef struct {
  * 2048..8192 for the reduced precisions, 2048..4096 for FP32 (operands as
  * f16 pairs plus remainders, within the FP32 bound). */
 #define GXC_FBLOCK_MFMA (-1)
-/* In a batch's tuning result: the subbands of 2048 points and more have
- * launches of their own on the register F-stage (gxc_batch_config.fstage_mfma
- * 2; the name is from when its workgroups took one polarisation each, as
- * they still do above 8192 points).  No counterpart in the reference (its
- * subbands are separate runs). */
+/* Not returned any more: named launches of their own for a batch's subbands
+ * of 2048 points and more, which they now always have. */
 #define GXC_FBLOCK_ONEPOL (-2)
 
 typedef struct gxc_handle gxc_handle;
@@ -356,8 +355,8 @@ gxc_status gxc_xengine(const gxc_cf32 *spectra, int nant, int nchan, int nfft,
 gxc_status gxc_xengine_noalloc(const gxc_cf32 *d_spectra, int nant, int nchan, int nfft,
                                int autos, int precision, gxc_cf32 *d_vis, void *stream);
 
-/* Autotuner: with input and delays set, times the F-stage at each available
- * workgroup size (FFT blocks per workgroup), the X-stage at each channel
+/* Autotuner: with input and delays set, times the F-stage kernels that cover
+ * the length, the X-stage at each channel
  * tile and split count, and whole subintegrations with and without graph
  * replay, on this handle's own data; keeps the fastest.  The choice is
  * returned (may be NULL) and applies to later gxc_process calls; it can be
@@ -406,9 +405,10 @@ gxc_status gxc_get_timings(const gxc_handle *h, gxc_timings *t);
  * an observation with several subbands runs one object per subband.  A batch
  * holds every subband of a subintegration: the same stations, each subband
  * with its own channel count, bandwidth, LO, FFT count, delays and input.
- * Each stage runs for all subbands in one persistent launch (F-stage,
- * X-stage, row counts, finalise), and with graph on the whole subintegration
- * is captured as one hipGraph.  Per subband the visibilities are those of a
+ * Each stage runs for all subbands in one persistent launch (F-stage below
+ * 2048 points, X-stage, row counts, finalise; longer FFTs have a launch per
+ * subband), and with graph on the whole subintegration is captured as one
+ * hipGraph.  Per subband the visibilities are those of a
  * gxc_handle with the same settings (same layout, same normalisation).
  * Real 2-bit input, FFT lengths 2*nchan of 256..8192. */
 typedef struct {
@@ -434,13 +434,12 @@ typedef struct {
                                    within 32 GiB (eight with overlap) */
   int overlap;                  /* as gxc_config.overlap */
   int graph;                    /* as gxc_config.graph */
-  int fstage_mfma;              /* 1: subbands of 2048 points and more get a
-                                   launch each, on the matrix-core F-stage
-                                   (GXC_FBLOCK_MFMA) where it covers them,
-                                   else on the register F-stage; 2: a launch
-                                   each on the register F-stage; the others
-                                   stay in the multi-subband launch.
-                                   gxc_batch_autotune chooses. */
+  int fstage_mfma;              /* the subbands of 2048 points and more have a
+                                   launch each: 1 runs it on the matrix-core
+                                   F-stage (GXC_FBLOCK_MFMA) where that covers
+                                   the length, 0 and 2 on the F-stage of a
+                                   handle's default.  gxc_batch_autotune
+                                   chooses. */
   int reserved[3];
 } gxc_batch_config;
 
@@ -479,15 +478,12 @@ gxc_status gxc_batch_synchronize(gxc_batch *b);
 gxc_status gxc_batch_get_visibilities(gxc_batch *b, int sub, gxc_cf32 *out, size_t nelem);
 gxc_status gxc_batch_get_row_counts(gxc_batch *b, int sub, int *counts, size_t n);
 /* Autotuner of a batch (input and delays of every subband set): times whole
- * subintegrations for each F-stage workgroup size (256/512 threads) and X
- * unit count (1024..8192, which sets every subband's FFT splits), with and
- * without launches of their own for the subbands of 2048 points and more
- * (gxc_batch_config.fstage_mfma), then with and without graph replay, and
- * keeps the fastest.  In the result, fblock is the multi-subband workgroup
- * size, or GXC_FBLOCK_MFMA / GXC_FBLOCK_ONEPOL when the own launches (on
- * the matrix cores where they cover the length / on the register kernel)
- * were chosen (the choice is kept in the batch); xsplits holds the chosen
- * X unit count and fstage_ms/xstage_ms are 0. */
+ * subintegrations for each X unit count (1024..8192, which sets every
+ * subband's FFT splits) with either F-stage (gxc_batch_config.fstage_mfma 0
+ * and 1), then with and without graph replay, and keeps the fastest.  In the
+ * result, fblock is the multi-subband workgroup size, or GXC_FBLOCK_MFMA when
+ * the matrix-core F-stage was chosen (the choice is kept in the batch);
+ * xsplits holds the chosen X unit count and fstage_ms/xstage_ms are 0. */
 gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out);
 
 /* Timing over all subbands (launch counts are per-stage launches, one per

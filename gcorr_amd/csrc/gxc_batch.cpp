@@ -150,6 +150,16 @@ void mark(gxc_batch *b, int kind, hipStream_t s) {
   b->marks.push_back({kind, idx});
 }
 
+// channels per unit of the X launch
+int x_channels(const gxc_batch *b) {
+  return b->out_mode == gxc::OUT_F32 ? gxc::xsplit_channels(b->M) : gxc::xm_channels_per_group(b->M, b->out_mode);
+}
+
+// Fewest X units per launch worth trying: two FP32 workgroups per CU in turn
+// (8 subbands x 8 stations, X-stage: 3.89 ms with 256 units, 2.47 with 512, 2.50
+// with 1024, 2.61 with 2048), four of the others'.
+int x_units_min(const gxc_batch *b) { return b->out_mode == gxc::OUT_F32 ? 512 : 1024; }
+
 // F-stage parameters of subband s, FFTs t0.. (stride tstride), output mode.
 gxc::FParams fparams(const gxc_batch *b, const Sub &u, int t0, int nt, int tstride, int mode, void *out) {
   gxc::FParams p{};
@@ -199,7 +209,7 @@ gxc_status build_tables(gxc_batch *b) {
   b->d_powseg = nullptr;
   b->d_scaleseg = nullptr;
   const int ns = (int)b->sub.size(), C = b->nchunks;
-  const int ct = gxc::xm_channels_per_group(b->M, b->out_mode);
+  const int ct = x_channels(b);
   // The subbands of 2048 points and more get launches of their own: their
   // kernel holds 32 points per thread and one length's LDS per workgroup, and
   // in one persistent launch with the shorter lengths every workgroup would
@@ -242,6 +252,10 @@ gxc_status build_tables(gxc_batch *b) {
       x.p.nchan = u.cfg.nchan;
       x.p.splits = u.splits;
       x.p.accumulate = c > 0;
+      if (b->out_mode == gxc::OUT_F32) {
+        x.p.scale = gxc::xsplit_scale(u.d.L, u.cfg.is_complex != 0);
+        x.p.unscale = 1.f / (x.p.scale * x.p.scale);
+      }
       x.unit0 = xu;
       xu += (long long)(u.cfg.nchan / ct) * u.splits;
     }
@@ -320,7 +334,7 @@ gxc_status build_tables(gxc_batch *b) {
 // covering a similar number of FFTs (a unit's X work is channels x FFTs x
 // M^2); partial buffers grow when needed.
 gxc_status assign_splits(gxc_batch *b) {
-  const int ct = gxc::xm_channels_per_group(b->M, b->out_mode);
+  const int ct = x_channels(b);
   const int tb = b->out_mode == gxc::OUT_F32 ? 16 : 32;
   double work = 0;
   for (const Sub &u : b->sub) work += (double)(u.cfg.nchan / ct) * u.ntc;
@@ -375,7 +389,9 @@ gxc_status enqueue_device_work(gxc_batch *b) {
       GXB_HIP(b, hipStreamWaitEvent(xs, b->ev_f[buf], 0));
     }
     mark(b, 2, xs);
-    GXB_HIP(b, gxc::launch_xmfma_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->out_mode, b->M, xs));
+    GXB_HIP(b, b->out_mode == gxc::OUT_F32
+                   ? gxc::launch_xsplit_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->M, xs)
+                   : gxc::launch_xmfma_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->out_mode, b->M, xs));
     mark(b, 3, xs);
     if (overlap) GXB_HIP(b, hipEventRecord(b->ev_x[buf], xs));
   }
@@ -558,6 +574,7 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
   b->sub = std::move(subs);
   b->device = dev;
   b->out_mode = out_mode;
+  b->xunits = out_mode == gxc::OUT_F32 ? 512 : 2048;
   b->M = 2 * cfg->nant;
   b->nrows = b->sub[0].d.nrows;
   auto fail = [&](gxc_status st) {
@@ -871,7 +888,8 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   for (const Sub &u : b->sub)
     any_mfma = any_mfma || gxc::fstage_mfma_supported(u.d.L, false, b->out_mode == gxc::OUT_F32);
   for (int mf = 0; mf <= (any_mfma ? 1 : 0); mf++)
-    for (int units : {1024, 2048, 4096, 8192}) {
+    for (int f : {1, 2, 4, 8}) {
+      const int units = f * x_units_min(b);
       if (st != GXC_OK) continue;
       b->cfg.fstage_mfma = mf;
       b->xunits = units;
@@ -900,7 +918,7 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   b->profiling = prof;
   if (st != GXC_OK) return st;
   t.fblock = b->cfg.fstage_mfma == 1 ? gxc::kFBlockMfma : gxc::fstage_multi_block();
-  t.xtile = gxc::xm_channels_per_group(b->M, b->out_mode);
+  t.xtile = x_channels(b);
   t.xsplits = b->xunits;  // for a batch: the X units per launch the splits aim at
   t.graph = b->cfg.graph;
   t.process_ms = std::min(best, graph_ms);

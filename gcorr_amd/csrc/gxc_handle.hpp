@@ -55,6 +55,7 @@ struct gxc_handle {
   int out_mode = gxc::OUT_F32;
   int chunk = 0, nbuf = 1, splits = 1;
   int fblock = 0, xtile = 0;  // launch shapes (0 = default)
+  float xscale = 0.f;         // > 0: FP32 spectra go through launch_xsplit
   int partial_cap = 0;        // splits the partial buffer holds
   void *d_spec[2] = {nullptr, nullptr};  // [chunk][M][nchan] packed complex
   float *d_partial = nullptr;             // [splits][nchan][2][M][M]

@@ -12,7 +12,8 @@ namespace gxc {
 // part Re(V) (upper block triangle), plane 1 G_IR[a][b] = sum Im(x_a) Re(x_b)
 // (all entries), so Im V_ab = G_IR[a][b] - G_IR[b][a].  FP32 blocks off the
 // diagonal hold Im V_ab itself at [a][b] (a's block before b's) and 0 at
-// [b][a], which the same difference returns.
+// [b][a], which the same difference returns; so does half of Im V in all
+// entries of launch_xsplit's blocks on the diagonal.
 struct XMParams {
   const void *spectra;  // [nt][M][nchan] complex (2 x 32, 16 or 8 bits)
   float *partial;       // [splits][nchan][2][M][M]
@@ -20,6 +21,7 @@ struct XMParams {
                         // chunks (Neumaier), or null (one chunk)
   int nt, M, nchan, splits;
   int accumulate;       // add into partial instead of overwriting
+  float scale, unscale; // launch_xsplit: xsplit_scale and 1 / scale^2
 };
 
 struct FinMParams {
@@ -57,9 +59,18 @@ int xm_choose_splits(int M, int nchan, int nt, int out_mode);
 size_t xm_partial_bytes(int M, int nchan, int splits);
 int xm_element_bytes(int out_mode);   // bytes of one packed complex value
 
-// ct: channel tile, one of xm_tiles (0 = default)
+// ct: channel tile, one of xm_tiles (0 = default; FP32 has the default only)
 hipError_t launch_xmfma(const XMParams &p, int out_mode, int ct, hipStream_t s);
-// Channel tiles available for M inputs (default first); returns the count (<= 3).
+// The same for FP32 spectra that an F-stage of this build wrote (xsplit.hip):
+// p.scale and p.unscale set, nchan a multiple of xsplit_channels, the
+// channels of a workgroup.
+int xsplit_channels(int M);
+float xsplit_scale(int L, bool cplx);
+int xsplit_choose_splits(int M, int nchan, int nt);
+hipError_t launch_xsplit(const XMParams &p, hipStream_t s);
+hipError_t launch_xsplit_multi(const XSeg *segs, int nseg, long long total, int M, hipStream_t s);
+// Channel tiles that gxc_config.xtile may name for M inputs (default first);
+// returns the count (<= 3).  FP32 handles run launch_xsplit's one tile.
 int xm_tiles(int M, int out_mode, int *out);
 // scales[i] = power of two nearest target / sqrt(mean_r power[r][i]), r < nrows.
 hipError_t launch_scales(float *scales, const float *power, int n, int nrows, float target, hipStream_t s);

@@ -12,7 +12,9 @@
 // P1 = R_i R_j^T, P2 = I_i I_j^T, P3 = (R_i + I_i)(R_j - I_j)^T, with
 // Re V = P1 + P2 and Im V = P3 - P1 + P2 (the packed forms are read from
 // HBM at full speed with the MFMAs mostly idle, and their sums R + I would
-// add a rounding).
+// add a rounding).  FP32 here serves spectra that a caller hands in, of any
+// magnitude; those of the F-stage, whose magnitude is bounded, are taken by
+// xsplit.hip in half to two thirds of the time.
 //
 // The F-stage writes spectra channel-contiguous ([t][input][chan]), the
 // layout its last FFT pass stores coalesced.  Each workgroup stages a
@@ -32,10 +34,12 @@
 // finalise reads a channel's partials as one contiguous block.
 #include <type_traits>
 
-#include "gxc_xengine.hpp"
+#include "xengine_common.hpp"
 
 namespace gxc {
 namespace {
+
+using namespace xs;
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -288,18 +292,6 @@ struct Stage {
   }
 };
 
-// sum + comp += v with Neumaier's compensation (the rounding error of each
-// addition kept in comp).
-__device__ __forceinline__ void neumaier(float &sum, float &comp, float v) {
-#pragma clang fp contract(off)
-  const float t = sum + v;
-  if (fabsf(sum) >= fabsf(v))
-    comp += (sum - t) + v;
-  else
-    comp += (v - t) + sum;
-  sum = t;
-}
-
 // Channels group*CT .. group*CT+CT-1, FFT split `split`, on a workgroup of
 // NWV waves, wave w taking channels w, w + NWV, ... (every thread calls it
 // with the same arguments: it contains __syncthreads).  lds holds XM::LDSB
@@ -398,23 +390,8 @@ __device__ __forceinline__ void xmfma_item(const XMParams &p, int group, int spl
   // D[i][j] of a 16x16 tile sits in lane j + 16*(i/4), element i%4.
   // Partials: [split][channel][plane][a][b], so a wave's stores and the
   // read-modify-write of later chunks cover whole rows of one channel.
-  // With a compensation buffer (subintegrations of several chunks) each
-  // later chunk is added with Neumaier's compensation, the first clears it.
   const size_t MM = (size_t)M * M;
-  // one value of this chunk into element e of a partial plane
-  auto put = [&](float *pl, float *cpl, size_t e, float v) {
-    if (!p.accumulate) {
-      pl[e] = v;
-      if (cpl) cpl[e] = 0.f;
-    } else if (cpl) {
-      float sum = pl[e], comp = cpl[e];
-      neumaier(sum, comp, v);
-      pl[e] = sum;
-      cpl[e] = comp;
-    } else {
-      pl[e] += v;
-    }
-  };
+  auto put = [&](float *pl, float *cpl, size_t e, float v) { put_partial(p.accumulate, pl, cpl, e, v); };
 #pragma unroll
   for (int w = 0; w < X::CPW; w++) {
     const int c = c0 + wave + NWV * w;
@@ -453,18 +430,6 @@ __device__ __forceinline__ void xmfma_item(const XMParams &p, int group, int spl
   }
 }
 
-// Workgroups are dealt to the 8 XCDs round robin in dispatch order, and each
-// XCD has its own L2.  A channel group's rows are CT*CB bytes wide, less
-// than a 128-byte line when CT is small, so neighbouring groups share lines:
-// renumber the units so that consecutive units (neighbouring channel groups)
-// run on the same XCD one after another and meet the line in its L2.
-constexpr int kXcds = 8;
-__device__ __forceinline__ long long xcd_swizzle(long long u, long long total) {
-  const long long per = total / kXcds;  // units per XCD in the swizzled range
-  if (u >= per * kXcds) return u;       // tail: unchanged
-  return (u % kXcds) * per + u / kXcds;
-}
-
 // Waves per SIMD the register allocation must leave room for: two
 // workgroups of 8 waves per CU (4 per SIMD, 128 registers per wave) where
 // their LDS tiles fit and the accumulators take at most 96 registers;
@@ -482,14 +447,6 @@ xmfma_kernel(XMParams p) {
   const int groups = p.nchan / CT;
   const long long u = xcd_swizzle(blockIdx.x, (long long)groups * p.splits);
   xmfma_item<ET, MB, CT, NWV>(p, (int)(u % groups), (int)(u / groups), lds);
-}
-
-// Segment of a multi-subband launch holding unit u (segments in order).
-template <typename Seg>
-__device__ __forceinline__ int find_seg(const Seg *segs, int nseg, long long u) {
-  int s = 0;
-  while (s + 1 < nseg && u >= segs[s + 1].unit0) ++s;
-  return s;
 }
 
 // Persistent X-stage over several subbands of the same M: unit = (subband,
@@ -725,9 +682,11 @@ hipError_t launch_xm_multi_mb(const XSeg *segs, int nseg, long long total, int M
 template <int ET, int MB>
 hipError_t launch_xm_ct(const XMParams &p, int ct, hipStream_t s) {
   constexpr int D = xm_default_ct(ET, MB);
-  if (ct == 0 || ct == D) return launch_xm<ET, MB, D>(p, s);
-  if (ct == D / 2) return launch_xm_if<ET, MB, D / 2>(p, s);
-  if (ct == 2 * D) return launch_xm_if<ET, MB, 2 * D>(p, s);
+  if (ET == OUT_F32 || ct == 0 || ct == D) return launch_xm<ET, MB, D>(p, s);
+  if constexpr (ET != OUT_F32) {
+    if (ct == D / 2) return launch_xm_if<ET, MB, D / 2>(p, s);
+    if (ct == 2 * D) return launch_xm_if<ET, MB, 2 * D>(p, s);
+  }
   return hipErrorInvalidValue;
 }
 
@@ -824,7 +783,6 @@ int xm_tiles(int M, int out_mode, int *out) {
 hipError_t launch_xmfma_multi(const XSeg *segs, int nseg, long long total, int out_mode, int M, hipStream_t s) {
   if (total <= 0) return hipSuccess;
   switch (out_mode) {
-    case OUT_F32: return launch_xm_multi_mb<OUT_F32>(segs, nseg, total, M, s);
     case OUT_F16: return launch_xm_multi_mb<OUT_F16>(segs, nseg, total, M, s);
     case OUT_BF16: return launch_xm_multi_mb<OUT_BF16>(segs, nseg, total, M, s);
     case OUT_FP8: return launch_xm_multi_mb<OUT_FP8>(segs, nseg, total, M, s);

@@ -94,7 +94,8 @@ typedef struct {
                       size (fftchannels/16 times a power of two, or
                       fftchannels/32), which all name the one kernel of the
                       length */
-  int xtile;       /* X-stage channel tile (channels per workgroup) */
+  int xtile;       /* X-stage channel tile (channels per workgroup); FP32
+                      has one tile, which every accepted value runs */
   int xsplits;     /* X-stage FFT splits (workgroups per channel tile) */
   int reserved[1];
 } gxc_config;
@@ -478,7 +479,7 @@ gxc_status gxc_batch_synchronize(gxc_batch *b);
 gxc_status gxc_batch_get_visibilities(gxc_batch *b, int sub, gxc_cf32 *out, size_t nelem);
 gxc_status gxc_batch_get_row_counts(gxc_batch *b, int sub, int *counts, size_t n);
 /* Autotuner of a batch (input and delays of every subband set): times whole
- * subintegrations for each X unit count (1024..8192, which sets every
+ * subintegrations for each X unit count (512..8192, which sets every
  * subband's FFT splits) with either F-stage (gxc_batch_config.fstage_mfma 0
  * and 1), then with and without graph replay, and keeps the fastest.  In the
  * result, fblock is the multi-subband workgroup size, or GXC_FBLOCK_MFMA when

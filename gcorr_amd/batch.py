@@ -93,8 +93,7 @@ class Batch:
     def set_delays(self, sub, d, f):
         d = np.ascontiguousarray(d, dtype=np.float64).reshape(self.nant, 3)
         f = np.ascontiguousarray(f, dtype=np.float64).reshape(self.nant)
-        rows = (ctypes.POINTER(ctypes.c_double) * self.nant)(
-            *[d[a].ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in range(self.nant)])
+        rows = _lib.row_pointers(d)
         check_batch(self._L.gxc_batch_set_delays(self._h, int(sub), rows,
                                                  f.ctypes.data_as(ctypes.POINTER(ctypes.c_double))),
                     self._h)

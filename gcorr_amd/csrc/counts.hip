@@ -42,7 +42,10 @@ __device__ __forceinline__ void count_row(const CountParams &p, int row) {
     if (threadIdx.x < s) red[threadIdx.x] += red[threadIdx.x + s];
     __syncthreads();
   }
-  if (threadIdx.x == 0) p.counts[row] = red[0];
+  if (threadIdx.x == 0) {
+    p.counts[row] = red[0];
+    if (p.host_counts) p.host_counts[row] = red[0];
+  }
   __syncthreads();  // red is reused by the next row of a persistent launch
 }
 

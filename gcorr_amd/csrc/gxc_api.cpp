@@ -126,6 +126,7 @@ gxc_status run_finalise(gxc_handle *h, hipStream_t s) {
   cp.valid = h->d_valid;
   cp.rowmap = h->d_rowmap;
   cp.counts = h->d_counts;
+  cp.host_counts = h->h_counts;
   cp.numffts = h->cfg.numffts;
   cp.nrows = h->d.nrows;
   GXC_HIP(h, gxc::launch_counts(cp, s));
@@ -195,9 +196,14 @@ gxc_status ensure_owned_input(gxc_handle *h) {
   if (h->d_input_owned) return GXC_OK;
   const int nant = h->cfg.nant;
   GXC_TRY(dmalloc(h, &h->d_input_owned, h->d.station_bytes * (size_t)nant));
-  std::vector<const uint8_t *> ptrs(nant);
-  for (int a = 0; a < nant; a++) ptrs[a] = h->d_input_owned + (size_t)a * h->d.station_bytes;
-  GXC_HIP(h, hipMemcpy(h->d_station_ptrs, ptrs.data(), nant * sizeof(void *), hipMemcpyHostToDevice));
+  return point_at_owned(h);
+}
+
+gxc_status point_at_owned(gxc_handle *h) {
+  GXC_HIP(h, hipStreamSynchronize(h->stream));
+  for (int a = 0; a < h->cfg.nant; a++)
+    h->h_station_ptrs[a] = h->d_input_owned + (size_t)a * h->d.station_bytes;
+  h->mail.dirty = true;
   return GXC_OK;
 }
 
@@ -216,6 +222,7 @@ gxc_status enqueue_process(gxc_handle *h) {
   h->marks.clear();
   mark(h, 7, h->stream);
   GXC_TRY(enqueue_input_copy(h));
+  GXC_HIP(h, h->mail.flush(h->stream));
   mark(h, 6, h->stream);
   const bool use_graph = h->cfg.graph && !h->profiling;
   if (!use_graph) return enqueue_device_work(h);
@@ -363,9 +370,17 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
       return fail(set_err(h, GXC_ERR_HIP, "hipEventCreate failed"));
   if ((s = upload_tables(h)) != GXC_OK) return fail(s);
   const int nant = cfg->nant, nchan = cfg->nchan;
-  h->h_delays.assign((size_t)nant * 4, 0.0);
-  if ((s = dmalloc(h, &h->d_delays, (size_t)nant * 4)) != GXC_OK) return fail(s);
-  if ((s = dmalloc(h, &h->d_station_ptrs, (size_t)nant)) != GXC_OK) return fail(s);
+  {
+    const size_t ptrs = (size_t)nant * 4 * sizeof(double);  // after the delays
+    if (h->mail.create(ptrs + nant * sizeof(void *), d.nrows * sizeof(int)) != hipSuccess ||
+        h->out.create((size_t)d.nrows * 4 * nchan * sizeof(float2)) != hipSuccess)
+      return fail(set_err(h, GXC_ERR_OUT_OF_MEMORY, "pinned host memory"));
+    h->h_delays = reinterpret_cast<double *>(h->mail.h);
+    h->d_delays = reinterpret_cast<double *>(h->mail.d);
+    h->h_station_ptrs = reinterpret_cast<const uint8_t **>(h->mail.h + ptrs);
+    h->d_station_ptrs = reinterpret_cast<const uint8_t **>(h->mail.d + ptrs);
+    h->h_counts = reinterpret_cast<int *>(h->mail.h + h->mail.in);
+  }
   if ((s = dmalloc(h, &h->d_valid, (size_t)nant * cfg->numffts)) != GXC_OK) return fail(s);
   std::vector<int2> rm = make_rowmap(nant, cfg->autos != 0);
   if ((s = dmalloc(h, &h->d_rowmap, rm.size())) != GXC_OK) return fail(s);
@@ -479,8 +494,8 @@ void gxc_destroy(gxc_handle *h) {
   hipFree(h->d_scales);
   hipFree(h->d_power);
   hipFree(h->d_input_owned);
-  hipFree(h->d_station_ptrs);
-  hipFree(h->d_delays);
+  h->mail.release();
+  h->out.release();
   hipFree(h->d_twiddle);
   hipFree(h->d_subfreq);
   hipFree(h->d_stepfreq);
@@ -504,10 +519,7 @@ gxc_status gxc_set_input(gxc_handle *h, const uint8_t *const *per_station) {
   if (h->input_device || !h->d_input_owned) {
     h->input_device = false;
     GXC_TRY(ensure_owned_input(h));
-    // restore the station pointers to the owned copy
-    std::vector<const uint8_t *> ptrs(h->cfg.nant);
-    for (int a = 0; a < h->cfg.nant; a++) ptrs[a] = h->d_input_owned + (size_t)a * h->d.station_bytes;
-    GXC_HIP(h, hipMemcpy(h->d_station_ptrs, ptrs.data(), h->cfg.nant * sizeof(void *), hipMemcpyHostToDevice));
+    GXC_TRY(point_at_owned(h));  // an earlier call may have named other buffers
   }
   h->input_device = false;
   h->input_set = true;
@@ -524,8 +536,8 @@ gxc_status gxc_set_input_device(gxc_handle *h, const void *const *per_station) {
   }
   GXC_HIP(h, hipStreamSynchronize(h->stream));
   leave_vdif(h);
-  h->dev_in = in;
-  GXC_HIP(h, hipMemcpy(h->d_station_ptrs, h->dev_in.data(), h->cfg.nant * sizeof(void *), hipMemcpyHostToDevice));
+  for (int a = 0; a < h->cfg.nant; a++) h->h_station_ptrs[a] = static_cast<const uint8_t *>(in[a]);
+  h->mail.dirty = true;
   h->input_device = true;
   h->input_set = true;
   return GXC_OK;
@@ -535,13 +547,12 @@ gxc_status gxc_set_delays(gxc_handle *h, const double *const *poly3, const doubl
   if (!h || !poly3 || !fileoffsets) return set_err(h, GXC_ERR_INVALID_ARG, "null delays");
   for (int a = 0; a < h->cfg.nant; a++)
     if (!poly3[a]) return set_err(h, GXC_ERR_INVALID_ARG, "null delay polynomial");
+  GXC_HIP(h, hipStreamSynchronize(h->stream));
   for (int a = 0; a < h->cfg.nant; a++) {
     for (int i = 0; i < 3; i++) h->h_delays[4 * a + i] = poly3[a][i];
     h->h_delays[4 * a + 3] = fileoffsets[a];
   }
-  GXC_HIP(h, hipStreamSynchronize(h->stream));
-  GXC_HIP(h, hipMemcpy(h->d_delays, h->h_delays.data(), h->h_delays.size() * sizeof(double),
-                       hipMemcpyHostToDevice));
+  h->mail.dirty = true;
   h->delays_set = true;
   return GXC_OK;
 }
@@ -567,8 +578,7 @@ gxc_status gxc_get_visibilities(gxc_handle *h, gxc_cf32 *out, size_t nelem) {
   if (!h || !out) return set_err(h, GXC_ERR_INVALID_ARG, "null argument");
   const size_t n = (size_t)h->d.nrows * 4 * h->cfg.nchan;
   if (nelem < n) return set_err(h, GXC_ERR_INVALID_ARG, "output buffer too small");
-  GXC_HIP(h, hipStreamSynchronize(h->stream));
-  GXC_HIP(h, hipMemcpy(out, h->d_vis, n * sizeof(gxc_cf32), hipMemcpyDeviceToHost));
+  GXC_HIP(h, h->out.copy(out, h->d_vis, n * sizeof(gxc_cf32), h->stream));
   return GXC_OK;
 }
 
@@ -576,7 +586,7 @@ gxc_status gxc_get_row_counts(gxc_handle *h, int *counts, size_t n) {
   if (!h || !counts) return set_err(h, GXC_ERR_INVALID_ARG, "null argument");
   if (n < (size_t)h->d.nrows) return set_err(h, GXC_ERR_INVALID_ARG, "output buffer too small");
   GXC_HIP(h, hipStreamSynchronize(h->stream));
-  GXC_HIP(h, hipMemcpy(counts, h->d_counts, h->d.nrows * sizeof(int), hipMemcpyDeviceToHost));
+  std::memcpy(counts, h->h_counts, h->d.nrows * sizeof(int));
   return GXC_OK;
 }
 
@@ -635,6 +645,7 @@ gxc_status gxc_fstage(gxc_handle *h, int t0, int nfft, gxc_cf32 *spectra, uint8_
     return set_err(h, GXC_ERR_INVALID_ARG, "FFT range outside the subintegration");
   if (!h->input_set || !h->delays_set) return set_err(h, GXC_ERR_STATE, "input or delays not set");
   GXC_TRY(enqueue_input_copy(h));
+  GXC_HIP(h, h->mail.flush(h->stream));
   const size_t per_fft = (size_t)h->d.M * h->cfg.nchan;
   float2 *tmp = nullptr;
   GXC_TRY(dmalloc(h, &tmp, per_fft * nfft));

@@ -23,6 +23,7 @@
 #include "../../include/gxcorr.h"
 #include "gxc_host.hpp"
 #include "gxc_internal.hpp"
+#include "gxc_pinned.hpp"
 #include "gxc_vdif_state.hpp"
 #include "gxc_xengine.hpp"
 
@@ -41,16 +42,15 @@ struct Sub {
   bool input_set = false, input_device = false;
   std::vector<const uint8_t *> host_in;
   uint8_t *d_input_owned = nullptr;
-  const uint8_t **d_station_ptrs = nullptr;
+  const uint8_t **h_station_ptrs = nullptr, **d_station_ptrs = nullptr;  // [nant], in the batch's mail
   // delays
   bool delays_set = false;
-  std::vector<double> h_delays;
-  double *d_delays = nullptr;
+  double *h_delays = nullptr, *d_delays = nullptr;  // [nant][4], in the batch's mail
   // tables and outputs
   float2 *d_twiddle = nullptr;
   float *d_subfreq = nullptr, *d_stepfreq = nullptr;
   uint8_t *d_valid = nullptr;
-  int *d_counts = nullptr;
+  int *d_counts = nullptr, *h_counts = nullptr;  // [nrows], h_ in the batch's mail
   float2 *d_vis = nullptr;
   float *d_partial = nullptr;
   float *d_comp = nullptr;  // compensation of d_partial across chunks (several chunks only)
@@ -76,6 +76,10 @@ struct gxc_batch {
   hipStream_t stream = nullptr, xstream = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr, ev_f[2] = {nullptr, nullptr}, ev_x[2] = {nullptr, nullptr};
   hipGraphExec_t graph_exec = nullptr;
+  // delays and station pointers of every subband as the host last wrote them,
+  // their device copies, and the last row counts
+  gxc::host::Mailbox mail;
+  gxc::host::HostOut out;
   int2 *d_rowmap = nullptr;
   void *d_spec[2] = {nullptr, nullptr};
   // segment tables and unit totals
@@ -273,6 +277,7 @@ gxc_status build_tables(gxc_batch *b) {
     cseg[s].p.valid = u.d_valid;
     cseg[s].p.rowmap = b->d_rowmap;
     cseg[s].p.counts = u.d_counts;
+    cseg[s].p.host_counts = u.h_counts;
     cseg[s].p.numffts = u.cfg.numffts;
     cseg[s].p.nrows = b->nrows;
     cseg[s].unit0 = cu;
@@ -431,9 +436,9 @@ gxc_status vdif_mode(gxc_batch *b, Sub &u, bool on) {
 gxc_status leave_vdif(gxc_batch *b, Sub &u) { return vdif_mode(b, u, false); }
 
 gxc_status point_at_owned(gxc_batch *b, Sub &u) {
-  std::vector<const uint8_t *> ptrs(b->cfg.nant);
-  for (int a = 0; a < b->cfg.nant; a++) ptrs[a] = u.d_input_owned + (size_t)a * u.d.station_bytes;
-  GXB_HIP(b, hipMemcpy(u.d_station_ptrs, ptrs.data(), ptrs.size() * sizeof(void *), hipMemcpyHostToDevice));
+  GXB_HIP(b, hipStreamSynchronize(b->stream));
+  for (int a = 0; a < b->cfg.nant; a++) u.h_station_ptrs[a] = u.d_input_owned + (size_t)a * u.d.station_bytes;
+  b->mail.dirty = true;
   return GXC_OK;
 }
 
@@ -445,6 +450,7 @@ gxc_status enqueue_process(gxc_batch *b) {
   }
   b->marks.clear();
   mark(b, 7, b->stream);
+  GXB_HIP(b, b->mail.flush(b->stream));
   for (Sub &u : b->sub) {
     if (u.input_device || u.vdif) continue;
     for (int a = 0; a < b->cfg.nant; a++)
@@ -613,6 +619,26 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
   const size_t eb = gxc::xm_element_bytes(out_mode);
   gxc_status s = GXC_OK;
   if ((s = upload(b, &b->d_rowmap, gxc::host::make_rowmap(nant, cfg->autos != 0))) != GXC_OK) return fail(s);
+  {
+    // [subband][delays, station pointers], then [subband][row counts]
+    const size_t ptrs = (size_t)nant * 4 * sizeof(double), per = ptrs + nant * sizeof(void *);
+    size_t vis = 0;
+    for (const Sub &u : b->sub) vis = std::max(vis, (size_t)b->nrows * 4 * u.cfg.nchan * sizeof(float2));
+    if (b->mail.create(b->sub.size() * per, b->sub.size() * b->nrows * sizeof(int)) != hipSuccess ||
+        b->out.create(vis) != hipSuccess)
+      return fail(set_err(b, GXC_ERR_OUT_OF_MEMORY, "pinned host memory"));
+    size_t at = 0;
+    int *counts = reinterpret_cast<int *>(b->mail.h + b->mail.in);
+    for (Sub &u : b->sub) {
+      u.h_delays = reinterpret_cast<double *>(b->mail.h + at);
+      u.d_delays = reinterpret_cast<double *>(b->mail.d + at);
+      u.h_station_ptrs = reinterpret_cast<const uint8_t **>(b->mail.h + at + ptrs);
+      u.d_station_ptrs = reinterpret_cast<const uint8_t **>(b->mail.d + at + ptrs);
+      u.h_counts = counts;
+      at += per;
+      counts += b->nrows;
+    }
+  }
   size_t spec_bytes = 0;
   b->maxL = maxL;
   for (Sub &u : b->sub) u.ntc = (u.cfg.numffts + C - 1) / C;
@@ -624,9 +650,6 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
     if ((s = gxc::host::upload_tables(u.d, u.cfg.bw, u.cfg.nchan, &u.d_twiddle, &u.d_subfreq, &u.d_stepfreq,
                                       &why)) != GXC_OK)
       return fail(set_err(b, s, why));
-    u.h_delays.assign((size_t)nant * 4, 0.0);
-    if ((s = dmalloc(b, &u.d_delays, (size_t)nant * 4)) != GXC_OK) return fail(s);
-    if ((s = dmalloc(b, &u.d_station_ptrs, (size_t)nant)) != GXC_OK) return fail(s);
     if ((s = dmalloc(b, &u.d_valid, (size_t)nant * u.cfg.numffts)) != GXC_OK) return fail(s);
     if ((s = dmalloc(b, &u.d_counts, (size_t)b->nrows)) != GXC_OK) return fail(s);
     if ((s = dmalloc(b, &u.d_vis, (size_t)b->nrows * 4 * u.cfg.nchan)) != GXC_OK) return fail(s);
@@ -656,8 +679,6 @@ void gxc_batch_destroy(gxc_batch *b) {
     if (e) hipEventDestroy(e);
   for (Sub &u : b->sub) {
     hipFree(u.d_input_owned);
-    hipFree(u.d_station_ptrs);
-    hipFree(u.d_delays);
     hipFree(u.d_twiddle);
     hipFree(u.d_subfreq);
     hipFree(u.d_stepfreq);
@@ -671,6 +692,8 @@ void gxc_batch_destroy(gxc_batch *b) {
     hipFree(u.d_scales);
     hipFree(u.d_power);
   }
+  b->mail.release();
+  b->out.release();
   for (void *p : b->d_spec) hipFree(p);
   hipFree(b->d_rowmap);
   hipFree(b->d_fseg);
@@ -708,7 +731,8 @@ gxc_status gxc_batch_set_input_device(gxc_batch *b, int sub, const void *const *
     if (!p) return set_err(b, GXC_ERR_INVALID_ARG, "null station buffer");
   GXB_HIP(b, hipStreamSynchronize(b->stream));
   GXB_TRY(leave_vdif(b, *u));
-  GXB_HIP(b, hipMemcpy(u->d_station_ptrs, in.data(), in.size() * sizeof(void *), hipMemcpyHostToDevice));
+  for (int a = 0; a < b->cfg.nant; a++) u->h_station_ptrs[a] = static_cast<const uint8_t *>(in[a]);
+  b->mail.dirty = true;
   u->input_device = true;
   u->input_set = true;
   return GXC_OK;
@@ -717,14 +741,14 @@ gxc_status gxc_batch_set_input_device(gxc_batch *b, int sub, const void *const *
 gxc_status gxc_batch_set_delays(gxc_batch *b, int sub, const double *const *poly3, const double *fileoffsets) {
   Sub *u = get_sub(b, sub);
   if (!u || !poly3 || !fileoffsets) return set_err(b, GXC_ERR_INVALID_ARG, "bad subband or null delays");
-  for (int a = 0; a < b->cfg.nant; a++) {
+  for (int a = 0; a < b->cfg.nant; a++)
     if (!poly3[a]) return set_err(b, GXC_ERR_INVALID_ARG, "null delay polynomial");
+  GXB_HIP(b, hipStreamSynchronize(b->stream));
+  for (int a = 0; a < b->cfg.nant; a++) {
     for (int i = 0; i < 3; i++) u->h_delays[4 * a + i] = poly3[a][i];
     u->h_delays[4 * a + 3] = fileoffsets[a];
   }
-  GXB_HIP(b, hipStreamSynchronize(b->stream));
-  GXB_HIP(b, hipMemcpy(u->d_delays, u->h_delays.data(), u->h_delays.size() * sizeof(double),
-                       hipMemcpyHostToDevice));
+  b->mail.dirty = true;
   u->delays_set = true;
   return GXC_OK;
 }
@@ -811,8 +835,7 @@ gxc_status gxc_batch_get_visibilities(gxc_batch *b, int sub, gxc_cf32 *out, size
   if (!u || !out) return set_err(b, GXC_ERR_INVALID_ARG, "bad subband or null output");
   const size_t n = (size_t)b->nrows * 4 * u->cfg.nchan;
   if (nelem < n) return set_err(b, GXC_ERR_INVALID_ARG, "output buffer too small");
-  GXB_HIP(b, hipStreamSynchronize(b->stream));
-  GXB_HIP(b, hipMemcpy(out, u->d_vis, n * sizeof(gxc_cf32), hipMemcpyDeviceToHost));
+  GXB_HIP(b, b->out.copy(out, u->d_vis, n * sizeof(gxc_cf32), b->stream));
   return GXC_OK;
 }
 
@@ -821,7 +844,7 @@ gxc_status gxc_batch_get_row_counts(gxc_batch *b, int sub, int *counts, size_t n
   if (!u || !counts) return set_err(b, GXC_ERR_INVALID_ARG, "bad subband or null output");
   if (n < (size_t)b->nrows) return set_err(b, GXC_ERR_INVALID_ARG, "output buffer too small");
   GXB_HIP(b, hipStreamSynchronize(b->stream));
-  GXB_HIP(b, hipMemcpy(counts, u->d_counts, b->nrows * sizeof(int), hipMemcpyDeviceToHost));
+  std::memcpy(counts, u->h_counts, b->nrows * sizeof(int));
   return GXC_OK;
 }
 

@@ -15,6 +15,7 @@
 
 #include "gxc_host.hpp"
 #include "gxc_internal.hpp"
+#include "gxc_pinned.hpp"
 #include "gxc_vdif_state.hpp"
 #include "gxc_xengine.hpp"
 
@@ -29,9 +30,14 @@ struct gxc_handle {
   // input
   bool input_set = false, input_device = false;
   std::vector<const uint8_t *> host_in;
-  std::vector<const void *> dev_in;
   uint8_t *d_input_owned = nullptr;
-  const uint8_t **d_station_ptrs = nullptr;
+
+  // delays and station pointers as the host last wrote them, their device
+  // copies, and the row counts of the last subintegration
+  gxc::host::Mailbox mail;
+  gxc::host::HostOut out;
+  const uint8_t **h_station_ptrs = nullptr, **d_station_ptrs = nullptr;  // [nant], in mail
+  int *h_counts = nullptr;                                               // [nrows], in mail
 
   // VDIF ingest (gxc_set_input_vdif): payloads go into d_input_owned, and
   // the per-station frame flags make FFTs over missing frames invalid
@@ -44,8 +50,7 @@ struct gxc_handle {
 
   // delays
   bool delays_set = false;
-  std::vector<double> h_delays;  // [nant][4]
-  double *d_delays = nullptr;
+  double *h_delays = nullptr, *d_delays = nullptr;  // [nant][4], in mail
 
   // constant tables
   float2 *d_twiddle = nullptr;
@@ -145,6 +150,8 @@ gxc_status run_finalise(gxc_handle *h, hipStream_t s);
 // Device work of one subintegration once the input is resident.
 gxc_status enqueue_device_work(gxc_handle *h);
 gxc_status ensure_owned_input(gxc_handle *h);
+// The station pointers to the owned input buffer.
+gxc_status point_at_owned(gxc_handle *h);
 gxc_status enqueue_input_copy(gxc_handle *h);
 // Input copy, then the device work (replayed as a graph when enabled).
 gxc_status enqueue_process(gxc_handle *h);

@@ -102,6 +102,7 @@ struct CountParams {
   const uint8_t *valid;  // [nant][numffts]
   const int2 *rowmap;    // [nrows]
   int *counts;           // [nrows]
+  int *host_counts;      // the same in pinned host memory, or null
   int numffts, nrows;
 };
 

@@ -100,7 +100,7 @@ gxc_status gxc_integrate_end(gxc_handle *h, gxc_cf32 *out, size_t nelem, int *ns
   const size_t nvis = (size_t)h->d.nrows * 4 * h->cfg.nchan;
   if (out && nelem < nvis) return set_err(h, GXC_ERR_INVALID_ARG, "output buffer too small");
   GXC_HIP(h, hipStreamSynchronize(h->stream));
-  if (out) GXC_HIP(h, hipMemcpy(out, h->d_acc, nvis * sizeof(gxc_cf32), hipMemcpyDeviceToHost));
+  if (out) GXC_HIP(h, h->out.copy(out, h->d_acc, nvis * sizeof(gxc_cf32), h->stream));
   if (nsubints) *nsubints = (int)h->nsubmitted;
   h->integrating = false;
   return GXC_OK;

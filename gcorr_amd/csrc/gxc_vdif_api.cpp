@@ -47,9 +47,7 @@ gxc_status gxc_set_input_vdif(gxc_handle *h, int station, const void *d_frames, 
   if (st != GXC_OK) return set_err(h, st, why);
   if (!h->vdif) {
     // enter VDIF mode: station pointers to the owned buffer, flags on
-    std::vector<const uint8_t *> ptrs(nant);
-    for (int a = 0; a < nant; a++) ptrs[a] = h->d_input_owned + (size_t)a * h->d.station_bytes;
-    GXC_HIP(h, hipMemcpy(h->d_station_ptrs, ptrs.data(), nant * sizeof(void *), hipMemcpyHostToDevice));
+    GXC_TRY(point_at_owned(h));
     destroy_graph(h);
     h->vdif = true;
     h->input_device = false;

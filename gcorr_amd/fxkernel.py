@@ -176,8 +176,7 @@ class FxKernel:
         """d: [nant][3] polynomial (s, t in FFTs), f: [nant] file offsets (s)."""
         d = np.ascontiguousarray(d, dtype=np.float64).reshape(self.nant, 3)
         f = np.ascontiguousarray(f, dtype=np.float64).reshape(self.nant)
-        rows = (ctypes.POINTER(ctypes.c_double) * self.nant)(
-            *[d[a].ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in range(self.nant)])
+        rows = _lib.row_pointers(d)
         check(self._L.gxc_set_delays(self._h, rows, f.ctypes.data_as(ctypes.POINTER(ctypes.c_double))),
               self._h)
 
@@ -280,8 +279,7 @@ class FxKernel:
         f = np.ascontiguousarray(f, dtype=np.float64).reshape(self.nant)
         ptrs = (ctypes.POINTER(ctypes.c_uint8) * self.nant)(
             *[a.ctypes.data_as(ctypes.POINTER(ctypes.c_uint8)) for a in arrs])
-        rows = (ctypes.POINTER(ctypes.c_double) * self.nant)(
-            *[d[a].ctypes.data_as(ctypes.POINTER(ctypes.c_double)) for a in range(self.nant)])
+        rows = _lib.row_pointers(d)
         check(self._L.gxc_submit(self._h, ptrs, rows, f.ctypes.data_as(ctypes.POINTER(ctypes.c_double))),
               self._h)
         self._inflight.append(arrs)

@@ -372,7 +372,7 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
   const int nant = cfg->nant, nchan = cfg->nchan;
   {
     const size_t ptrs = (size_t)nant * 4 * sizeof(double);  // after the delays
-    if (h->mail.create(ptrs + nant * sizeof(void *), d.nrows * sizeof(int)) != hipSuccess ||
+    if (h->mail.create(ptrs + nant * sizeof(void *), d.nrows * (sizeof(int) + 4 * (sizeof(float) + sizeof(int)))) != hipSuccess ||
         h->out.create((size_t)d.nrows * 4 * nchan * sizeof(float2)) != hipSuccess)
       return fail(set_err(h, GXC_ERR_OUT_OF_MEMORY, "pinned host memory"));
     h->h_delays = reinterpret_cast<double *>(h->mail.h);
@@ -380,6 +380,7 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
     h->h_station_ptrs = reinterpret_cast<const uint8_t **>(h->mail.h + ptrs);
     h->d_station_ptrs = reinterpret_cast<const uint8_t **>(h->mail.d + ptrs);
     h->h_counts = reinterpret_cast<int *>(h->mail.h + h->mail.in);
+    h->h_lag_snr = reinterpret_cast<float *>(h->h_counts + d.nrows);
   }
   if ((s = dmalloc(h, &h->d_valid, (size_t)nant * cfg->numffts)) != GXC_OK) return fail(s);
   std::vector<int2> rm = make_rowmap(nant, cfg->autos != 0);

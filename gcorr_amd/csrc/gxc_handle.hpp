@@ -10,6 +10,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -38,6 +39,8 @@ struct gxc_handle {
   gxc::host::HostOut out;
   const uint8_t **h_station_ptrs = nullptr, **d_station_ptrs = nullptr;  // [nant], in mail
   int *h_counts = nullptr;                                               // [nrows], in mail
+  float *h_lag_snr = nullptr;  // [4 nrows] and the peaks [4 nrows] after it, in mail; under lag_mu
+  std::mutex lag_mu;
 
   // VDIF ingest (gxc_set_input_vdif): payloads go into d_input_owned, and
   // the per-station frame flags make FFTs over missing frames invalid

@@ -98,12 +98,15 @@ gxc_status lag_snr_on(gxc_handle *h, const void *src, hipMemcpyKind kind, int ns
   float *dsnr = nullptr;
   int *dpeak = nullptr;
   gxc_status st = dmalloc(h, &a, n);
-  if (st == GXC_OK) st = dmalloc(h, &b, n);
+  const bool in_lds = gxc::lag_in_lds(nchan);
+  if (st == GXC_OK && !in_lds) st = dmalloc(h, &b, n);
   if (st == GXC_OK) st = dmalloc(h, &dsnr, (size_t)nseries);
   if (st == GXC_OK) st = dmalloc(h, &dpeak, (size_t)nseries);
   hipError_t e = hipSuccess;
   if (st == GXC_OK) e = hipMemcpyAsync(a, src, n * sizeof(float2), kind, s);
-  if (st == GXC_OK && e == hipSuccess) e = gxc::launch_lag_snr(a, b, nchan, nseries, dsnr, dpeak, s);
+  if (st == GXC_OK && e == hipSuccess)
+    e = in_lds ? gxc::launch_lag_series(a, nchan, nseries, dsnr, dpeak, s)
+               : gxc::launch_lag_snr(a, b, nchan, nseries, dsnr, dpeak, s);
   if (st == GXC_OK && e == hipSuccess) e = hipMemcpyAsync(snr, dsnr, nseries * sizeof(float), hipMemcpyDeviceToHost, s);
   if (st == GXC_OK && e == hipSuccess) e = hipMemcpyAsync(peak, dpeak, nseries * sizeof(int), hipMemcpyDeviceToHost, s);
   if (st == GXC_OK && e == hipSuccess) e = hipStreamSynchronize(s);
@@ -120,6 +123,15 @@ gxc_status gxc_lag_snr(gxc_handle *h, float *snr, int *peak, size_t n) {
   if (!h || !snr || !peak) return set_err(h, GXC_ERR_INVALID_ARG, "null argument");
   const int nseries = h->d.nrows * 4;
   if (n < (size_t)nseries) return set_err(h, GXC_ERR_INVALID_ARG, "output arrays too small");
+  if (gxc::lag_in_lds(h->cfg.nchan) && h->cfg.nchan >= 2 && nseries > 0) {
+    std::lock_guard<std::mutex> lock(h->lag_mu);
+    int *h_peak = reinterpret_cast<int *>(h->h_lag_snr + nseries);
+    GXC_HIP(h, gxc::launch_lag_series(h->d_vis, h->cfg.nchan, nseries, h->h_lag_snr, h_peak, h->stream));
+    GXC_HIP(h, hipStreamSynchronize(h->stream));
+    std::memcpy(snr, h->h_lag_snr, nseries * sizeof(float));
+    std::memcpy(peak, h_peak, nseries * sizeof(int));
+    return GXC_OK;
+  }
   GXC_HIP(h, hipStreamSynchronize(h->stream));
   return lag_snr_on(h, h->d_vis, hipMemcpyDeviceToDevice, nseries, h->cfg.nchan, snr, peak, h->stream);
 }

@@ -114,7 +114,7 @@ gxc_status run_xstage(gxc_handle *h, const void *spec, int nt, int accumulate, h
   if (h->xscale > 0.f) {  // FP32 spectra of this handle's own F-stage
     x.scale = h->xscale;
     x.unscale = 1.f / (h->xscale * h->xscale);
-    GXC_HIP(h, gxc::launch_xsplit(x, s));
+    GXC_HIP(h, gxc::launch_xsplit(x, h->out_mode, s));
   } else {
     GXC_HIP(h, gxc::launch_xmfma(x, h->out_mode, h->xtile, s));
   }
@@ -447,7 +447,7 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
   }
   if (out_mode == gxc::OUT_F32) h->xscale = gxc::xsplit_scale(d.L, cfg->is_complex != 0);
   h->splits = cfg->xsplits > 0        ? std::min(cfg->xsplits, h->chunk)
-              : out_mode == gxc::OUT_F32 ? gxc::xsplit_choose_splits(d.M, nchan, h->chunk)
+              : out_mode == gxc::OUT_F32 ? gxc::xsplit_choose_splits(out_mode, d.M, nchan, h->chunk)
                                          : gxc::xm_choose_splits(d.M, nchan, h->chunk, out_mode);
   h->partial_cap = h->splits;
   if ((s = dmalloc(h, reinterpret_cast<unsigned char **>(&h->d_partial),

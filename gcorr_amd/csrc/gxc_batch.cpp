@@ -154,15 +154,23 @@ void mark(gxc_batch *b, int kind, hipStream_t s) {
   b->marks.push_back({kind, idx});
 }
 
-// channels per unit of the X launch
-int x_channels(const gxc_batch *b) {
-  return b->out_mode == gxc::OUT_F32 ? gxc::xsplit_channels(b->M) : gxc::xm_channels_per_group(b->M, b->out_mode);
+// X launch of xsplit.hip: its channel tile divides every subband
+bool x_streams(const gxc_batch *b) {
+  for (const Sub &u : b->sub)
+    if (!gxc::xsplit_channels(b->out_mode, b->M, u.cfg.nchan)) return false;
+  return true;
 }
 
-// Fewest X units per launch worth trying: two FP32 workgroups per CU in turn
-// (8 subbands x 8 stations, X-stage: 3.89 ms with 256 units, 2.47 with 512, 2.50
-// with 1024, 2.61 with 2048), four of the others'.
-int x_units_min(const gxc_batch *b) { return b->out_mode == gxc::OUT_F32 ? 512 : 1024; }
+// channels per unit of the X launch
+int x_channels(const gxc_batch *b) {
+  return x_streams(b) ? gxc::xsplit_channels(b->out_mode, b->M, b->sub[0].cfg.nchan)
+                      : gxc::xm_channels_per_group(b->M, b->out_mode);
+}
+
+// Fewest X units per launch worth trying: two workgroups per CU in turn where
+// one fills it (8 subbands x 8 stations, FP32, X-stage: 3.89 ms with 256 units,
+// 2.47 with 512, 2.50 with 1024, 2.61 with 2048), four of the others'.
+int x_units_min(const gxc_batch *b) { return x_streams(b) ? 512 : 1024; }
 
 // F-stage parameters of subband s, FFTs t0.. (stride tstride), output mode.
 gxc::FParams fparams(const gxc_batch *b, const Sub &u, int t0, int nt, int tstride, int mode, void *out) {
@@ -394,8 +402,8 @@ gxc_status enqueue_device_work(gxc_batch *b) {
       GXB_HIP(b, hipStreamWaitEvent(xs, b->ev_f[buf], 0));
     }
     mark(b, 2, xs);
-    GXB_HIP(b, b->out_mode == gxc::OUT_F32
-                   ? gxc::launch_xsplit_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->M, xs)
+    GXB_HIP(b, x_streams(b)
+                   ? gxc::launch_xsplit_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->out_mode, b->M, xs)
                    : gxc::launch_xmfma_multi(b->d_xseg + (size_t)c * ns, ns, b->xtotal[c], b->out_mode, b->M, xs));
     mark(b, 3, xs);
     if (overlap) GXB_HIP(b, hipEventRecord(b->ev_x[buf], xs));
@@ -580,8 +588,8 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
   b->sub = std::move(subs);
   b->device = dev;
   b->out_mode = out_mode;
-  b->xunits = out_mode == gxc::OUT_F32 ? 512 : 2048;
   b->M = 2 * cfg->nant;
+  b->xunits = x_streams(b) ? 512 : 2048;
   b->nrows = b->sub[0].d.nrows;
   auto fail = [&](gxc_status st) {
     g_batch_error = b->err;

@@ -88,7 +88,7 @@ gxc_status gxc_autotune(gxc_handle *h, gxc_tuning *out) {
   int best_xt = h->xtile, best_sp = h->splits;
   if (st == GXC_OK) {
     const int tb = h->out_mode == gxc::OUT_F32 ? 16 : 32;
-    const int s0 = h->xscale > 0.f ? gxc::xsplit_choose_splits(h->d.M, h->cfg.nchan, nt)
+    const int s0 = h->xscale > 0.f ? gxc::xsplit_choose_splits(h->out_mode, h->d.M, h->cfg.nchan, nt)
                                    : gxc::xm_choose_splits(h->d.M, h->cfg.nchan, nt, h->out_mode);
     const int smax = std::max(1, std::min(1024, nt / (2 * tb)));
     std::vector<int> sps;
@@ -119,7 +119,8 @@ gxc_status gxc_autotune(gxc_handle *h, gxc_tuning *out) {
       }
     }
     int xt[4], nxt = gxc::xm_tiles(h->d.M, h->out_mode, xt);
-    if (h->xscale > 0.f) nxt = 1;  // one channel tile, whatever xtile says
+    if (h->out_mode == gxc::OUT_F32 || (h->out_mode != gxc::OUT_FP8 && h->d.M <= 32))
+      nxt = 1;  // one channel tile, whatever xtile says
     for (int i = 0; i < nxt && st == GXC_OK; i++) {
       if (h->cfg.nchan % xt[i]) continue;
       h->xtile = xt[i];

@@ -21,7 +21,7 @@ struct XMParams {
                         // chunks (Neumaier), or null (one chunk)
   int nt, M, nchan, splits;
   int accumulate;       // add into partial instead of overwriting
-  float scale, unscale; // launch_xsplit: xsplit_scale and 1 / scale^2
+  float scale, unscale; // launch_xsplit, FP32: xsplit_scale and 1 / scale^2
 };
 
 struct FinMParams {
@@ -59,18 +59,20 @@ int xm_choose_splits(int M, int nchan, int nt, int out_mode);
 size_t xm_partial_bytes(int M, int nchan, int splits);
 int xm_element_bytes(int out_mode);   // bytes of one packed complex value
 
-// ct: channel tile, one of xm_tiles (0 = default; FP32 has the default only)
+// ct: channel tile, one of xm_tiles (0 = default; FP32, and FP16 and BF16 up to
+// 32 inputs, have the default only)
 hipError_t launch_xmfma(const XMParams &p, int out_mode, int ct, hipStream_t s);
-// The same for FP32 spectra that an F-stage of this build wrote (xsplit.hip):
-// p.scale and p.unscale set, nchan a multiple of xsplit_channels, the
-// channels of a workgroup.
-int xsplit_channels(int M);
+// The streaming form (xsplit.hip): FP16 and BF16 spectra of up to 32 inputs,
+// and FP32 spectra that an F-stage of this build wrote (p.scale and p.unscale
+// set).  xsplit_channels: the channels of its workgroup, 0 where it does not
+// cover the shape.
+int xsplit_channels(int out_mode, int M, int nchan);
 float xsplit_scale(int L, bool cplx);
-int xsplit_choose_splits(int M, int nchan, int nt);
-hipError_t launch_xsplit(const XMParams &p, hipStream_t s);
-hipError_t launch_xsplit_multi(const XSeg *segs, int nseg, long long total, int M, hipStream_t s);
+int xsplit_choose_splits(int out_mode, int M, int nchan, int nt);
+hipError_t launch_xsplit(const XMParams &p, int out_mode, hipStream_t s);
+hipError_t launch_xsplit_multi(const XSeg *segs, int nseg, long long total, int out_mode, int M, hipStream_t s);
 // Channel tiles that gxc_config.xtile may name for M inputs (default first);
-// returns the count (<= 3).  FP32 handles run launch_xsplit's one tile.
+// returns the count (<= 3).  Where launch_xsplit runs it has one tile.
 int xm_tiles(int M, int out_mode, int *out);
 // scales[i] = power of two nearest target / sqrt(mean_r power[r][i]), r < nrows.
 hipError_t launch_scales(float *scales, const float *power, int n, int nrows, float target, hipStream_t s);

@@ -12,9 +12,11 @@
 // P1 = R_i R_j^T, P2 = I_i I_j^T, P3 = (R_i + I_i)(R_j - I_j)^T, with
 // Re V = P1 + P2 and Im V = P3 - P1 + P2 (the packed forms are read from
 // HBM at full speed with the MFMAs mostly idle, and their sums R + I would
-// add a rounding).  FP32 here serves spectra that a caller hands in, of any
-// magnitude; those of the F-stage, whose magnitude is bounded, are taken by
-// xsplit.hip in half to two thirds of the time.
+// add a rounding).
+//
+// Runs here: FP8; FP16 and BF16 at 33 and more inputs (or a channel count that
+// is no multiple of 64); FP32 spectra that a caller hands in, of any magnitude.
+// xsplit.hip takes the rest in half to nine tenths of the time.
 //
 // The F-stage writes spectra channel-contiguous ([t][input][chan]), the
 // layout its last FFT pass stores coalesced.  Each workgroup stages a
@@ -671,9 +673,11 @@ hipError_t launch_xm_multi(const XSeg *segs, int nseg, long long total, hipStrea
 
 template <int ET>
 hipError_t launch_xm_multi_mb(const XSeg *segs, int nseg, long long total, int M, hipStream_t s) {
+  if constexpr (ET == OUT_FP8) {  // FP16 and BF16 go through launch_xsplit_multi up to 32 inputs
+    if (xm_blocks(M) == 1) return launch_xm_multi<ET, 1>(segs, nseg, total, s);
+    if (xm_blocks(M) == 2) return launch_xm_multi<ET, 2>(segs, nseg, total, s);
+  }
   switch (xm_blocks(M)) {
-    case 1: return launch_xm_multi<ET, 1>(segs, nseg, total, s);
-    case 2: return launch_xm_multi<ET, 2>(segs, nseg, total, s);
     case 4: return launch_xm_multi<ET, 4>(segs, nseg, total, s);
     default: return hipErrorInvalidValue;
   }
@@ -682,8 +686,9 @@ hipError_t launch_xm_multi_mb(const XSeg *segs, int nseg, long long total, int M
 template <int ET, int MB>
 hipError_t launch_xm_ct(const XMParams &p, int ct, hipStream_t s) {
   constexpr int D = xm_default_ct(ET, MB);
-  if (ET == OUT_F32 || ct == 0 || ct == D) return launch_xm<ET, MB, D>(p, s);
-  if constexpr (ET != OUT_F32) {
+  constexpr bool one = ET == OUT_F32 || (ET != OUT_FP8 && MB <= 2);
+  if (one || ct == 0 || ct == D) return launch_xm<ET, MB, D>(p, s);
+  if constexpr (!one) {
     if (ct == D / 2) return launch_xm_if<ET, MB, D / 2>(p, s);
     if (ct == 2 * D) return launch_xm_if<ET, MB, 2 * D>(p, s);
   }
@@ -738,6 +743,7 @@ int xm_channels_per_group(int M, int out_mode) {
 int xm_choose_splits(int M, int nchan, int nt, int out_mode) {
   const int ct = xm_channels_per_group(M, out_mode);
   if (ct == 0) return 1;
+  if (out_mode != OUT_F32 && xsplit_channels(out_mode, M, nchan)) return xsplit_choose_splits(out_mode, M, nchan, nt);
   const long long groups = nchan / ct;
   const int tb = out_mode == OUT_F32 ? 16 : 32;
   long long s = (1024 + groups - 1) / groups;  // ~4 workgroups per CU
@@ -761,6 +767,7 @@ float xm_target_rms(int out_mode) {
 }
 
 hipError_t launch_xmfma(const XMParams &p, int out_mode, int ct, hipStream_t s) {
+  if (out_mode != OUT_F32 && xsplit_channels(out_mode, p.M, p.nchan)) return launch_xsplit(p, out_mode, s);
   switch (out_mode) {
     case OUT_F32: return launch_xm_mb<OUT_F32>(p, ct, s);
     case OUT_F16: return launch_xm_mb<OUT_F16>(p, ct, s);

@@ -1,16 +1,19 @@
-// X-stage of the F-stage's FP32 spectra on the f16 matrix cores: every value
-// x is taken as hi + lo, two f16 (x - hi is exact and has at most 13 bits, of
-// which lo keeps 11 and its sign: 2^-24 of x, an FP32 rounding), and every
-// product x y as hi hi + hi lo + lo hi with FP32 sums.  The term left out, lo
-// lo, is 2^-24 of the product and of random sign, except where an input meets
-// itself: the blocks on the diagonal take it as well.
+// Streaming X-stage: FP16 and BF16 spectra of up to 32 inputs, and the F-stage's
+// FP32 spectra, on the 16-bit matrix cores.
+//
+// FP32: every value x is taken as hi + lo, two f16 (x - hi is exact and has at
+// most 13 bits, of which lo keeps 11 and its sign: 2^-24 of x, an FP32
+// rounding), and every product x y as hi hi + hi lo + lo hi with FP32 sums.  The
+// term left out, lo lo, is 2^-24 of the product and of random sign, except
+// where an input meets itself: the blocks on the diagonal take it as well.
 //
 // For channel c over FFTs t, with x_a = a_a + i b_a (a = input index):
 //   Re V_ab = sum_t a_a a_b + b_a b_b,  Im V_ab = sum_t b_a a_b - a_a b_b
 // so with K slots (a, b) of 16 FFTs one v_mfma_f32_16x16x32_f16 of the slots
-// [a, b] with [a, b] adds to Re, and one with [-b, a] to Im.
+// [a, b] with [a, b] adds to Re, and one with [-b, a] to Im.  A 16-bit complex
+// value is such a slot pair as it lies in memory.
 //
-// The spectra come from the framework's own F-stage, whose |X| is at most L
+// The FP32 spectra come from the framework's own F-stage, whose |X| is at most L
 // times the largest sample: p.scale, a power of two, brings that below f16's
 // largest value.  2-bit noise (rms sqrt(L) and more) then lies above 54, f16's
 // lo parts lose bits below 2^-2; complex noise of one level rms lies above 1
@@ -20,21 +23,23 @@
 // What bounds it is the reading of the spectra: the FP32 matrix products that
 // it replaces kept the MFMAs busy for 70 % of the time, here they, the VALU
 // (the split: about 20 instructions per value and wave) and LDS are busy for
-// 15-30 %.  A workgroup takes 32 channels (33 and more inputs: 16) of all M
-// inputs, so that a row is 256 bytes (with 128 the same kernel read 5.5
-// instead of 6.2 TB/s; a plain read of this pattern reaches 5.5-6.2 and 6.4).
-// Stages of SB FFTs go straight from memory to LDS in 16-byte units (two
-// channels) into a ring of five, four of them under way; the lanes of a row
-// take its units in an order rotated by the row, so that the 16 lanes of an
-// operand read find 16 distinct bank groups.  A wave owns two neighbouring
-// channels (33 and more inputs: one), so each value is read from LDS and split
-// once.  Nontemporal loads, since a row is read once: 3.21 -> 2.94 ms at 16
-// stations before the ring.
-// X-stage, FP32 products -> this: 16 stations x 4096 channels x 15625 FFTs 3.18
-// -> 2.64 ms (6.2 TB/s), 6 x 1024 x 62500 1.16 -> 0.93 ms, 32 x 1024 x 6000
+// 15-30 %.  A workgroup takes 32 channels (FP32, 33 and more inputs: 16; 16-bit:
+// 64) of all M inputs, so that a row is 256 bytes (with 128 the same kernel read
+// 5.5 instead of 6.2 TB/s; a plain read of this pattern reaches 5.5-6.2 and
+// 6.4).  Stages of SB FFTs go straight from memory to LDS in 16-byte units into
+// a ring of five, four of them under way; the lanes of a row take its units in
+// an order rotated by the row, so that the 16 lanes of an operand read find 16
+// distinct bank groups.  A wave owns the channels of one unit (33 and more
+// inputs: one channel), so each value is read from LDS and split once.
+// Nontemporal loads, since a row is read once: 3.21 -> 2.94 ms at 16 stations
+// before the ring.
+// X-stage, before -> with this, FP32: 16 stations x 4096 channels x 15625 FFTs
+// 3.18 -> 2.64 ms (6.2 TB/s), 6 x 1024 x 62500 1.16 -> 0.93 ms, 32 x 1024 x 6000
 // 1.15 -> 0.63 ms, a batch of 8 subbands x 8 stations 3.45 -> 2.47 ms.  Errors of
 // the visibilities against 64 bits (with the F-stage's): 3.6e-7 -> 1.4e-7, 5.1e-7
-// -> 1.6e-7, 4.5e-7 -> 4.0e-7, 9.5e-7 -> 3.3e-7.
+// -> 1.6e-7, 4.5e-7 -> 4.0e-7, 9.5e-7 -> 3.3e-7.  16-bit (loads through registers,
+// one stage ahead, 8 or 16 FFTs transposed per lane): 16 x 4096 x 15625 1.46 ->
+// 1.41 ms, 10 x 2048 x 5001 0.217 -> 0.143 ms, 8 x 32768 x 1000 0.460 -> 0.367 ms.
 #include <algorithm>
 #include <cmath>
 
@@ -54,26 +59,54 @@ constexpr int kNontemporal = 2;                               // cache policy of
 constexpr int kVmcnt(int n) { return 0x0f70 | (n & 15); }  // s_waitcnt vmcnt(n), n < 16
 
 
-template <int MB>
+template <int ET, int MB>
 struct XS {
-  static constexpr int CT = MB == 4 ? 16 : 32;  // channels of a workgroup
-  static constexpr int CPW = MB == 4 ? 1 : 2;    // channels per wave
+  static constexpr bool F32 = ET == OUT_F32;
+  static constexpr int CB = F32 ? 8 : 4;           // bytes of a complex value
+  static constexpr int CT = F32 ? (MB == 4 ? 16 : 32) : 64;  // channels of a workgroup
+  static constexpr int CPW = F32 ? (MB == 4 ? 1 : 2) : 4;    // channels per wave
   static constexpr int NWV = CT / CPW, NTHR = 64 * NWV;
-  static constexpr int UPR = CT / 2, RPI = 64 / UPR;  // 16-byte units per row, rows per load instruction
-    // unit u of a row lies at position u ^ swz(row)
+  static constexpr int ROWB = CT * CB;
+  static constexpr int UPR = ROWB / 16, RPI = 64 / UPR;  // 16-byte units per row, rows per load instruction
+  // unit u of a row lies at position u ^ swz(row)
   __device__ static constexpr int swz(int row) { return UPR == 8 ? (row >> 1) & 7 : row & 15; }
   static constexpr int SB = MB == 1 ? 8 : 4;   // FFTs per stage
   static constexpr int NU = SB / 4;            // a lane's units of an input and stage
-  static constexpr int NST = 16 / SB;          // stages per MFMA K-step of 16 FFTs
-  static constexpr int RING = 5;               // stages in LDS: 80 KiB at 16 and 32 inputs, 160 at 64
+  // FFTs per MFMA: 16 (K = 32), or 8 (K = 16) where the 96 running sums of four
+  // channels leave no registers for the operands of 16
+  static constexpr int KF = !F32 && MB == 2 ? 8 : 16, KD = KF / 4;
+  static constexpr int NST = KF / SB;          // stages per MFMA K-step
+  static constexpr int RING = 5;               // stages in LDS: 160 KiB at 16, 32 and 64 inputs
   static constexpr int NTILE = MB * (MB + 1) / 2;
-  // rows of CT channels: the stages', and those that padded inputs of the last FFT read
-  static int lds_bytes(int M) { return 8 * CT * (RING * SB * M + 16 * MB - M); }
+  // the stages' rows, and those that padded inputs of the last FFT read
+  static int lds_bytes(int M) { return ROWB * (RING * SB * M + 16 * MB - M); }
 };
 
-__device__ __forceinline__ floatx4 mfma16(const uint4 &a, const uint4 &b, floatx4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
-                                                0);
+// An MFMA operand of one lane: KD pairs (a, b), one per FFT.
+template <int KD>
+struct Op {
+  uint32_t d[KD];
+};
+typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short short4v __attribute__((ext_vector_type(4)));
+template <int ET>
+__device__ __forceinline__ floatx4 mfma(const Op<4> &a, const Op<4> &b, floatx4 c) {
+  if constexpr (ET == OUT_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
+                                                    0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
+                                                   0);
+}
+template <int ET>
+__device__ __forceinline__ floatx4 mfma(const Op<2> &a, const Op<2> &b, floatx4 c) {
+  if constexpr (ET == OUT_BF16)
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(short4v, a), __builtin_bit_cast(short4v, b), c,
+                                                     0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_16x16x16f16(__builtin_bit_cast(half4, a), __builtin_bit_cast(half4, b), c, 0, 0,
+                                                 0);
 }
 
 // (re, im) * scale as an f16 pair and the f16 pair of the remainder
@@ -86,8 +119,13 @@ __device__ __forceinline__ void split(float re, float im, float scale, uint32_t 
 }
 
 // [a, b] -> [-b, a]
-__device__ __forceinline__ uint32_t turn(uint32_t v) { return __builtin_amdgcn_alignbit(v, v, 16) ^ 0x00008000u; }
-__device__ __forceinline__ uint4 turn(const uint4 &v) { return make_uint4(turn(v.x), turn(v.y), turn(v.z), turn(v.w)); }
+template <int KD>
+__device__ __forceinline__ Op<KD> turn(const Op<KD> &v) {
+  Op<KD> w;
+#pragma unroll
+  for (int i = 0; i < KD; i++) w.d[i] = __builtin_amdgcn_alignbit(v.d[i], v.d[i], 16) ^ 0x00008000u;
+  return w;
+}
 
 typedef __attribute__((address_space(1))) void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
@@ -104,7 +142,7 @@ __device__ __forceinline__ void read_units(floatx4 &a, floatx4 &b, unsigned addr
 __device__ __forceinline__ void read_blocks(floatx4 &a, floatx4 &b, unsigned addr) {
   asm volatile("ds_read_b128 %0, %2\n\tds_read_b128 %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
                : "=&v"(a), "=&v"(b)
-               : "v"(addr), "n"(16 * 8 * XS<2>::CT)
+               : "v"(addr), "n"(16 * 256)
                : "memory");
 }
 __device__ __forceinline__ void read_blocks(floatx2 &a, floatx2 &b, floatx2 &c, floatx2 &d, unsigned addr) {
@@ -119,19 +157,20 @@ __device__ __forceinline__ void read_blocks(floatx2 &a, floatx2 &b, floatx2 &c, 
 // Channels CT group .., FFT split `unit_split`, on a workgroup of XS::NTHR
 // threads (every thread calls it with the same arguments: it contains
 // barriers).  lds holds XS::lds_bytes(M) bytes, 16-byte aligned.
-template <int MB>
+template <int ET, int MB>
 __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int unit_split, unsigned char *lds) {
   const int group = __builtin_amdgcn_readfirstlane(group_), split_ = __builtin_amdgcn_readfirstlane(unit_split);
-  using X = XS<MB>;
-  constexpr int CPW = X::CPW, SB = X::SB;
+  using X = XS<ET, MB>;
+  constexpr int CPW = X::CPW, SB = X::SB, KD = X::KD;
+  static_assert(X::F32 || X::ROWB == 256, "read_blocks");
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int M = p.M, l15 = lane & 15, g = lane >> 4;
   // uniform, which 64-bit divisions on the VALU hide
   const int tb = __builtin_amdgcn_readfirstlane((int)((long long)p.nt * split_ / p.splits));
   const int te = __builtin_amdgcn_readfirstlane((int)((long long)p.nt * (split_ + 1) / p.splits));
-  const size_t rowbytes = (size_t)p.nchan * 8;
-  const unsigned char *src = static_cast<const unsigned char *>(p.spectra) + (size_t)group * (8 * X::CT);
-  const int stage_bytes = SB * M * 8 * X::CT;
+  const size_t rowbytes = (size_t)p.nchan * X::CB;
+  const unsigned char *src = static_cast<const unsigned char *>(p.spectra) + (size_t)group * X::ROWB;
+  const int stage_bytes = SB * M * X::ROWB;
 
   // A wave's load instruction fills 64 units, RPI rows (row = t M + input) of
   // a stage; it has nld, at most two, per stage, NWV RPI rows apart (a multiple
@@ -154,12 +193,12 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
   // operand reads: FFT 4 u + g of a stage, input 16 b + l15.  (Lanes of
   // inputs past M read other rows: what they make of them lands in rows and
   // columns past M.)
-  const int pw = CPW == 2 ? wave : wave >> 1;
+  const int pw = CPW == 1 ? wave >> 1 : wave;
   unsigned addr[X::NU];
 #pragma unroll
   for (int u = 0; u < X::NU; u++) {
     const int row = (4 * u + g) * M + l15;
-    addr[u] = (unsigned)(uintptr_t)(lvoid *)lds + row * 8 * X::CT + 16 * (pw ^ X::swz(row)) +
+    addr[u] = (unsigned)(uintptr_t)(lvoid *)lds + row * X::ROWB + 16 * (pw ^ X::swz(row)) +
               (CPW == 1 ? 8 * (wave & 1) : 0);
   }
 
@@ -169,12 +208,12 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
 #pragma unroll
     for (int t = 0; t < X::NTILE; t++) re[c][t] = im[c][t] = floatx4{0, 0, 0, 0};
 
-  const int nst = tb < te ? (te - tb + 15) / 16 * X::NST : 0;  // stages
+  const int nst = tb < te ? (te - tb + X::KF - 1) / X::KF * X::NST : 0;  // stages
   for (int n = 0; n < X::RING - 1 && n < nst; n++) request(tb + n * SB, n);
   int slot = 0;
   for (int n0 = 0; n0 < nst; n0 += X::NST) {
-    typedef float unit __attribute__((ext_vector_type(2 * CPW)));
-    uint4 H[CPW][MB], L[CPW][MB];  // K slots: FFTs 4 i + g, i = 0..3 in .x .. .w
+    typedef float unit __attribute__((ext_vector_type(CPW == 1 ? 2 : 4)));
+    Op<KD> H[CPW][MB], L[CPW][MB];  // K slots: FFTs 4 i + g in d[i]; L: FP32 only
 #pragma unroll
     for (int s = 0; s < X::NST; s++) {
       const int n = n0 + s;
@@ -209,9 +248,13 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
 #pragma unroll
         for (int c = 0; c < CPW; c++)
 #pragma unroll
-          for (int b = 0; b < MB; b++)
-            split(raw[b][u][2 * c], raw[b][u][2 * c + 1], p.scale, (&H[c][b].x)[s * X::NU + u],
-                  (&L[c][b].x)[s * X::NU + u]);
+          for (int b = 0; b < MB; b++) {
+            uint32_t &h = H[c][b].d[s * X::NU + u];
+            if constexpr (X::F32)
+              split(raw[b][u][2 * c], raw[b][u][2 * c + 1], p.scale, h, L[c][b].d[s * X::NU + u]);
+            else
+              h = __builtin_bit_cast(uint32_t, (float)raw[b][u][c]);
+          }
       }
     }
 #pragma unroll
@@ -219,11 +262,11 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
 #pragma unroll
       for (int bj = 0; bj < MB; bj++) {
         // The products of one kind for all blocks of a column, then the next:
-        // two MFMAs on one sum are MB others apart.  Up to 32 inputs a K-step's
-        // products are summed by themselves, small ones first, and added once
-        // (one rounding of the running sum instead of four); at 64 inputs the
-        // registers hold only the running sums.
-        constexpr bool OWN = MB <= 2;
+        // two MFMAs on one sum are MB others apart.  FP32, up to 32 inputs: a
+        // K-step's products are summed by themselves, small ones first, and
+        // added once (one rounding of the running sum instead of four); at 64
+        // inputs the registers hold only the running sums.
+        constexpr bool OWN = X::F32 && MB <= 2;
         floatx4 *sr = re[c] + bj * (bj + 1) / 2, *sq = im[c] + bj * (bj + 1) / 2;
         floatx4 r[MB], q[MB];
 #pragma unroll
@@ -231,23 +274,27 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
           r[bi] = OWN ? floatx4{0, 0, 0, 0} : sr[bi];
           q[bi] = OWN ? floatx4{0, 0, 0, 0} : sq[bi];
         }
-        r[bj] = mfma16(L[c][bj], L[c][bj], r[bj]);
-        uint4 w = turn(L[c][bj]);
+        if constexpr (X::F32) {
+          r[bj] = mfma<ET>(L[c][bj], L[c][bj], r[bj]);
+          const Op<KD> w = turn(L[c][bj]);
 #pragma unroll
-        for (int bi = 0; bi <= bj; bi++) {
-          r[bi] = mfma16(H[c][bi], L[c][bj], r[bi]);
-          q[bi] = mfma16(H[c][bi], w, q[bi]);
+          for (int bi = 0; bi <= bj; bi++) {
+            r[bi] = mfma<ET>(H[c][bi], L[c][bj], r[bi]);
+            q[bi] = mfma<ET>(H[c][bi], w, q[bi]);
+          }
         }
-        w = turn(H[c][bj]);
+        const Op<KD> w = turn(H[c][bj]);
+        if constexpr (X::F32) {
 #pragma unroll
-        for (int bi = 0; bi <= bj; bi++) {
-          r[bi] = mfma16(L[c][bi], H[c][bj], r[bi]);
-          q[bi] = mfma16(L[c][bi], w, q[bi]);
+          for (int bi = 0; bi <= bj; bi++) {
+            r[bi] = mfma<ET>(L[c][bi], H[c][bj], r[bi]);
+            q[bi] = mfma<ET>(L[c][bi], w, q[bi]);
+          }
         }
 #pragma unroll
         for (int bi = 0; bi <= bj; bi++) {
-          r[bi] = mfma16(H[c][bi], H[c][bj], r[bi]);
-          q[bi] = mfma16(H[c][bi], w, q[bi]);
+          r[bi] = mfma<ET>(H[c][bi], H[c][bj], r[bi]);
+          q[bi] = mfma<ET>(H[c][bi], w, q[bi]);
         }
 #pragma unroll
         for (int bi = 0; bi <= bj; bi++) {
@@ -266,7 +313,7 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
   int zero = 0;
   asm volatile("" : "+s"(zero));  // the lane is worked out here, not held over the loop
   const int tid = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
-  const float us = p.unscale, ush = 0.5f * p.unscale;
+  const float us = X::F32 ? p.unscale : 1.f, ush = 0.5f * us;
 #pragma unroll
   for (int c = 0; c < CPW; c++) {
     const int ch = group * X::CT + wave * CPW + c;
@@ -291,78 +338,93 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
   }
 }
 
-template <int MB>
-__global__ void __launch_bounds__(XS<MB>::NTHR) __attribute__((amdgpu_waves_per_eu(4))) xsplit_kernel(XMParams p) {
+template <int ET, int MB>
+__global__ void __launch_bounds__((XS<ET, MB>::NTHR)) __attribute__((amdgpu_waves_per_eu(4))) xsplit_kernel(XMParams p) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
-  const int groups = p.nchan / XS<MB>::CT;
+  const int groups = p.nchan / XS<ET, MB>::CT;
   const long long u = xcd_swizzle(blockIdx.x, (long long)groups * p.splits);
-  xsplit_item<MB>(p, (int)(u % groups), (int)(u / groups), lds);
+  xsplit_item<ET, MB>(p, (int)(u % groups), (int)(u / groups), lds);
 }
 
 // Several subbands of the same M: unit = (subband, split, channel group), a
 // workgroup each.
-template <int MB>
-__global__ void __launch_bounds__(XS<MB>::NTHR) __attribute__((amdgpu_waves_per_eu(4)))
+template <int ET, int MB>
+__global__ void __launch_bounds__((XS<ET, MB>::NTHR)) __attribute__((amdgpu_waves_per_eu(4)))
 xsplit_multi_kernel(const XSeg *__restrict__ segs, int nseg) {
   extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
   const long long u = xcd_swizzle(blockIdx.x, gridDim.x);
   const int k = __builtin_amdgcn_readfirstlane(find_seg(segs, nseg, u));
   const XMParams p = segs[k].p;
-  const int local = (int)(u - segs[k].unit0), groups = p.nchan / XS<MB>::CT;
-  xsplit_item<MB>(p, local % groups, local / groups, lds);
+  const int local = (int)(u - segs[k].unit0), groups = p.nchan / XS<ET, MB>::CT;
+  xsplit_item<ET, MB>(p, local % groups, local / groups, lds);
 }
 
-template <int MB>
+template <int ET, int MB>
 hipError_t launch_mb(const XMParams &p, hipStream_t s) {
-  const long long units = (long long)(p.nchan / XS<MB>::CT) * p.splits;
-  if (p.nchan % XS<MB>::CT || units > 0x7fffffffLL) return hipErrorInvalidValue;
-  const int lds = XS<MB>::lds_bytes(p.M);
+  using X = XS<ET, MB>;
+  const long long units = (long long)(p.nchan / X::CT) * p.splits;
+  if (p.nchan % X::CT || units > 0x7fffffffLL) return hipErrorInvalidValue;
   const hipError_t e =
-      allow_dynamic_lds(reinterpret_cast<const void *>(&xsplit_kernel<MB>), XS<MB>::lds_bytes(16 * MB));
+      allow_dynamic_lds(reinterpret_cast<const void *>(&xsplit_kernel<ET, MB>), X::lds_bytes(16 * MB));
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((xsplit_kernel<MB>), dim3((unsigned)units), dim3(XS<MB>::NTHR), lds, s, p);
+  hipLaunchKernelGGL((xsplit_kernel<ET, MB>), dim3((unsigned)units), dim3(X::NTHR), X::lds_bytes(p.M), s, p);
   return hipGetLastError();
 }
 
-template <int MB>
+template <int ET, int MB>
 hipError_t launch_multi_mb(const XSeg *segs, int nseg, long long total, int M, hipStream_t s) {
-  const void *fn = reinterpret_cast<const void *>(&xsplit_multi_kernel<MB>);
-  const int lds = XS<MB>::lds_bytes(M);
-  const hipError_t e = allow_dynamic_lds(fn, XS<MB>::lds_bytes(16 * MB));
+  using X = XS<ET, MB>;
+  const void *fn = reinterpret_cast<const void *>(&xsplit_multi_kernel<ET, MB>);
+  const hipError_t e = allow_dynamic_lds(fn, X::lds_bytes(16 * MB));
   if (e != hipSuccess) return e;
   if (total > 0x7fffffffLL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((xsplit_multi_kernel<MB>), dim3((unsigned)total), dim3(XS<MB>::NTHR), lds, s, segs, nseg);
+  hipLaunchKernelGGL((xsplit_multi_kernel<ET, MB>), dim3((unsigned)total), dim3(X::NTHR), X::lds_bytes(M), s, segs,
+                     nseg);
   return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t launch_xsplit(const XMParams &p, hipStream_t s) {
-  switch (xm_blocks(p.M)) {
-    case 1: return launch_mb<1>(p, s);
-    case 2: return launch_mb<2>(p, s);
-    case 4: return launch_mb<4>(p, s);
+hipError_t launch_xsplit(const XMParams &p, int out_mode, hipStream_t s) {
+  const int mb = xm_blocks(p.M);
+  switch (out_mode * 8 + mb) {
+    case OUT_F32 * 8 + 1: return launch_mb<OUT_F32, 1>(p, s);
+    case OUT_F32 * 8 + 2: return launch_mb<OUT_F32, 2>(p, s);
+    case OUT_F32 * 8 + 4: return launch_mb<OUT_F32, 4>(p, s);
+    case OUT_F16 * 8 + 1: return launch_mb<OUT_F16, 1>(p, s);
+    case OUT_F16 * 8 + 2: return launch_mb<OUT_F16, 2>(p, s);
+    case OUT_BF16 * 8 + 1: return launch_mb<OUT_BF16, 1>(p, s);
+    case OUT_BF16 * 8 + 2: return launch_mb<OUT_BF16, 2>(p, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-hipError_t launch_xsplit_multi(const XSeg *segs, int nseg, long long total, int M, hipStream_t s) {
+hipError_t launch_xsplit_multi(const XSeg *segs, int nseg, long long total, int out_mode, int M, hipStream_t s) {
   if (total <= 0) return hipSuccess;
-  switch (xm_blocks(M)) {
-    case 1: return launch_multi_mb<1>(segs, nseg, total, M, s);
-    case 2: return launch_multi_mb<2>(segs, nseg, total, M, s);
-    case 4: return launch_multi_mb<4>(segs, nseg, total, M, s);
+  switch (out_mode * 8 + xm_blocks(M)) {
+    case OUT_F32 * 8 + 1: return launch_multi_mb<OUT_F32, 1>(segs, nseg, total, M, s);
+    case OUT_F32 * 8 + 2: return launch_multi_mb<OUT_F32, 2>(segs, nseg, total, M, s);
+    case OUT_F32 * 8 + 4: return launch_multi_mb<OUT_F32, 4>(segs, nseg, total, M, s);
+    case OUT_F16 * 8 + 1: return launch_multi_mb<OUT_F16, 1>(segs, nseg, total, M, s);
+    case OUT_F16 * 8 + 2: return launch_multi_mb<OUT_F16, 2>(segs, nseg, total, M, s);
+    case OUT_BF16 * 8 + 1: return launch_multi_mb<OUT_BF16, 1>(segs, nseg, total, M, s);
+    case OUT_BF16 * 8 + 2: return launch_multi_mb<OUT_BF16, 2>(segs, nseg, total, M, s);
     default: return hipErrorInvalidValue;
   }
 }
 
-int xsplit_channels(int M) { return M > 32 ? XS<4>::CT : XS<1>::CT; }
+int xsplit_channels(int out_mode, int M, int nchan) {
+  const int ct = out_mode == OUT_F32                        ? (M > 32 ? 16 : 32)
+                 : out_mode == OUT_F16 || out_mode == OUT_BF16 ? (M > 32 ? 0 : 64)
+                                                               : 0;
+  return ct && nchan % ct == 0 ? ct : 0;
+}
 
 // One workgroup per CU, which its LDS admits at 16, 32 and 64 inputs, where
 // there are FFTs enough: 6 stations x 1024 channels 0.93 ms with 256
 // workgroups, 0.96 with 512; 16 x 4096 2.59 with 256, 2.64 with 1024.
-int xsplit_choose_splits(int M, int nchan, int nt) {
-  const long long groups = nchan / xsplit_channels(M);
+int xsplit_choose_splits(int out_mode, int M, int nchan, int nt) {
+  const long long groups = nchan / std::max(1, xsplit_channels(out_mode, M, nchan));
   long long s = (256 + groups - 1) / groups;
   s = std::min<long long>(s, std::max(1, nt / 32));
   return (int)std::max(1LL, std::min(s, 256LL));

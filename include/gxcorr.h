@@ -94,8 +94,9 @@ typedef struct {
                       size (fftchannels/16 times a power of two, or
                       fftchannels/32), which all name the one kernel of the
                       length */
-  int xtile;       /* X-stage channel tile (channels per workgroup); FP32
-                      has one tile, which every accepted value runs */
+  int xtile;       /* X-stage channel tile (channels per workgroup); FP32,
+                      and FP16 and BF16 up to 16 stations, have one tile,
+                      which every accepted value runs */
   int xsplits;     /* X-stage FFT splits (workgroups per channel tile) */
   int reserved[1];
 } gxc_config;

@@ -1,5 +1,7 @@
-"""The X-stage of FP32 handles (f16 hi + lo products) against 64-bit sums of
-the same spectra and against the general X-stage (FP32 products).
+"""The streaming X-stage: FP32 handles (f16 hi + lo products) against 64-bit sums
+of the same spectra and against the general X-stage (FP32 products); FP16 and
+BF16 against the general X-stage, which takes the channel counts that the
+streaming one does not.
 
 V_ab / sqrt(V_aa V_bb) must agree to 1e-6 of 64-bit sums: per product, hi + lo
 of either factor rounds by 2^-24 and the dropped term is 2^-24 at most; a sum
@@ -84,3 +86,15 @@ def test_largest_spectra(gpu, nchan, is_complex):
     want = (L * 128.0) ** 2 * 2 if is_complex else (L * float(np.float32(3.3359))) ** 2
     np.testing.assert_allclose(v[:, :, 0].real, want, rtol=2e-6)
     assert np.all(np.isfinite(v.view(np.float32)))
+
+
+@pytest.mark.parametrize("precision", ["fp16", "bf16"])
+@pytest.mark.parametrize("nant,nfft", [(1, 1), (3, 7), (8, 16), (8, 33), (9, 100), (13, 8), (16, 41), (16, 100)])
+def test_16_bit_matches_general_path(gpu, precision, nant, nfft):
+    """The first 32 of 64 channels (streaming) and the 32 alone (general)."""
+    rng = np.random.default_rng(nant * 100 + nfft)
+    spec = (rng.standard_normal((nfft, 2 * nant, 64)) + 1j * rng.standard_normal((nfft, 2 * nant, 64))).astype(np.complex64)
+    got = gcorr_amd.xengine(spec, nant, autos=True, precision=precision)[..., :32].astype(np.complex128)
+    want = gcorr_amd.xengine(spec[..., :32], nant, autos=True, precision=precision).astype(np.complex128)
+    _, scale = reference(spec[..., :32], rows_of(nant))
+    assert np.max(np.abs(got - want) * nfft / scale) < TOL

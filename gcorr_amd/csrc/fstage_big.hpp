@@ -11,11 +11,12 @@
 // waves, with both polarisations side by side, and with a pipeline over items
 // in a persistent workgroup all measured 3-15 % slower at 8192 points (their
 // waves met at barriers more often and wrote as much LDS).
-// What bounds it: VALU issue and LDS writes (~80 bytes per clock and CU), each
-// about half of the time.  16 stations x 4096 channels x 4096 FFTs (FP32, 4.3
-// GB of spectra): 6.7 ms with the first pass on the VALU and both
-// polarisations in registers, 6.1 ms now; 6 stations x 1024 channels 3.3 ->
-// 2.3 ms, 10 stations x 2048 channels (BF16) 1.05 -> 0.54 ms.
+// What bounds it: VALU issue (45 instructions per point, ~2.7 cycles each: 4 of
+// the 5.8 ms below) and LDS writes (~80 bytes per clock and CU: 2 ms), which 16
+// waves per CU overlap in part.  16 stations x 4096 channels x 15625 FFTs (FP32,
+// 16.4 GB of spectra): 6.7 ms with the first pass on the VALU and both
+// polarisations in registers, 5.8 ms now; 6 stations x 1024 channels 3.3 -> 2.26
+// ms, 10 stations x 2048 channels (BF16) 1.05 -> 0.49 ms.
 #pragma once
 
 #include "fstage_pass0.hpp"
@@ -44,7 +45,8 @@ struct BG {
 template <int L, bool CPLX>
 struct BLds {
   static constexpr int TAB = 4 * L;
-  static constexpr int LUT = TAB + TabGeom<L, CPLX>::NTAB * 8;
+  static constexpr int INC = TAB + TabGeom<L, CPLX>::NTAB * 8;
+  static constexpr int LUT = INC + (rho_in_passes<L>() ? kNumIncs * 8 : 0);
   static constexpr int STAGE = LUT + (CPLX ? 0 : 128);
   static constexpr int BYTES = STAGE + (CPLX ? 0 : L / 2);
   static_assert(MatLds<CPLX>::BYTES <= 4 * L, "M's operands fit the plane");
@@ -124,6 +126,7 @@ __device__ __forceinline__ void fstage_big_item(const FParams &p, int u, unsigne
   static_assert(!BOTH || !CPLX, "both polarisations in turn: 2-bit samples");
   float *splane = reinterpret_cast<float *>(smem);
   float2 *stab = reinterpret_cast<float2 *>(smem + LD::TAB);
+  float2 *sinc = reinterpret_cast<float2 *>(smem + LD::INC);
   uint2 *slut = reinterpret_cast<uint2 *>(smem + LD::LUT);
   uint32_t *stage = reinterpret_cast<uint32_t *>(smem + LD::STAGE);
 
@@ -164,6 +167,8 @@ __device__ __forceinline__ void fstage_big_item(const FParams &p, int u, unsigne
   Pass0In<L, CPLX, true, 4> in;
   in.template load<T>((gbyte *)p.station[st], offset, tid, tid);
   fill_tables<L, CPLX>(p, frac, a, b, stab, tid, T, pass0_unscale<CPLX>());
+  // by the second wave: the first has the tables' last entries
+  if (rho_in_passes<L>() && (unsigned)(tid - 64) < kNumIncs) sinc[tid - 64] = inc_entry(p, a, 1.0 / L, tid - 64);
   if (!CPLX && tid < 16) slut[tid] = level_pair(tid);
   in.template put<T>(stage, tid);
   __syncthreads();
@@ -238,7 +243,8 @@ __device__ __forceinline__ void fstage_big_item(const FParams &p, int u, unsigne
     get_plane<L, CPLX, CON_, 1>(v, splane, j);
     constexpr int TWS = f_tw_step(L, 2);
     static_assert(CON % TWS == 0 || CON == 1, "the first butterfly's powers are in the table");
-    last_butterflies<L, CPLX, CON_>(v, load_powers<RL, f_tw_entries(L, 2), f_tw_off(L, 2)>(tw, (unsigned)j * (CON / TWS)));
+    last_butterflies<L, CPLX, CON_>(
+        v, turn_powers<L>(load_powers<RL, f_tw_entries(L, 2), f_tw_off(L, 2)>(tw, (unsigned)j * (CON / TWS)), sinc + z));
 
     // outputs: bins q = CON (j + g T) + bf + k L/RL, q < nchan, CON neighbours
     // of a thread in one store

@@ -296,12 +296,45 @@ struct Pass0In {
   }
 };
 
-// Outputs r of columns j0 + e times rho of the column and pass 1's twiddle
-// W_1024^(r k1), k1 = (j0 + e) / TR the column's pass-1 input index, TR = L/1024.
+// rho_j of column j = TR k1 + b (TR = L/1024, b < TR) is sub[TR k1 % S2]
+// step[TR k1 / S2] times the rotator's turn over b samples.  Pass 1 runs over
+// k1 at one b, so the first factor joins pass 1's twiddle W_1024^(r k1), once
+// for the columns of a k1, and the second, kIncs[i] samples' turn, joins the
+// powers of the last pass's twiddle, which runs over b: one product per point
+// instead of two (8192 points, 16 stations: F-stage 5.98 -> 5.80 ms; 32768 complex
+// 1.43 -> 1.34 ms).  At 2048 points (TR = 2) a thread's four columns have two k1:
+// less is saved and 15 registers spill (6 stations: 2.26 -> 2.43 ms), so there
+// each column takes its whole rho.
+template <int L>
+constexpr bool rho_in_passes() { return L >= 4096; }
+constexpr int kNumIncs = 6;
+__device__ __forceinline__ int inc_samples(int i) { return i < 3 ? i + 1 : 4 << (i - 3); }  // 1, 2, 3, 4, 8, 16
+__device__ __forceinline__ float2 inc_entry(const FParams &p, double a, double over_l, int i) {
+#pragma clang fp contract(off)
+  const double ph = -((double)inc_samples(i) * over_l * a * p.lo);
+  float sn, cs;
+  sincospif((float)(2.0 * (ph - rint(ph))), &sn, &cs);
+  return make_float2(cs, sn);
+}
+template <int L>
+__device__ __forceinline__ Powers turn_powers(Powers w, const float2 *inc) {
+  constexpr int R = L / 1024;
+  if constexpr (!rho_in_passes<L>()) return w;
+  w.p1 = cmul(w.p1, inc[0]);
+  if constexpr (R > 2) w.p2 = cmul(w.p2, inc[1]), w.p3 = cmul(w.p3, inc[2]);
+  if constexpr (R > 4) w.q0 = cmul(w.q0, inc[3]);
+  if constexpr (R > 8) w.q1 = cmul(w.q1, inc[4]);
+  if constexpr (R > 16) w.q2 = cmul(w.q2, inc[5]);
+  return w;
+}
+
+// Outputs r of columns j0 + e times W_1024^(r k1) and rho (its first factor).
 template <int L, bool CPLX, int NT>
 __device__ __forceinline__ void finish_columns(floatx4 (&acc)[NT][2][2], const float2 *sub, const float2 *step,
                                                const float2 *__restrict__ tw, int j0, int g) {
   constexpr int S2 = TabGeom<L, CPLX>::S2, TR = L / 1024;
+  constexpr bool IN_PASSES = rho_in_passes<L>();
+  static_assert(S2 % TR == 0, "rho's factors");
   const unsigned char *wb = reinterpret_cast<const unsigned char *>(tw + 32);
   float2 pw[8];
 #pragma unroll
@@ -314,12 +347,19 @@ __device__ __forceinline__ void finish_columns(floatx4 (&acc)[NT][2][2], const f
         pw[2 * i] = make_float2(w.x, w.y);
         pw[2 * i + 1] = make_float2(w.z, w.w);
       }
+      if constexpr (IN_PASSES) {
+        const float2 rho = cmul(sub[k1 * TR % S2], step[k1 * TR / S2]);
+#pragma unroll
+        for (int i = 0; i < 8; i++) pw[i] = cmul(rho, pw[i]);
+      }
     }
-    const float2 rho = cmul(sub[(j0 + e) % S2], step[(j0 + e) / S2]);
+    float2 rho;
+    if constexpr (!IN_PASSES) rho = cmul(sub[(j0 + e) % S2], step[(j0 + e) / S2]);
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-      const float2 y = make_float2(acc[e][i >> 2][0][i & 3], acc[e][i >> 2][1][i & 3]);
-      const float2 x = cmul(cmul(y, rho), pw[i]);
+      float2 y = make_float2(acc[e][i >> 2][0][i & 3], acc[e][i >> 2][1][i & 3]);
+      if constexpr (!IN_PASSES) y = cmul(y, rho);
+      const float2 x = cmul(y, pw[i]);
       acc[e][i >> 2][0][i & 3] = x.x;
       acc[e][i >> 2][1][i & 3] = x.y;
     }

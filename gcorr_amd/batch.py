@@ -18,7 +18,7 @@ from .fxkernel import num_rows, station_bytes
 class Batch:
     """Batch(nant, [(nchan, numffts, lo, bw), ...]) over gxc_batch_*.
 
-    The subbands of 2048 points and more have an F-stage launch each:
+    Every subband has an F-stage launch: those of 2048 points and more with
     fstage_mfma 1 (True) on the matrix-core F-stage (f16 operands) where it
     covers the length, 0 (False) and 2 on a handle's default F-stage.
     autotune() chooses.

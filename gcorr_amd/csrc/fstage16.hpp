@@ -1,6 +1,5 @@
 // The F-stage for FFT lengths 64..1024 as a device function over one
-// workgroup's items (station, FFT), shared by the per-subband launch
-// (fstage.hip) and the multi-subband launch (fstage_multi.hip).
+// workgroup's items (station, FFT).
 //
 // Per item, fused so the packed samples are read once and the spectra
 // written once:

@@ -1,16 +1,16 @@
 // Multi-subband batch (include/gxcorr.h, gxc_batch_*): every subband of a
-// subintegration through one persistent launch per stage.
+// subintegration, the F-stage in a launch per subband, the other stages in one
+// launch for all.
 //
 // Device work of one subintegration:
 //   [H2D copies of host input, per subband]
 //   [reduced precision: power pass over 64 sampled FFTs of every subband
-//    (one launch), power-of-two scales (one launch)]
+//    (a launch each), power-of-two scales (one launch)]
 //   for each chunk c (1/chunks of every subband's FFTs):
-//     F-stage of the subbands below 2048 points (one launch) and of each
-//     longer one -> spectra buffer c % 2
+//     F-stage (a launch per subband) -> spectra buffer c % 2
 //     X-stage of all subbands (one launch), accumulating split partials
 //   row counts (one launch), finalise (one launch)
-// The launches read segment tables built once at gxc_batch_create: one
+// The launches for all subbands read segment tables built once at gxc_batch_create: one
 // entry per subband with its parameters and its first unit.
 #include <hip/hip_runtime.h>
 
@@ -83,17 +83,18 @@ struct gxc_batch {
   int2 *d_rowmap = nullptr;
   void *d_spec[2] = {nullptr, nullptr};
   // segment tables and unit totals
-  gxc::FSeg *d_fseg = nullptr;  // [nchunks][nmulti]: subbands of the multi-subband F launch
-  int nmulti = 0;
-  std::vector<std::vector<gxc::FSeg>> mseg;  // [nchunks]: subbands with launches of their own
-  std::vector<gxc::FSeg> mpow;               // the same subbands' power pass
+  struct FLaunch {  // one subband's F launch
+    gxc::FParams p;
+    int L;
+  };
+  std::vector<std::vector<FLaunch>> fseg;  // [nchunks][subband]
+  std::vector<FLaunch> fpow;               // [subband], the power pass
   gxc::XSeg *d_xseg = nullptr;  // [nchunks][nsub]
-  gxc::FSeg *d_powseg = nullptr;
   gxc::ScaleSeg *d_scaleseg = nullptr;
   gxc::CountSeg *d_countseg = nullptr;
   gxc::FinSeg *d_finseg = nullptr;
-  std::vector<long long> ftotal, xtotal;
-  long long powtotal = 0, scaletotal = 0, counttotal = 0, fintotal = 0;
+  std::vector<long long> xtotal;
+  long long scaletotal = 0, counttotal = 0, fintotal = 0;
   // profiling
   bool profiling = false;
   std::vector<hipEvent_t> tev;
@@ -211,50 +212,31 @@ int chunk_begin(const Sub &u, int c, int nchunks) {
 // Segment tables of every launch, from the handle's buffers (fixed for the
 // handle's lifetime: inputs and delays are reached through device arrays).
 gxc_status build_tables(gxc_batch *b) {
-  for (void *p : {(void *)b->d_fseg, (void *)b->d_xseg, (void *)b->d_countseg, (void *)b->d_finseg,
-                  (void *)b->d_powseg, (void *)b->d_scaleseg})
+  for (void *p : {(void *)b->d_xseg, (void *)b->d_countseg, (void *)b->d_finseg, (void *)b->d_scaleseg})
     hipFree(p);
-  b->d_fseg = nullptr;
   b->d_xseg = nullptr;
   b->d_countseg = nullptr;
   b->d_finseg = nullptr;
-  b->d_powseg = nullptr;
   b->d_scaleseg = nullptr;
   const int ns = (int)b->sub.size(), C = b->nchunks;
   const int ct = x_channels(b);
-  // The subbands of 2048 points and more get launches of their own: their
-  // kernel holds 32 points per thread and one length's LDS per workgroup, and
-  // in one persistent launch with the shorter lengths every workgroup would
-  // take the largest length's (8 subbands of 512..8192 points, FP32, 0.25 s:
-  // F-stage 12.4 -> 6.6 ms).  fstage_mfma 1 runs them with f16 operands in
-  // every pass where that form covers the length.
-  auto own_launch = [&](const Sub &u) { return u.d.L >= 2048; };
-  b->nmulti = 0;
-  for (const Sub &u : b->sub) b->nmulti += own_launch(u) ? 0 : 1;
-  b->mseg.assign(C, {});
-  std::vector<gxc::FSeg> fseg((size_t)C * std::max(1, b->nmulti));
+  // An F launch per subband: in one persistent launch of several FFT lengths
+  // every workgroup takes the largest length's registers and LDS (8 subbands of
+  // 512..8192 points, FP32, 0.25 s, F-stage 12.4 ms; with 2048 points and more
+  // apart 5.83, all apart 5.53; subbands of 20 ms the same either way).
+  // fstage_mfma 1 runs them with f16 operands in every pass where that form
+  // covers the length.
+  b->fseg.assign(C, {});
   std::vector<gxc::XSeg> xseg((size_t)C * ns);
-  b->ftotal.assign(C, 0);
   b->xtotal.assign(C, 0);
   for (int c = 0; c < C; c++) {
     const int buf = b->nbuf == 2 ? (c & 1) : 0;
-    long long fu = 0, xu = 0;
-    int m = 0;
+    long long xu = 0;
     for (int s = 0; s < ns; s++) {
       const Sub &u = b->sub[s];
       const int t0 = chunk_begin(u, c, C), nt = chunk_begin(u, c + 1, C) - t0;
       void *spec = static_cast<unsigned char *>(b->d_spec[buf]) + u.spec_off;
-      gxc::FSeg f;
-      f.p = fparams(b, u, t0, nt, 1, b->out_mode, spec);
-      f.L = u.d.L;
-      if (own_launch(u)) {
-        f.unit0 = 0;
-        b->mseg[c].push_back(f);
-      } else {
-        f.unit0 = fu;
-        fu += gxc::fstage_multi_units(u.d.L, (long long)b->cfg.nant * nt);
-        fseg[(size_t)c * b->nmulti + m++] = f;
-      }
+      b->fseg[c].push_back({fparams(b, u, t0, nt, 1, b->out_mode, spec), u.d.L});
       gxc::XSeg &x = xseg[(size_t)c * ns + s];
       x.p.spectra = spec;
       x.p.partial = u.d_partial;
@@ -271,10 +253,8 @@ gxc_status build_tables(gxc_batch *b) {
       x.unit0 = xu;
       xu += (long long)(u.cfg.nchan / ct) * u.splits;
     }
-    b->ftotal[c] = fu;
     b->xtotal[c] = xu;
   }
-  GXB_TRY(upload(b, &b->d_fseg, fseg));
   GXB_TRY(upload(b, &b->d_xseg, xseg));
 
   std::vector<gxc::CountSeg> cseg(ns);
@@ -310,23 +290,12 @@ gxc_status build_tables(gxc_batch *b) {
   GXB_TRY(upload(b, &b->d_finseg, finseg));
 
   if (b->out_mode != gxc::OUT_F32) {
-    std::vector<gxc::FSeg> pseg;
     std::vector<gxc::ScaleSeg> sseg(ns);
-    long long pu = 0, su = 0;
-    b->mpow.clear();
+    long long su = 0;
+    b->fpow.clear();
     for (int s = 0; s < ns; s++) {
       const Sub &u = b->sub[s];
-      gxc::FSeg f;
-      f.p = fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr);
-      f.L = u.d.L;
-      f.unit0 = 0;
-      if (own_launch(u)) {
-        b->mpow.push_back(f);
-      } else {
-        f.unit0 = pu;
-        pu += gxc::fstage_multi_units(u.d.L, (long long)b->cfg.nant * u.npow);
-        pseg.push_back(f);
-      }
+      b->fpow.push_back({fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr), u.d.L});
       sseg[s].scales = u.d_scales;
       sseg[s].power = u.d_power;
       sseg[s].n = b->M * u.cfg.nchan;
@@ -335,9 +304,7 @@ gxc_status build_tables(gxc_batch *b) {
       sseg[s].unit0 = su;
       su += (sseg[s].n + 255) / 256;
     }
-    b->powtotal = pu;
     b->scaletotal = su;
-    GXB_TRY(upload(b, &b->d_powseg, pseg));
     GXB_TRY(upload(b, &b->d_scaleseg, sseg));
   }
   return GXC_OK;
@@ -376,8 +343,7 @@ gxc_status enqueue_device_work(gxc_batch *b) {
   const bool overlap = b->nbuf == 2;
   hipStream_t fs = b->stream, xs = overlap ? b->xstream : b->stream;
   if (b->out_mode != gxc::OUT_F32) {
-    GXB_HIP(b, gxc::launch_fstage_multi(b->d_powseg, b->nmulti, b->powtotal, gxc::OUT_POWER, fs));
-    for (const gxc::FSeg &f : b->mpow)
+    for (const auto &f : b->fpow)
       GXB_HIP(b, gxc::launch_fstage(f.p, f.L, b->cfg.is_complex != 0, 0, fs));
     GXB_HIP(b, gxc::launch_scales_multi(b->d_scaleseg, ns, b->scaletotal, fs));
   }
@@ -389,9 +355,7 @@ gxc_status enqueue_device_work(gxc_batch *b) {
     const int buf = overlap ? (c & 1) : 0;
     if (overlap && c >= 2) GXB_HIP(b, hipStreamWaitEvent(fs, b->ev_x[buf], 0));
     mark(b, 0, fs);
-    if (b->nmulti > 0 && b->ftotal[c] > 0)
-      GXB_HIP(b, gxc::launch_fstage_multi(b->d_fseg + (size_t)c * b->nmulti, b->nmulti, b->ftotal[c], b->out_mode, fs));
-    for (const gxc::FSeg &f : b->mseg[c])
+    for (const auto &f : b->fseg[c])
       GXB_HIP(b, b->cfg.fstage_mfma == 1 &&
                          gxc::fstage_mfma_supported(f.L, b->cfg.is_complex != 0, b->out_mode == gxc::OUT_F32)
                      ? gxc::launch_fstage_mfma(f.p, f.L, fs)
@@ -704,9 +668,7 @@ void gxc_batch_destroy(gxc_batch *b) {
   b->out.release();
   for (void *p : b->d_spec) hipFree(p);
   hipFree(b->d_rowmap);
-  hipFree(b->d_fseg);
   hipFree(b->d_xseg);
-  hipFree(b->d_powseg);
   hipFree(b->d_scaleseg);
   hipFree(b->d_countseg);
   hipFree(b->d_finseg);
@@ -948,7 +910,7 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   b->graph_exec = nullptr;
   b->profiling = prof;
   if (st != GXC_OK) return st;
-  t.fblock = b->cfg.fstage_mfma == 1 ? gxc::kFBlockMfma : gxc::fstage_multi_block();
+  t.fblock = b->cfg.fstage_mfma == 1 ? gxc::kFBlockMfma : 256;  // the workgroup below 2048 points
   t.xtile = x_channels(b);
   t.xsplits = b->xunits;  // for a batch: the X units per launch the splits aim at
   t.graph = b->cfg.graph;

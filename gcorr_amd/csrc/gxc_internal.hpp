@@ -108,11 +108,6 @@ struct CountParams {
 
 // One subband's share of a multi-subband launch (units of segment k are
 // unit0[k] .. unit0[k+1]-1, segments in increasing unit0).
-struct FSeg {  // units = workgroups of the multi F launch for this subband
-  FParams p;
-  int L;
-  long long unit0;
-};
 struct CountSeg {  // units = nrows
   CountParams p;
   long long unit0;
@@ -142,11 +137,6 @@ constexpr int kFBlockMfma = -1;
 bool fstage_mfma_supported(int L, bool cplx, bool fp32);
 hipError_t launch_fstage_mfma(const FParams &p, int L, hipStream_t s);
 hipError_t launch_counts(const CountParams &p, hipStream_t s);
-// Multi-subband F-stage: real 2-bit input, FFT lengths 256..1024, workgroups
-// of fstage_multi_block() threads; units of a subband of `items` = nant * nt.
-int fstage_multi_block();
-long long fstage_multi_units(int L, long long items);
-hipError_t launch_fstage_multi(const FSeg *segs, int nseg, long long total, int out_mode, hipStream_t s);
 hipError_t launch_counts_multi(const CountSeg *segs, int nseg, long long total, hipStream_t s);
 
 }  // namespace gxc

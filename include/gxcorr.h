@@ -407,10 +407,9 @@ gxc_status gxc_get_timings(const gxc_handle *h, gxc_timings *t);
  * an observation with several subbands runs one object per subband.  A batch
  * holds every subband of a subintegration: the same stations, each subband
  * with its own channel count, bandwidth, LO, FFT count, delays and input.
- * Each stage runs for all subbands in one persistent launch (F-stage below
- * 2048 points, X-stage, row counts, finalise; longer FFTs have a launch per
- * subband), and with graph on the whole subintegration is captured as one
- * hipGraph.  Per subband the visibilities are those of a
+ * The F-stage has a launch per subband, every other stage (X-stage, row counts,
+ * finalise) one for all subbands, and with graph on the whole subintegration
+ * is captured as one hipGraph.  Per subband the visibilities are those of a
  * gxc_handle with the same settings (same layout, same normalisation).
  * Real 2-bit input, FFT lengths 2*nchan of 256..8192. */
 typedef struct {
@@ -483,7 +482,7 @@ gxc_status gxc_batch_get_row_counts(gxc_batch *b, int sub, int *counts, size_t n
  * subintegrations for each X unit count (512..8192, which sets every
  * subband's FFT splits) with either F-stage (gxc_batch_config.fstage_mfma 0
  * and 1), then with and without graph replay, and keeps the fastest.  In the
- * result, fblock is the multi-subband workgroup size, or GXC_FBLOCK_MFMA when
+ * result, fblock is 256, or GXC_FBLOCK_MFMA when
  * the matrix-core F-stage was chosen (the choice is kept in the batch);
  * xsplits holds the chosen X unit count and fstage_ms/xstage_ms are 0. */
 gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out);

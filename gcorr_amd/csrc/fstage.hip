@@ -1,4 +1,4 @@
-// Per-subband F-stage launch.  FFT lengths 64..1024 run fstage16_item
+// Per-subband F-stage launch.  FFT lengths 64..1024 (1024: complex) run fstage16_item
 // (fstage16.hpp), a workgroup of 256 threads per group of items (station,
 // FFT); longer FFTs go to fstage_big.hip.
 #include "fstage16.hpp"
@@ -78,6 +78,7 @@ hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStrea
   if (block == kFBlockMfma)
     return fstage_mfma_supported(L, cplx, p.out_mode == OUT_F32) ? launch_fstage_mfma(p, L, s) : hipErrorInvalidValue;
   if (f_matrix(L)) return launch_fstage_big(p, L, cplx, s);
+  if (fstage_one_wave(L, !cplx)) return launch_fstage_1k(p, s);
 #define GXC_F_CASE(LL) \
   case LL: return cplx ? launch_one<LL, true>(p, s) : launch_one<LL, false>(p, s);
   switch (L) {
@@ -85,7 +86,7 @@ hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStrea
     GXC_F_CASE(128)
     GXC_F_CASE(256)
     GXC_F_CASE(512)
-    GXC_F_CASE(1024)
+    case 1024: return launch_one<1024, true>(p, s);
     default: return hipErrorInvalidValue;
   }
 #undef GXC_F_CASE

@@ -104,17 +104,23 @@ gxc_status check_device(int *dev, std::string *why) {
 gxc_status upload_tables(const Derived &d, double bw, int nchan, float2 **twiddle, float **subfreq,
                          float **stepfreq, std::string *why) {
   const int L = d.L, s = d.g.s, nsf = d.g.fracsteps;
-  std::vector<float2> tw(f_tw_size(L));
+  const bool one_wave = fstage_one_wave(L, d.g.L != nchan);
+  std::vector<float2> tw(f_tw_size(L) + (one_wave ? 32 + 1024 : 0));
   auto w = [](long long m, int n) {  // exp(-2 pi i m / n)
     const double ang = -2.0 * kPi * (double)(m % n) / (double)n;
     return make_float2((float)std::cos(ang), (float)std::sin(ang));
   };
   for (int m = 0; m < 32; m++) tw[m] = w(m, 32);
-  if (f_matrix(L))
-    for (int k1 = 0; k1 < f_radix(L, 1); k1++)
+  auto put_w1024 = [&](int at) {
+    for (int k1 = 0; k1 < 32; k1++)
       for (int r = 0; r < 32; r++)
-        tw[32 + 2 * (((2 * (r / 16) + r / 2 % 2) * 4 + r / 4 % 4) * f_radix(L, 1) + k1) + r % 2] =
-            w((long long)k1 * r, 32 * f_radix(L, 1));
+        tw[at + 2 * (((2 * (r / 16) + r / 2 % 2) * 4 + r / 4 % 4) * 32 + k1) + r % 2] = w((long long)k1 * r, 1024);
+  };
+  if (f_matrix(L)) put_w1024(32);
+  if (one_wave) {
+    for (int m = 0; m < 32; m++) tw[f_tw_size(L) + m] = w(m, 32);
+    put_w1024(f_tw_size(L) + 32);
+  }
   for (int p = f_tw_first(L); p < f_npass(L); p++) {
     const int R = f_radix(L, p), ns = f_ns(L, p), n = f_tw_entries(L, p);
     for (int i = 0; i < f_npowers(R); i++)

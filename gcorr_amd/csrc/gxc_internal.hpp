@@ -63,6 +63,9 @@ constexpr int f_tw_off(int L, int p) {
                             : f_tw_off(L, p - 1) + f_npowers(f_radix(L, p - 1)) * f_tw_entries(L, p - 1);
 }
 constexpr int f_tw_size(int L) { return f_tw_off(L, f_npass(L)); }
+// Real input of 1024 points: a wave per (station, FFT), radices 32 * 32
+// (fstage_1k.hip); its W_32 and W_1024 follow the length's other tables.
+constexpr bool fstage_one_wave(int L, bool real) { return L == 1024 && real; }
 
 // What the F-stage writes per (station, FFT): FP32 spectra, scaled
 // reduced-precision spectra (complex: 2 x 16 bits or 2 x 8 bits), or |X|^2
@@ -130,6 +133,7 @@ int fstage_blocks(int L, bool cplx, int *out /* [4] */);
 // the length's one kernel
 hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s);
 hipError_t launch_fstage_big(const FParams &p, int L, bool cplx, hipStream_t s);  // L = 2048..32768
+hipError_t launch_fstage_1k(const FParams &p, hipStream_t s);                     // L = 1024, real
 // F-stage with the FFT passes on the matrix cores (fstage_mfma.hip): real
 // input; reduced-precision outputs (and the power pass) at L = 2048..8192,
 // FP32 spectra (operands as f16 hi + lo) at L = 2048..4096.

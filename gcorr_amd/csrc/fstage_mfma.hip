@@ -115,6 +115,42 @@ struct Split {
   double frac, a, b;
   int offset, valid;
 };
+// The item's tables of the reduced-precision forms, as fill_tables but with the
+// hardware's sine and cosine of FP32 radians: reduced arguments, within 5e-7 of
+// the exact values, against 2^-12 of the rounding to f16 that follows (16
+// stations x 4096 channels: F-stage 4.38 ms with fill_tables, 4.25 with this).
+template <int L>
+__device__ __forceinline__ void fill_tables_f16(const FParams &p, double frac, double a, double b, float2 *tab, int e0,
+                                                int estep) {
+#pragma clang fp contract(off)
+  using TG = TabGeom<L, false>;
+  constexpr int S = TG::S, S2 = TG::S2, NSTEPS = TG::NSTEPS;
+  const double intdelay = trunc(b);  // whole seconds removed, fxkernel.cpp:503-505
+  const float ffrac = (float)frac;   // fxkernel.cpp:600
+  for (int e = e0; e < TG::NTAB; e += estep) {
+    float arg;
+    if (e < S2 + NSTEPS) {
+      double ph;
+      if (e < S2) {  // subphase, fxkernel.cpp:107,508,514,519,525-530,535
+        ph = ((double)e / (double)L) * a;
+        ph = ph + (b - intdelay);
+        ph = ph * p.lo;
+        if (p.fraclo) ph = ph + p.lofrac * intdelay;
+      } else {  // stepphase, fxkernel.cpp:112,511,522,539
+        ph = ((double)((e - S2) * p.stepmul) / (double)L) * a;
+        ph = ph * p.lo;
+      }
+      arg = (float)((-2.0 * kPi) * (ph - trunc(ph)));
+    } else {  // fxkernel.cpp:600-611
+      const int i = e - S2 - NSTEPS;
+      arg = (i < S ? p.subchanfreq[i] : p.stepchanfreq[i - S]) * ffrac;
+    }
+    float sn, cs;
+    __sincosf(arg, &sn, &cs);
+    tab[e] = make_float2(cs, sn);
+  }
+}
+
 constexpr int kSplitBatch = 16;  // units whose splits one wave computes at once
 
 template <int L>
@@ -401,7 +437,10 @@ __global__ void __launch_bounds__(MG<L>::NTHR, 4) fstage_mfma_kernel(FParams p, 
       }
       continue;
     }
-    fill_tables<L, false>(p, frac, a, b, stab, tid, G::NTHR);
+    if constexpr (SPLIT)
+      fill_tables<L, false>(p, frac, a, b, stab, tid, G::NTHR);
+    else
+      fill_tables_f16<L>(p, frac, a, b, stab, tid, G::NTHR);
     __syncthreads();
 
     // The polarisations in turn, through the one buffer.

@@ -184,6 +184,7 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
 #pragma unroll
     for (int k = 0; k < 2; k++) {
       const int row = lrow + X::RPI * k * X::NWV;
+      // rowbytes < 2^24 (xsplit_channels), so at most 127 rows fit 31 bits
       const unsigned off = __umul24(row < last ? row : last, (unsigned)rowbytes) + 16u * pairq;
       if (k < nld)
         __builtin_amdgcn_global_load_lds((gvoid *)(base + off), (lvoid *)(d + 1024 * k * X::NWV), 16, 0, kNontemporal);
@@ -417,7 +418,10 @@ int xsplit_channels(int out_mode, int M, int nchan) {
   const int ct = out_mode == OUT_F32                        ? (M > 32 ? 16 : 32)
                  : out_mode == OUT_F16 || out_mode == OUT_BF16 ? (M > 32 ? 0 : 64)
                                                                : 0;
-  return ct && nchan % ct == 0 ? ct : 0;
+  // request()'s 24-bit products: rows of 2^24 bytes (2^22 channels of 16 bits,
+  // which a caller's spectra may have) and more go through xengine.hip
+  const bool fits = (long long)nchan * (out_mode == OUT_F32 ? 8 : 4) < 1 << 24;
+  return ct && nchan % ct == 0 && fits ? ct : 0;
 }
 
 // One workgroup per CU, which its LDS admits at 16, 32 and 64 inputs, where

@@ -120,7 +120,7 @@ def declared_functions():
 def row_pointers(a):
     """double *[] of the rows of a C-contiguous float64 matrix (by address: a
     ctypes view per row takes ~3 us)."""
-    base, step = a.ctypes.data, a.strides[0]
+    base, step = a.ctypes.data, a.shape[1] * a.itemsize  # one row has any first stride
     rows = (ctypes.c_void_p * a.shape[0])(*range(base, base + step * a.shape[0], step))
     return ctypes.cast(rows, ctypes.POINTER(ctypes.POINTER(ctypes.c_double)))
 

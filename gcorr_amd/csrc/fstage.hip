@@ -74,9 +74,9 @@ int fstage_blocks(int L, bool cplx, int *out) {
   return n;
 }
 
-hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s) {
-  if (block == kFBlockMfma)
-    return fstage_mfma_supported(L, cplx, p.out_mode == OUT_F32) ? launch_fstage_mfma(p, L, s) : hipErrorInvalidValue;
+namespace {
+
+hipError_t launch_piece(const FParams &p, int L, bool cplx, hipStream_t s) {
   if (f_matrix(L)) return launch_fstage_big(p, L, cplx, s);
   if (fstage_one_wave(L, !cplx)) return launch_fstage_1k(p, s);
 #define GXC_F_CASE(LL) \
@@ -90,6 +90,36 @@ hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStrea
     default: return hipErrorInvalidValue;
   }
 #undef GXC_F_CASE
+}
+
+}  // namespace
+
+int fstage_most_ffts(int L, int nant) {
+  const long long n = 0xff000000LL / ((long long)nant * (L / 8));
+  return (int)(n < 1 ? 1 : n > 0x7fffffff ? 0x7fffffff : n);
+}
+
+hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s) {
+  if (block == kFBlockMfma)
+    return fstage_mfma_supported(L, cplx, p.out_mode == OUT_F32) ? launch_fstage_mfma(p, L, s) : hipErrorInvalidValue;
+  const int most = fstage_most_ffts(L, p.nant);
+  FParams q = p;
+  for (int t = 0; t < p.nt || t == 0; t += q.nt) {
+    const size_t bin = (size_t)t * p.nant * 2 * (cplx ? L : L / 2);  // of the piece's first FFT
+    q.t0 = p.t0 + t * p.tstride;
+    q.nt = p.nt - t < most ? p.nt - t : most;
+    if (t > 0) {
+      if (p.out_mode == OUT_F32)
+        q.spectra = p.spectra + bin;
+      else if (p.out_mode == OUT_POWER)
+        q.power = p.power + bin;
+      else
+        q.out = static_cast<unsigned char *>(p.out) + bin * (p.out_mode == OUT_FP8 ? 2 : 4);
+    }
+    const hipError_t e = launch_piece(q, L, cplx, s);
+    if (e != hipSuccess || q.nt <= 0) return e;
+  }
+  return hipSuccess;
 }
 
 }  // namespace gxc

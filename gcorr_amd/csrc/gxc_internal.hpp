@@ -129,6 +129,11 @@ bool fstage_supported(int L, bool cplx);
 // F-stage workgroup sizes that gxc_config.fblock may name at FFT length L
 // (default first).
 int fstage_blocks(int L, bool cplx, int *out /* [4] */);
+// FFTs of nant stations that one launch takes at length L: a grid has fewer
+// than 2^32 work items, and the kernels at most L/8 per (station, FFT).  From
+// 2^32 on (32 stations x 64 points: 16.7 million FFTs) launch_fstage launches in
+// pieces.
+int fstage_most_ffts(int L, int nant);
 // block: kFBlockMfma, else one of fstage_blocks (0 = default), which all run
 // the length's one kernel
 hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s);

@@ -90,10 +90,17 @@ __global__ void __launch_bounds__(256) requant8_kernel(const float *__restrict__
 
 }  // namespace
 
+// (in pieces: a grid has fewer than 2^32 work items, 8 samples each)
 hipError_t launch_requant2(const float *a, const float *b, long long n, float t, uint8_t *out, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(requant2_kernel, dim3((unsigned)((n + kBlock2 - 1) / kBlock2)), dim3(256), 0, s, a, b, n, t, out);
-  return hipGetLastError();
+  constexpr long long kMost = 1LL << 34;
+  for (long long at = 0; at < n; at += kMost) {
+    const long long m = n - at < kMost ? n - at : kMost;
+    hipLaunchKernelGGL(requant2_kernel, dim3((unsigned)((m + kBlock2 - 1) / kBlock2)), dim3(256), 0, s, a + at, b + at,
+                       m, t, out + at / 2);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
 }
 
 hipError_t launch_requant8(const float *a, const float *b, long long n, float scale, uint8_t *out, hipStream_t s) {

@@ -38,8 +38,9 @@ hipError_t Mailbox::create(size_t in_bytes, size_t out_bytes) {
 
 hipError_t Mailbox::flush(hipStream_t s) {
   if (!dirty) return hipSuccess;
-  dirty = false;
-  return launch_copy(d, h, in, s);
+  const hipError_t e = launch_copy(d, h, in, s);
+  dirty = e != hipSuccess;
+  return e;
 }
 
 void Mailbox::release() {

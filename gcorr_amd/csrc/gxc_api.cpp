@@ -372,8 +372,10 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
   const int nant = cfg->nant, nchan = cfg->nchan;
   {
     const size_t ptrs = (size_t)nant * 4 * sizeof(double);  // after the delays
-    if (h->mail.create(ptrs + nant * sizeof(void *), d.nrows * (sizeof(int) + 4 * (sizeof(float) + sizeof(int)))) != hipSuccess ||
-        h->out.create((size_t)d.nrows * 4 * nchan * sizeof(float2)) != hipSuccess)
+    const size_t vis = (size_t)d.nrows * 4 * nchan * sizeof(float2);
+    if (h->mail.create(ptrs + nant * sizeof(void *), d.nrows * (sizeof(int) + 4 * (sizeof(float) + sizeof(int))),
+                       gxc::host::HostOut::bytes(vis)) != hipSuccess ||
+        h->out.create(h->mail.spare, vis) != hipSuccess)
       return fail(set_err(h, GXC_ERR_OUT_OF_MEMORY, "pinned host memory"));
     h->h_delays = reinterpret_cast<double *>(h->mail.h);
     h->d_delays = reinterpret_cast<double *>(h->mail.d);

@@ -596,8 +596,9 @@ gxc_status gxc_batch_create(const gxc_batch_config *cfg, gxc_batch **out) {
     const size_t ptrs = (size_t)nant * 4 * sizeof(double), per = ptrs + nant * sizeof(void *);
     size_t vis = 0;
     for (const Sub &u : b->sub) vis = std::max(vis, (size_t)b->nrows * 4 * u.cfg.nchan * sizeof(float2));
-    if (b->mail.create(b->sub.size() * per, b->sub.size() * b->nrows * sizeof(int)) != hipSuccess ||
-        b->out.create(vis) != hipSuccess)
+    if (b->mail.create(b->sub.size() * per, b->sub.size() * b->nrows * sizeof(int), gxc::host::HostOut::bytes(vis)) !=
+            hipSuccess ||
+        b->out.create(b->mail.spare, vis) != hipSuccess)
       return fail(set_err(b, GXC_ERR_OUT_OF_MEMORY, "pinned host memory"));
     size_t at = 0;
     int *counts = reinterpret_cast<int *>(b->mail.h + b->mail.in);

@@ -25,12 +25,13 @@ size_t round16(size_t n) { return (n + 15) / 16 * 16; }
 
 namespace host {
 
-hipError_t Mailbox::create(size_t in_bytes, size_t out_bytes) {
+hipError_t Mailbox::create(size_t in_bytes, size_t out_bytes, size_t spare_bytes) {
   in = round16(in_bytes);
   const size_t n = in + round16(out_bytes);
-  hipError_t e = hipHostMalloc((void **)&h, n, hipHostMallocDefault);
+  hipError_t e = hipHostMalloc((void **)&h, n + spare_bytes, hipHostMallocDefault);
   if (e != hipSuccess) return e;
   std::memset(h, 0, n);
+  spare = h + n;
   if ((e = hipMalloc((void **)&d, in)) != hipSuccess) return e;
   dirty = true;
   return hipSuccess;
@@ -46,12 +47,15 @@ hipError_t Mailbox::flush(hipStream_t s) {
 void Mailbox::release() {
   if (h) hipHostFree(h);
   hipFree(d);
-  h = d = nullptr;
+  h = d = spare = nullptr;
 }
 
-hipError_t HostOut::create(size_t largest) {
+size_t HostOut::bytes(size_t largest) { return largest > kChunk ? 2 * kChunk : round16(largest); }
+
+hipError_t HostOut::create(unsigned char *pinned, size_t largest) {
+  buf_ = pinned;
   chunk_ = std::min(round16(std::max<size_t>(largest, 1)), kChunk);
-  hipError_t e = hipHostMalloc((void **)&buf_, 2 * chunk_, hipHostMallocDefault);
+  hipError_t e = hipSuccess;
   for (hipEvent_t &ev : ev_)
     if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
   return e;
@@ -86,7 +90,6 @@ hipError_t HostOut::copy(void *dst, const void *src, size_t n, hipStream_t s) {
 }
 
 void HostOut::release() {
-  if (buf_) hipHostFree(buf_);
   for (hipEvent_t &ev : ev_)
     if (ev) hipEventDestroy(ev);
   buf_ = nullptr;

@@ -18,3 +18,11 @@ def test_a_failed_flush_keeps_the_parameters_pending():
     assert box.dirty
     box.dirty = False
     assert flush(ctypes.byref(box), None) == 0  # nothing to do
+
+
+def test_pinned_memory_of_a_readout():
+    """Nothing for no rows, one chunk for a copy of one, two for longer ones."""
+    size = ctypes.CDLL(gcorr_amd._lib.LIB_PATH)._ZN3gxc4host7HostOut5bytesEm
+    size.argtypes, size.restype = [ctypes.c_size_t], ctypes.c_size_t
+    assert [size(n) for n in (0, 48 << 10, 512 << 10, (512 << 10) + 32, 1 << 30)] == \
+        [0, 48 << 10, 512 << 10, 1 << 20, 1 << 20]

@@ -8,18 +8,6 @@ namespace {
 
 using namespace fs;
 
-// The workgroup sizes gxc_config.fblock names (0: not one for this length):
-// FFT blocks of L/16 threads, the default (256 threads or one block) times
-// mult / 2, as far as 1024 threads and a transform of both polarisations in
-// 160 KiB of LDS went.
-constexpr int fblock_for(int L, bool cplx, int mult) {
-  const int T = L / 16, def = T >= 256 ? T : 256, b = def * mult / 2;
-  if (b < T || b < 64 || b > 1024 || b % T) return 0;
-  const int nchan = cplx ? L : L / 2, sq = 1 << (ilog2c(nchan) / 2), s2 = cplx ? sq : 2 * sq;
-  const int slots = (b / T) * (2 * (L + L / 16) + s2 + L / s2 + sq + nchan / sq) + 16;
-  return slots * 8 > 160 * 1024 ? 0 : b;
-}
-
 // Items per workgroup of 256 threads.
 constexpr int f_ipw(int L) { return 2048 / L; }
 
@@ -61,16 +49,11 @@ bool fstage_supported(int L, bool cplx) {
 }
 
 int fstage_blocks(int L, bool cplx, int *out) {
-  if (L > 8192) {
-    out[0] = L / 32;  // one workgroup per (station, FFT, pol) in fstage_big.hip
-    return 1;
-  }
   int n = 0;
-  for (int mult : {2, 1, 4}) {  // default first
-    const int b = fblock_for(L, cplx, mult);
-    if (b) out[n++] = b;
-  }
-  if (L >= 2048) out[n++] = L / 32;
+  out[n++] = L <= 4096 ? 256 : L == 8192 ? 512 : L / 32;
+  if (L <= 2048) out[n++] = 128;
+  if (L <= 4096 && L >= (cplx ? 256 : 128)) out[n++] = 512;
+  if (L >= 2048 && L <= 8192) out[n++] = L / 32;
   return n;
 }
 

@@ -126,8 +126,10 @@ hipError_t allow_dynamic_lds(const void *kernel, int bytes);
 
 // Launchers (defined in the .hip files).  Return hipSuccess or the launch error.
 bool fstage_supported(int L, bool cplx);
-// F-stage workgroup sizes that gxc_config.fblock may name at FFT length L
-// (default first).
+// Values that gxc_config.fblock may have at FFT length L (default first): the
+// workgroup sizes of earlier kernels, which a tuning run may have written down.
+// They all run the length's one kernel, whose workgroup has 64 threads at 1024
+// real points, 256 at other lengths below 2048 and L/32 from there on.
 int fstage_blocks(int L, bool cplx, int *out /* [4] */);
 // FFTs of nant stations that one launch takes at length L: a grid has fewer
 // than 2^32 work items, and the kernels at most L/8 per (station, FFT).  From

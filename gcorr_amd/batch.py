@@ -163,7 +163,7 @@ class Batch:
         return out
 
     def autotune(self):
-        """gxc_batch_autotune: F workgroup size, X unit count (splits) and graph
+        """gxc_batch_autotune: F-stage kernel, X unit count (splits) and graph
         replay timed on this batch's input; the fastest is kept."""
         t = _lib.Tuning()
         check_batch(self._L.gxc_batch_autotune(self._h, ctypes.byref(t)), self._h)

@@ -878,9 +878,9 @@ gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out) {
   gxc_status st = time_process(b, &def_ms);
   cand++;
   int best_units = b->xunits, best_mfma = b->cfg.fstage_mfma;
-  bool any_mfma = false;  // a subband that the matrix-core F-stage covers
+  bool any_mfma = false;  // a subband that the matrix-core F-stage covers (reduced precision, as gxc_autotune)
   for (const Sub &u : b->sub)
-    any_mfma = any_mfma || gxc::fstage_mfma_supported(u.d.L, false, b->out_mode == gxc::OUT_F32);
+    any_mfma = any_mfma || (b->out_mode != gxc::OUT_F32 && gxc::fstage_mfma_supported(u.d.L, false, false));
   for (int mf = 0; mf <= (any_mfma ? 1 : 0); mf++)
     for (int f : {1, 2, 4, 8}) {
       const int units = f * x_units_min(b);

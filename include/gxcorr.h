@@ -358,15 +358,18 @@ gxc_status gxc_xengine_noalloc(const gxc_cf32 *d_spectra, int nant, int nchan, i
                                int autos, int precision, gxc_cf32 *d_vis, void *stream);
 
 /* Autotuner: with input and delays set, times the F-stage kernels that cover
- * the length, the X-stage at each channel
- * tile and split count, and whole subintegrations with and without graph
- * replay, on this handle's own data; keeps the fastest.  The choice is
- * returned (may be NULL) and applies to later gxc_process calls; it can be
+ * the length (FP32: its one kernel; GXC_FBLOCK_MFMA is slower there), the
+ * X-stage at each channel tile and split count, and whole subintegrations
+ * with and without graph replay, on this handle's own data; keeps the
+ * fastest.  The choice is returned (may be NULL) and applies to later gxc_process calls; it can be
  * given back through gxc_config.fblock/xtile/xsplits/graph of a new handle
  * with the same shape to skip the search.  No visibilities are kept from
  * the trial runs: call gxc_process afterwards. */
 typedef struct {
-  int fblock, xtile, xsplits, graph;  /* the choice */
+  /* The choice, as gxc_config takes it: where one kernel or one channel tile
+   * serves a shape, fblock and xtile are accepted values that name it, not its
+   * launch shape. */
+  int fblock, xtile, xsplits, graph;
   double fstage_ms, xstage_ms;        /* their times (all chunks of one subint) */
   double process_ms;                  /* one subintegration, as chosen */
   double default_ms;                  /* one subintegration at the defaults */
@@ -481,10 +484,10 @@ gxc_status gxc_batch_get_row_counts(gxc_batch *b, int sub, int *counts, size_t n
 /* Autotuner of a batch (input and delays of every subband set): times whole
  * subintegrations for each X unit count (512..8192, which sets every
  * subband's FFT splits) with either F-stage (gxc_batch_config.fstage_mfma 0
- * and 1), then with and without graph replay, and keeps the fastest.  In the
- * result, fblock is 256, or GXC_FBLOCK_MFMA when
- * the matrix-core F-stage was chosen (the choice is kept in the batch);
- * xsplits holds the chosen X unit count and fstage_ms/xstage_ms are 0. */
+ * and, reduced precision, 1), then with and without graph replay, and keeps
+ * the fastest.  In the result, fblock is 256, or GXC_FBLOCK_MFMA when the
+ * matrix-core F-stage was chosen (the choice is kept in the batch); xsplits
+ * holds the chosen X unit count and fstage_ms/xstage_ms are 0. */
 gxc_status gxc_batch_autotune(gxc_batch *b, gxc_tuning *out);
 
 /* Timing over all subbands (launch counts are per-stage launches, one per

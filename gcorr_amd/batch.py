@@ -18,9 +18,9 @@ from .fxkernel import num_rows, station_bytes
 class Batch:
     """Batch(nant, [(nchan, numffts, lo, bw), ...]) over gxc_batch_*.
 
-    Every subband has an F-stage launch: those of 2048 points and more with
-    fstage_mfma 1 (True) on the matrix-core F-stage (f16 operands) where it
-    covers the length, 0 (False) and 2 on a handle's default F-stage.
+    Subbands of one FFT length share an F-stage launch.  fstage_mfma 1 (True)
+    runs those of the lengths that the matrix-core F-stage (f16 operands) covers
+    on it, a launch each, 0 (False) and 2 on a handle's default F-stage.
     autotune() chooses.
     """
 

@@ -18,6 +18,32 @@ fstage_kernel(FParams p) {
   fstage16_item<L, CPLX, OUT, f_ipw(L)>(p, (int)xcd_order(blockIdx.x, gridDim.x), smem);
 }
 
+// Subbands of one length: units of f_ipw items, the last of a subband's partly
+// empty.
+template <int L, int OUT>
+__global__ void __launch_bounds__((2 * (L / 16) * f_ipw(L))) __attribute__((amdgpu_waves_per_eu(8)))
+fstage_group_kernel(const FSeg *__restrict__ segs, int nseg) {
+  __shared__ __align__(16) unsigned char smem[QLds<L, false, f_ipw(L)>::BYTES];
+  const long long u = xcd_order(blockIdx.x, gridDim.x);
+  const int k = find_fseg(segs, nseg, u);
+  const FParams p = segment_params(segs, k);
+  fstage16_item<L, false, OUT, f_ipw(L)>(p, (int)(u - segs[k].unit0), smem);
+}
+
+template <int L>
+hipError_t launch_group(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s) {
+  const dim3 grid((unsigned)units), block(2 * (L / 16) * f_ipw(L));
+  switch (out_mode) {
+    case OUT_F32: hipLaunchKernelGGL((fstage_group_kernel<L, OUT_F32>), grid, block, 0, s, segs, nseg); break;
+    case OUT_F16: hipLaunchKernelGGL((fstage_group_kernel<L, OUT_F16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_BF16: hipLaunchKernelGGL((fstage_group_kernel<L, OUT_BF16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_FP8: hipLaunchKernelGGL((fstage_group_kernel<L, OUT_FP8>), grid, block, 0, s, segs, nseg); break;
+    case OUT_POWER: hipLaunchKernelGGL((fstage_group_kernel<L, OUT_POWER>), grid, block, 0, s, segs, nseg); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <int L, bool CPLX, int OUT>
 hipError_t launch_out(const FParams &p, int items, hipStream_t s) {
   constexpr int IPW = f_ipw(L);
@@ -76,6 +102,22 @@ hipError_t launch_piece(const FParams &p, int L, bool cplx, hipStream_t s) {
 }
 
 }  // namespace
+
+long long fstage_units(int L, long long items) {
+  const int ipw = L < 1024 ? f_ipw(L) : 1;
+  return (items + ipw - 1) / ipw;
+}
+
+hipError_t launch_fstage_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s) {
+  if (units <= 0) return hipSuccess;
+  if (units > 0x7fffffffLL) return hipErrorInvalidValue;
+  switch (L) {
+    case 256: return launch_group<256>(segs, nseg, units, out_mode, s);
+    case 512: return launch_group<512>(segs, nseg, units, out_mode, s);
+    case 1024: return launch_fstage_1k_group(segs, nseg, units, out_mode, s);
+    default: return launch_fstage_big_group(segs, nseg, units, L, out_mode, s);
+  }
+}
 
 int fstage_most_ffts(int L, int nant) {
   const long long n = 0xff000000LL / ((long long)nant * (L / 8));

@@ -26,16 +26,15 @@ static_assert(T % TG::S2 == 0 && 16 % TG::S == 0, "table offsets");
 constexpr int kTab = 8 * L, kLut = kTab + TG::NTAB * 8, kStage = kLut + 128, kBytes = kStage + L / 2;
 static_assert(MatLds<false>::BYTES <= 8 * L, "M's operands fit the planes");
 
+// Item = station + nant * FFT; smem holds kBytes bytes, 16-byte aligned.
 template <int OUT>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) fstage_1k_kernel(FParams p) {
-  __shared__ __align__(16) unsigned char smem[kBytes];
+__device__ __forceinline__ void fstage_1k_item(const FParams &p, int item, unsigned char *smem) {
   float2 *sub = reinterpret_cast<float2 *>(smem + kTab), *step = sub + TG::S2;
   float2 *fsub = step + TG::NSTEPS, *fstep = fsub + TG::S;
   uint2 *slut = reinterpret_cast<uint2 *>(smem + kLut);
   uint32_t *stage = reinterpret_cast<uint32_t *>(smem + kStage);
   float *plane = reinterpret_cast<float *>(smem);
   const int lane = threadIdx.x;
-  const int item = (int)xcd_order(blockIdx.x, gridDim.x);  // grid = nant * nt exactly
   const int tl = item / p.nant, st = item - tl * p.nant, t = p.t0 + tl * p.tstride;
   constexpr unsigned EB = out_bytes(OUT);
   unsigned char *out = out_base<OUT>(p) + (size_t)item * 2 * (NCHAN * EB);
@@ -113,6 +112,23 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) fs
   }
 }
 
+template <int OUT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4))) fstage_1k_kernel(FParams p) {
+  __shared__ __align__(16) unsigned char smem[kBytes];
+  fstage_1k_item<OUT>(p, (int)xcd_order(blockIdx.x, gridDim.x), smem);  // grid = nant * nt exactly
+}
+
+// Several subbands: unit = item.
+template <int OUT>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(4)))
+fstage_1k_group_kernel(const FSeg *__restrict__ segs, int nseg) {
+  __shared__ __align__(16) unsigned char smem[kBytes];
+  const long long u = xcd_order(blockIdx.x, gridDim.x);
+  const int k = find_fseg(segs, nseg, u);
+  const FParams p = segment_params(segs, k);
+  fstage_1k_item<OUT>(p, (int)(u - segs[k].unit0), smem);
+}
+
 }  // namespace
 
 hipError_t launch_fstage_1k(const FParams &p, hipStream_t s) {
@@ -126,6 +142,19 @@ hipError_t launch_fstage_1k(const FParams &p, hipStream_t s) {
     case OUT_BF16: hipLaunchKernelGGL((fstage_1k_kernel<OUT_BF16>), grid, block, 0, s, p); break;
     case OUT_FP8: hipLaunchKernelGGL((fstage_1k_kernel<OUT_FP8>), grid, block, 0, s, p); break;
     case OUT_POWER: hipLaunchKernelGGL((fstage_1k_kernel<OUT_POWER>), grid, block, 0, s, p); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
+hipError_t launch_fstage_1k_group(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s) {
+  const dim3 grid((unsigned)units), block(64);
+  switch (out_mode) {
+    case OUT_F32: hipLaunchKernelGGL((fstage_1k_group_kernel<OUT_F32>), grid, block, 0, s, segs, nseg); break;
+    case OUT_F16: hipLaunchKernelGGL((fstage_1k_group_kernel<OUT_F16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_BF16: hipLaunchKernelGGL((fstage_1k_group_kernel<OUT_BF16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_FP8: hipLaunchKernelGGL((fstage_1k_group_kernel<OUT_FP8>), grid, block, 0, s, segs, nseg); break;
+    case OUT_POWER: hipLaunchKernelGGL((fstage_1k_group_kernel<OUT_POWER>), grid, block, 0, s, segs, nseg); break;
     default: return hipErrorInvalidValue;
   }
   return hipGetLastError();

@@ -27,6 +27,32 @@ fstage_big_kernel(FParams p) {
   fstage_big_item<L, CPLX, OUT, big_both<L, CPLX>()>(p, (int)xcd_order(blockIdx.x, gridDim.x), smem);
 }
 
+// Several subbands, real input: unit = item, both polarisations.
+template <int L, int OUT>
+__global__ void __launch_bounds__((BG<L, false>::T)) __attribute__((amdgpu_waves_per_eu(4)))
+fstage_big_group_kernel(const FSeg *__restrict__ segs, int nseg) {
+  static_assert(big_both<L, false>(), "unit = item");
+  __shared__ __align__(16) unsigned char smem[BLds<L, false>::BYTES];
+  const long long u = xcd_order(blockIdx.x, gridDim.x);
+  const int k = find_fseg(segs, nseg, u);
+  const FParams p = segment_params(segs, k);
+  fstage_big_item<L, false, OUT, true>(p, (int)(u - segs[k].unit0), smem);
+}
+
+template <int L>
+hipError_t launch_group(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s) {
+  const dim3 grid((unsigned)units), block(BG<L, false>::T);
+  switch (out_mode) {
+    case OUT_F32: hipLaunchKernelGGL((fstage_big_group_kernel<L, OUT_F32>), grid, block, 0, s, segs, nseg); break;
+    case OUT_F16: hipLaunchKernelGGL((fstage_big_group_kernel<L, OUT_F16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_BF16: hipLaunchKernelGGL((fstage_big_group_kernel<L, OUT_BF16>), grid, block, 0, s, segs, nseg); break;
+    case OUT_FP8: hipLaunchKernelGGL((fstage_big_group_kernel<L, OUT_FP8>), grid, block, 0, s, segs, nseg); break;
+    case OUT_POWER: hipLaunchKernelGGL((fstage_big_group_kernel<L, OUT_POWER>), grid, block, 0, s, segs, nseg); break;
+    default: return hipErrorInvalidValue;
+  }
+  return hipGetLastError();
+}
+
 template <int L, bool CPLX>
 hipError_t launch_big(const FParams &p, hipStream_t s) {
   using G = BG<L, CPLX>;
@@ -54,6 +80,15 @@ hipError_t launch_fstage_big(const FParams &p, int L, bool cplx, hipStream_t s) 
     case 8192: return cplx ? launch_big<8192, true>(p, s) : launch_big<8192, false>(p, s);
     case 16384: return cplx ? launch_big<16384, true>(p, s) : launch_big<16384, false>(p, s);
     case 32768: return cplx ? launch_big<32768, true>(p, s) : launch_big<32768, false>(p, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_fstage_big_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s) {
+  switch (L) {
+    case 2048: return launch_group<2048>(segs, nseg, units, out_mode, s);
+    case 4096: return launch_group<4096>(segs, nseg, units, out_mode, s);
+    case 8192: return launch_group<8192>(segs, nseg, units, out_mode, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -414,6 +414,44 @@ __device__ __forceinline__ long long xcd_order(long long v, long long total) {
   return (v % kXcdCount) * per + v / kXcdCount;
 }
 
+// Segment of a launch over several subbands that holds unit u.
+__device__ __forceinline__ int find_fseg(const FSeg *__restrict__ segs, int nseg, long long u) {
+  int a = 0;
+  for (int b = nseg; b - a > 1;) {
+    const int m = (a + b) / 2;
+    if (u >= segs[m].unit0)
+      a = m;
+    else
+      b = m;
+  }
+  return __builtin_amdgcn_readfirstlane(a);
+}
+
+// Parameters of segment k.  The compiler takes a kernel argument's pointers as
+// global memory, but those it loads from a table as generic ones (flat loads and
+// stores, and 12 registers spilled at 2048 points): each goes by the global
+// address space, from an integer, since a cast there and back is folded away.
+template <typename T>
+__device__ __forceinline__ T *as_global(T *p) {
+  return (T *)(__attribute__((address_space(1))) T *)reinterpret_cast<uintptr_t>(p);
+}
+__device__ __forceinline__ FParams segment_params(const FSeg *__restrict__ segs, int k) {
+  FParams p = segs[k].p;
+  p.station = as_global(p.station);
+  p.delays = as_global(p.delays);
+  p.subchanfreq = as_global(p.subchanfreq);
+  p.stepchanfreq = as_global(p.stepchanfreq);
+  p.twiddle = as_global(p.twiddle);
+  p.spectra = as_global(p.spectra);
+  p.out = as_global(p.out);
+  p.scales = as_global(p.scales);
+  p.power = as_global(p.power);
+  p.valid = as_global(p.valid);
+  p.frame_ok = as_global(p.frame_ok);
+  p.frame_samples = as_global(p.frame_samples);
+  return p;
+}
+
 // Global-address-space view of the packed station buffers: the loads then
 // use the global rather than the flat address path.
 typedef const __attribute__((address_space(1))) uint8_t gbyte;

@@ -1,5 +1,5 @@
 // Multi-subband batch (include/gxcorr.h, gxc_batch_*): every subband of a
-// subintegration, the F-stage in a launch per subband, the other stages in one
+// subintegration, the F-stage in a launch per FFT length, the other stages in one
 // launch for all.
 //
 // Device work of one subintegration:
@@ -7,7 +7,7 @@
 //   [reduced precision: power pass over 64 sampled FFTs of every subband
 //    (a launch each), power-of-two scales (one launch)]
 //   for each chunk c (1/chunks of every subband's FFTs):
-//     F-stage (a launch per subband) -> spectra buffer c % 2
+//     F-stage (a launch per FFT length) -> spectra buffer c % 2
 //     X-stage of all subbands (one launch), accumulating split partials
 //   row counts (one launch), finalise (one launch)
 // The launches for all subbands read segment tables built once at gxc_batch_create: one
@@ -83,12 +83,15 @@ struct gxc_batch {
   int2 *d_rowmap = nullptr;
   void *d_spec[2] = {nullptr, nullptr};
   // segment tables and unit totals
-  struct FLaunch {  // one subband's F launch
-    gxc::FParams p;
-    int L;
+  struct FLaunch {  // F launch of one subband (count 1) or several of one length
+    gxc::FParams p;   // of the first
+    int L, count;
+    size_t first;     // in d_fseg
+    long long units;
   };
-  std::vector<std::vector<FLaunch>> fseg;  // [nchunks][subband]
-  std::vector<FLaunch> fpow;               // [subband], the power pass
+  std::vector<std::vector<FLaunch>> fseg;  // [nchunks]
+  std::vector<FLaunch> fpow;               // the power pass
+  gxc::FSeg *d_fseg = nullptr;
   gxc::XSeg *d_xseg = nullptr;  // [nchunks][nsub]
   gxc::ScaleSeg *d_scaleseg = nullptr;
   gxc::CountSeg *d_countseg = nullptr;
@@ -209,23 +212,59 @@ int chunk_begin(const Sub &u, int c, int nchunks) {
   return (int)((long long)u.cfg.numffts * c / nchunks);
 }
 
+// F launches of subbands (parameters, FFT length), their segments appended to
+// `all`: one per length in the order of the subbands, or, matrix, one per subband
+// of the lengths that the matrix-core F-stage covers.
+std::vector<gxc_batch::FLaunch> f_launches(const gxc_batch *b, const std::vector<std::pair<gxc::FParams, int>> &subs,
+                                           bool matrix, std::vector<gxc::FSeg> *all) {
+  std::vector<gxc_batch::FLaunch> out;
+  std::vector<int> lengths;
+  for (const auto &s : subs)
+    if (std::find(lengths.begin(), lengths.end(), s.second) == lengths.end()) lengths.push_back(s.second);
+  for (int L : lengths) {
+    const bool own = matrix && gxc::fstage_mfma_supported(L, false, b->out_mode == gxc::OUT_F32);
+    long long ffts = 0;  // of the open launch
+    for (const auto &s : subs) {
+      if (s.second != L) continue;
+      const bool open = ffts > 0 && !own && ffts + s.first.nt <= gxc::fstage_most_ffts(L, s.first.nant);
+      if (!open) {
+        out.push_back({s.first, L, 0, all->size(), 0});
+        ffts = 0;
+      }
+      gxc_batch::FLaunch &f = out.back();
+      all->push_back({s.first, f.units});
+      f.count++;
+      f.units += gxc::fstage_units(L, (long long)s.first.nant * s.first.nt);
+      ffts += s.first.nt;
+    }
+  }
+  return out;
+}
+
 // Segment tables of every launch, from the handle's buffers (fixed for the
 // handle's lifetime: inputs and delays are reached through device arrays).
 gxc_status build_tables(gxc_batch *b) {
-  for (void *p : {(void *)b->d_xseg, (void *)b->d_countseg, (void *)b->d_finseg, (void *)b->d_scaleseg})
+  for (void *p : {(void *)b->d_fseg, (void *)b->d_xseg, (void *)b->d_countseg, (void *)b->d_finseg, (void *)b->d_scaleseg})
     hipFree(p);
+  b->d_fseg = nullptr;
   b->d_xseg = nullptr;
   b->d_countseg = nullptr;
   b->d_finseg = nullptr;
   b->d_scaleseg = nullptr;
   const int ns = (int)b->sub.size(), C = b->nchunks;
   const int ct = x_channels(b);
-  // An F launch per subband: in one persistent launch of several FFT lengths
-  // every workgroup takes the largest length's registers and LDS (8 subbands of
+  // An F launch per FFT length: in one persistent launch of several lengths
+  // every workgroup takes the largest one's registers and LDS (8 subbands of
   // 512..8192 points, FP32, 0.25 s, F-stage 12.4 ms; with 2048 points and more
-  // apart 5.83, all apart 5.53; subbands of 20 ms the same either way).
+  // apart 5.83, all apart 5.53), and a launch per subband costs 5 us and leaves
+  // a short subband's workgroups alone on the chip (4 stations, whole pass: 64
+  // subbands of 128 channels x 40 FFTs 0.42 ms apart, 0.12 together, FP8 0.76 and
+  // 0.16; 8 of 256 x 100 0.092 and 0.051; subbands of 4000 FFTs the same).
   // fstage_mfma 1 runs them with f16 operands in every pass where that form
-  // covers the length.
+  // covers the length, a subband a launch.
+  const bool matrix = b->cfg.fstage_mfma == 1;
+  std::vector<gxc::FSeg> all;
+  std::vector<std::pair<gxc::FParams, int>> subs(ns);
   b->fseg.assign(C, {});
   std::vector<gxc::XSeg> xseg((size_t)C * ns);
   b->xtotal.assign(C, 0);
@@ -236,7 +275,7 @@ gxc_status build_tables(gxc_batch *b) {
       const Sub &u = b->sub[s];
       const int t0 = chunk_begin(u, c, C), nt = chunk_begin(u, c + 1, C) - t0;
       void *spec = static_cast<unsigned char *>(b->d_spec[buf]) + u.spec_off;
-      b->fseg[c].push_back({fparams(b, u, t0, nt, 1, b->out_mode, spec), u.d.L});
+      subs[s] = {fparams(b, u, t0, nt, 1, b->out_mode, spec), u.d.L};
       gxc::XSeg &x = xseg[(size_t)c * ns + s];
       x.p.spectra = spec;
       x.p.partial = u.d_partial;
@@ -254,6 +293,7 @@ gxc_status build_tables(gxc_batch *b) {
       xu += (long long)(u.cfg.nchan / ct) * u.splits;
     }
     b->xtotal[c] = xu;
+    b->fseg[c] = f_launches(b, subs, matrix, &all);
   }
   GXB_TRY(upload(b, &b->d_xseg, xseg));
 
@@ -292,10 +332,9 @@ gxc_status build_tables(gxc_batch *b) {
   if (b->out_mode != gxc::OUT_F32) {
     std::vector<gxc::ScaleSeg> sseg(ns);
     long long su = 0;
-    b->fpow.clear();
     for (int s = 0; s < ns; s++) {
       const Sub &u = b->sub[s];
-      b->fpow.push_back({fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr), u.d.L});
+      subs[s] = {fparams(b, u, 0, u.npow, u.cfg.numffts / u.npow, gxc::OUT_POWER, nullptr), u.d.L};
       sseg[s].scales = u.d_scales;
       sseg[s].power = u.d_power;
       sseg[s].n = b->M * u.cfg.nchan;
@@ -305,9 +344,18 @@ gxc_status build_tables(gxc_batch *b) {
       su += (sseg[s].n + 255) / 256;
     }
     b->scaletotal = su;
+    b->fpow = f_launches(b, subs, false, &all);
     GXB_TRY(upload(b, &b->d_scaleseg, sseg));
   }
+  GXB_TRY(upload(b, &b->d_fseg, all));
   return GXC_OK;
+}
+
+hipError_t launch_f(const gxc_batch *b, const gxc_batch::FLaunch &f, bool matrix, hipStream_t s) {
+  if (matrix && gxc::fstage_mfma_supported(f.L, false, b->out_mode == gxc::OUT_F32))
+    return gxc::launch_fstage_mfma(f.p, f.L, s);
+  if (f.count == 1) return gxc::launch_fstage(f.p, f.L, false, 0, s);
+  return gxc::launch_fstage_group(b->d_fseg + f.first, f.count, f.units, f.L, f.p.out_mode, s);
 }
 
 // X splits per subband so that a launch has about b->xunits units, each
@@ -343,8 +391,7 @@ gxc_status enqueue_device_work(gxc_batch *b) {
   const bool overlap = b->nbuf == 2;
   hipStream_t fs = b->stream, xs = overlap ? b->xstream : b->stream;
   if (b->out_mode != gxc::OUT_F32) {
-    for (const auto &f : b->fpow)
-      GXB_HIP(b, gxc::launch_fstage(f.p, f.L, b->cfg.is_complex != 0, 0, fs));
+    for (const auto &f : b->fpow) GXB_HIP(b, launch_f(b, f, false, fs));
     GXB_HIP(b, gxc::launch_scales_multi(b->d_scaleseg, ns, b->scaletotal, fs));
   }
   if (overlap) {
@@ -355,11 +402,7 @@ gxc_status enqueue_device_work(gxc_batch *b) {
     const int buf = overlap ? (c & 1) : 0;
     if (overlap && c >= 2) GXB_HIP(b, hipStreamWaitEvent(fs, b->ev_x[buf], 0));
     mark(b, 0, fs);
-    for (const auto &f : b->fseg[c])
-      GXB_HIP(b, b->cfg.fstage_mfma == 1 &&
-                         gxc::fstage_mfma_supported(f.L, b->cfg.is_complex != 0, b->out_mode == gxc::OUT_F32)
-                     ? gxc::launch_fstage_mfma(f.p, f.L, fs)
-                     : gxc::launch_fstage(f.p, f.L, b->cfg.is_complex != 0, 0, fs));
+    for (const auto &f : b->fseg[c]) GXB_HIP(b, launch_f(b, f, b->cfg.fstage_mfma == 1, fs));
     mark(b, 1, fs);
     if (overlap) {
       GXB_HIP(b, hipEventRecord(b->ev_f[buf], fs));
@@ -669,6 +712,7 @@ void gxc_batch_destroy(gxc_batch *b) {
   b->out.release();
   for (void *p : b->d_spec) hipFree(p);
   hipFree(b->d_rowmap);
+  hipFree(b->d_fseg);
   hipFree(b->d_xseg);
   hipFree(b->d_scaleseg);
   hipFree(b->d_countseg);

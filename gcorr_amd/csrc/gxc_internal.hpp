@@ -111,6 +111,10 @@ struct CountParams {
 
 // One subband's share of a multi-subband launch (units of segment k are
 // unit0[k] .. unit0[k+1]-1, segments in increasing unit0).
+struct FSeg {  // subbands of one FFT length; units = fstage_units
+  FParams p;
+  long long unit0;
+};
 struct CountSeg {  // units = nrows
   CountParams p;
   long long unit0;
@@ -141,6 +145,13 @@ int fstage_most_ffts(int L, int nant);
 hipError_t launch_fstage(const FParams &p, int L, bool cplx, int block, hipStream_t s);
 hipError_t launch_fstage_big(const FParams &p, int L, bool cplx, hipStream_t s);  // L = 2048..32768
 hipError_t launch_fstage_1k(const FParams &p, hipStream_t s);                     // L = 1024, real
+// The F-stage of several subbands of one length in one launch, real input, L =
+// 256..8192.  Its work items, L/8 at most per (station, FFT), have to stay
+// below 2^32 (fstage_most_ffts).
+long long fstage_units(int L, long long items);
+hipError_t launch_fstage_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s);
+hipError_t launch_fstage_big_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s);
+hipError_t launch_fstage_1k_group(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s);
 // F-stage with the FFT passes on the matrix cores (fstage_mfma.hip): real
 // input; reduced-precision outputs (and the power pass) at L = 2048..8192,
 // FP32 spectra (operands as f16 hi + lo) at L = 2048..4096.

@@ -410,7 +410,7 @@ gxc_status gxc_get_timings(const gxc_handle *h, gxc_timings *t);
  * an observation with several subbands runs one object per subband.  A batch
  * holds every subband of a subintegration: the same stations, each subband
  * with its own channel count, bandwidth, LO, FFT count, delays and input.
- * The F-stage has a launch per subband, every other stage (X-stage, row counts,
+ * The F-stage has a launch per FFT length, every other stage (X-stage, row counts,
  * finalise) one for all subbands, and with graph on the whole subintegration
  * is captured as one hipGraph.  Per subband the visibilities are those of a
  * gxc_handle with the same settings (same layout, same normalisation).
@@ -438,12 +438,11 @@ typedef struct {
                                    within 32 GiB (eight with overlap) */
   int overlap;                  /* as gxc_config.overlap */
   int graph;                    /* as gxc_config.graph */
-  int fstage_mfma;              /* the subbands of 2048 points and more have a
-                                   launch each: 1 runs it on the matrix-core
-                                   F-stage (GXC_FBLOCK_MFMA) where that covers
-                                   the length, 0 and 2 on the F-stage of a
-                                   handle's default.  gxc_batch_autotune
-                                   chooses. */
+  int fstage_mfma;              /* 1: subbands of the lengths that the
+                                   matrix-core F-stage (GXC_FBLOCK_MFMA) covers
+                                   run on it, a launch each; 0 and 2: on the
+                                   F-stage of a handle's default.
+                                   gxc_batch_autotune chooses. */
   int reserved[3];
 } gxc_batch_config;
 

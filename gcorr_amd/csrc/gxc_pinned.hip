@@ -27,7 +27,7 @@ namespace host {
 
 hipError_t Mailbox::create(size_t in_bytes, size_t out_bytes, size_t spare_bytes) {
   in = round16(in_bytes);
-  const size_t n = in + round16(out_bytes);
+  const size_t n = (in + out_bytes + 4095) / 4096 * 4096;  // spare: whole pages
   hipError_t e = hipHostMalloc((void **)&h, n + spare_bytes, hipHostMallocDefault);
   if (e != hipSuccess) return e;
   std::memset(h, 0, n);

@@ -470,12 +470,24 @@ int xsplit_channels(int out_mode, int M, int nchan) {
 
 // One workgroup per CU, which its LDS admits at 16, 32 and 64 inputs, where
 // there are FFTs enough: 6 stations x 1024 channels 0.93 ms with 256
-// workgroups, 0.96 with 512; 16 x 4096 2.59 with 256, 2.64 with 1024.
+// workgroups, 0.96 with 512; 16 x 4096 2.59 with 256, 2.64 with 1024.  Short
+// subintegrations have fewer splits:
+//   a split saves its share of the loop and adds to the finalise's, ~M/9 FFTs'
+//   time each: the two meet at 3 sqrt(nt / M) splits;
+//   16 FFTs, a K-step, and as many bytes of spectra as of partials, at least;
+//   4 at a time, which the finalise has in flight together, and one rather than
+//   two unless they are long (its copy of one split is quicker).
+// FP32, whole pass with 1, 2, 4, 8, 16, 64 splits, the choice in brackets: 30
+// stations x 256 channels x 64 FFTs [67], 77, 71, 82 us; 30 x 256 x 500 209, 159,
+// 120, [114], 150; 16 x 128 x 500 169, 107, 76, 64, 67, [12: 66]; 3 x 32 x 5000 467, 255,
+// 147, 91, 63, 48, [84: 48], 156: 52.
 int xsplit_choose_splits(int out_mode, int M, int nchan, int nt) {
   const long long groups = nchan / std::max(1, xsplit_channels(out_mode, M, nchan));
-  long long s = (256 + groups - 1) / groups;
-  s = std::min<long long>(s, std::max(1, nt / 32));
-  return (int)std::max(1LL, std::min(s, 256LL));
+  const double most = std::min({256.0, 3 * std::sqrt((double)nt / M), nt / 16.0,
+                                nt * (double)xm_element_bytes(out_mode) / (8.0 * M)});
+  const int s = (int)std::max(1.0, std::min<double>((256 + groups - 1) / groups, most));
+  if (s >= 3) return (s + 1) / 4 * 4;
+  return s == 2 && nt < 8LL * M ? 1 : s;
 }
 
 // the largest |X| of an F-stage of L points is L times the largest sample

@@ -162,7 +162,7 @@ __device__ __forceinline__ void last16(const FParams &p, float2 (&v)[16], const 
                                                            : cmul(fsub[q % S], fstep[q / S]);
         float2 y = cmul(fr, v[BF * R + k]);
         if (!valid) y = make_float2(0.f, 0.f);
-        store_val<OUT>(out0 + (rowoff + (unsigned)q * EB), y, bin_scale<OUT, G::NCHAN>(p, srow, q));
+        store_val<OUT, (T * EB >= 64)>(out0 + (rowoff + (unsigned)q * EB), y, bin_scale<OUT, G::NCHAN>(p, srow, q));
       }
     }
     last16<L, CPLX, OUT, BF + 1>(p, v, w, j, fsub, fstep, out0, rowoff, srow, store, valid);

@@ -339,10 +339,19 @@ __device__ __forceinline__ unsigned char *out_base(const FParams &p) {
 // -> 2.78 ms, FP32 F-stage -0.8 %).  The 2-byte FP8 values keep ordinary
 // stores, which the caches combine (as streaming stores the 16-station FP8
 // F-stage measured 2-5 % slower).
-template <int OUT>
+// NT false: ordinary stores, which L2 combines to lines, where a store's
+// neighbouring lanes cover less than 64 bytes (8 stations, F-stage: 64 points,
+// FP32 235 -> 88 us, complex 287 -> 70; 128 points, FP16 142 -> 75, complex 162 ->
+// 52).  At 64 bytes (128 points, FP32) the F-stage takes 76 us either way, and the
+// X-stage behind ordinary stores 54 instead of 49.
+template <int OUT, bool NT = true>
 __device__ __forceinline__ void store_val(unsigned char *d, float2 y, float sc) {
   typedef float f32x2 __attribute__((ext_vector_type(2)));
-  if constexpr (OUT == OUT_F32) {
+  if constexpr (!NT && OUT == OUT_F32) {
+    *reinterpret_cast<f32x2 *>(d) = f32x2{y.x, y.y};
+  } else if constexpr (!NT && (OUT == OUT_F16 || OUT == OUT_BF16)) {
+    *reinterpret_cast<uint32_t *>(d) = OUT == OUT_F16 ? pack_f16(y.x * sc, y.y * sc) : pack_bf16(y.x * sc, y.y * sc);
+  } else if constexpr (OUT == OUT_F32) {
     const f32x2 v = {y.x, y.y};
     __builtin_nontemporal_store(v, reinterpret_cast<f32x2 *>(d));
   } else if constexpr (OUT == OUT_POWER) {

@@ -447,10 +447,11 @@ gxc_status gxc_create(const gxc_config *cfg, gxc_handle **out) {
     h->fblock = cfg->fblock;
     h->xtile = cfg->xtile;
   }
-  if (out_mode == gxc::OUT_F32) h->xscale = gxc::xsplit_scale(d.L, cfg->is_complex != 0);
-  h->splits = cfg->xsplits > 0        ? std::min(cfg->xsplits, h->chunk)
-              : out_mode == gxc::OUT_F32 ? gxc::xsplit_choose_splits(out_mode, d.M, nchan, h->chunk)
-                                         : gxc::xm_choose_splits(d.M, nchan, h->chunk, out_mode);
+  if (out_mode == gxc::OUT_F32 && gxc::xsplit_better(out_mode, d.M, nchan, h->chunk))
+    h->xscale = gxc::xsplit_scale(d.L, cfg->is_complex != 0);
+  h->splits = cfg->xsplits > 0  ? std::min(cfg->xsplits, h->chunk)
+              : h->xscale > 0.f ? gxc::xsplit_choose_splits(out_mode, d.M, nchan, h->chunk)
+                                : gxc::xm_choose_splits(d.M, nchan, h->chunk, out_mode);
   h->partial_cap = h->splits;
   if ((s = dmalloc(h, reinterpret_cast<unsigned char **>(&h->d_partial),
                    gxc::xm_partial_bytes(d.M, nchan, h->splits))) != GXC_OK)

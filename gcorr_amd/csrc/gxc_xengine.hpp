@@ -67,6 +67,9 @@ hipError_t launch_xmfma(const XMParams &p, int out_mode, int ct, hipStream_t s);
 // set).  xsplit_channels: the channels of its workgroup, 0 where it does not
 // cover the shape.
 int xsplit_channels(int out_mode, int M, int nchan);
+// Whether it is the quicker one for launches of nt FFTs, which launch_xmfma
+// (16-bit) and a handle (FP32) go by.
+bool xsplit_better(int out_mode, int M, int nchan, int nt);
 float xsplit_scale(int L, bool cplx);
 int xsplit_choose_splits(int out_mode, int M, int nchan, int nt);
 hipError_t launch_xsplit(const XMParams &p, int out_mode, hipStream_t s);

@@ -15,8 +15,9 @@
 // add a rounding).
 //
 // Runs here: FP8; FP16 and BF16 at 33 and more inputs (or a channel count that
-// is no multiple of 64); FP32 spectra that a caller hands in, of any magnitude.
-// xsplit.hip takes the rest in half to nine tenths of the time.
+// is no multiple of 64); FP32 spectra that a caller hands in, of any magnitude;
+// short subintegrations of 17 and more inputs (xsplit_better).  xsplit.hip takes
+// the rest in half to nine tenths of the time.
 //
 // The F-stage writes spectra channel-contiguous ([t][input][chan]), the
 // layout its last FFT pass stores coalesced.  Each workgroup stages a
@@ -743,7 +744,7 @@ int xm_channels_per_group(int M, int out_mode) {
 int xm_choose_splits(int M, int nchan, int nt, int out_mode) {
   const int ct = xm_channels_per_group(M, out_mode);
   if (ct == 0) return 1;
-  if (out_mode != OUT_F32 && xsplit_channels(out_mode, M, nchan)) return xsplit_choose_splits(out_mode, M, nchan, nt);
+  if (out_mode != OUT_F32 && xsplit_better(out_mode, M, nchan, nt)) return xsplit_choose_splits(out_mode, M, nchan, nt);
   const long long groups = nchan / ct;
   const int tb = out_mode == OUT_F32 ? 16 : 32;
   long long s = (1024 + groups - 1) / groups;  // ~4 workgroups per CU
@@ -767,7 +768,7 @@ float xm_target_rms(int out_mode) {
 }
 
 hipError_t launch_xmfma(const XMParams &p, int out_mode, int ct, hipStream_t s) {
-  if (out_mode != OUT_F32 && xsplit_channels(out_mode, p.M, p.nchan)) return launch_xsplit(p, out_mode, s);
+  if (out_mode != OUT_F32 && xsplit_better(out_mode, p.M, p.nchan, p.nt)) return launch_xsplit(p, out_mode, s);
   switch (out_mode) {
     case OUT_F32: return launch_xm_mb<OUT_F32>(p, ct, s);
     case OUT_F16: return launch_xm_mb<OUT_F16>(p, ct, s);

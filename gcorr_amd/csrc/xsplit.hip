@@ -468,26 +468,45 @@ int xsplit_channels(int out_mode, int M, int nchan) {
   return ct && nchan % ct == 0 && fits ? ct : 0;
 }
 
+// The general kernel has four to eight times the workgroups, each with a quarter
+// to an eighth of the channels, and wins where these cannot fill the chip and a
+// CU's own bandwidth binds.  At up to 16 inputs it wins nowhere.  X-stage and
+// finalise, general against streaming: FP32, 20 inputs, 2048 channels, 100 FFTs (33
+// MB of spectra) 37 : 41 us, 200 FFTs (66 MB) 56 : 49; 512 channels, 400 FFTs (33
+// MB) 40 : 43, 800 FFTs 51 : 49; 32 inputs, 512 x 400 (52 MB) 51 : 52, 512 x 800
+// 71 : 63; FP16, 32 inputs, 512 x 800 (52 MB) 51 : 58, 512 x 1600 76 : 73; 64 inputs,
+// FP32, 512 x 100 (26 MB) 67 : 70, 512 x 200 (52 MB) 91 : 74.  With 256 groups of
+// channels the chip is full at any length: 32 inputs, 8192 x 20 FP32 70 : 63.
+bool xsplit_better(int out_mode, int M, int nchan, int nt) {
+  const int ct = xsplit_channels(out_mode, M, nchan), mb = xm_blocks(M);
+  if (!ct || mb == 1) return ct != 0;
+  const double bytes = (double)nt * M * nchan * xm_element_bytes(out_mode);
+  return nchan / ct >= 256 || bytes >= (mb == 2 ? 56 << 20 : 32 << 20);
+}
+
 // One workgroup per CU, which its LDS admits at 16, 32 and 64 inputs, where
 // there are FFTs enough: 6 stations x 1024 channels 0.93 ms with 256
 // workgroups, 0.96 with 512; 16 x 4096 2.59 with 256, 2.64 with 1024.  Short
 // subintegrations have fewer splits:
 //   a split saves its share of the loop and adds to the finalise's, ~M/9 FFTs'
 //   time each: the two meet at 3 sqrt(nt / M) splits;
-//   16 FFTs, a K-step, and as many bytes of spectra as of partials, at least;
+//   with many channels the writing and reading of the partials adds more, 8 M^2
+//   bytes per channel at ~3 TB/s: they meet at 25 sqrt(nt / (nchan sqrt M));
+//   16 FFTs, a K-step, at least;
 //   4 at a time, which the finalise has in flight together, and one rather than
 //   two unless they are long (its copy of one split is quicker).
-// FP32, whole pass with 1, 2, 4, 8, 16, 64 splits, the choice in brackets: 30
-// stations x 256 channels x 64 FFTs [67], 77, 71, 82 us; 30 x 256 x 500 209, 159,
-// 120, [114], 150; 16 x 128 x 500 169, 107, 76, 64, 67, [12: 66]; 3 x 32 x 5000 467, 255,
-// 147, 91, 63, 48, [84: 48], 156: 52.
+// FP32, whole pass in us with 1, 2, 4, 8, 16, 64 splits, the choice in brackets: 30
+// stations x 256 channels x 500 FFTs 209, 159, 120, [114], 150; 8 x 512 x 200 58, 51,
+// 46, [44], 46; 24 x 1024 x 100 [91], 93, 86, 107; 3 x 32 x 5000 467, 255, 147, 91, 63,
+// [48], 256: 61.
 int xsplit_choose_splits(int out_mode, int M, int nchan, int nt) {
   const long long groups = nchan / std::max(1, xsplit_channels(out_mode, M, nchan));
-  const double most = std::min({256.0, 3 * std::sqrt((double)nt / M), nt / 16.0,
-                                nt * (double)xm_element_bytes(out_mode) / (8.0 * M)});
+  const double finalise = 3 * std::sqrt((double)nt / M);
+  const double partials = 25 * std::sqrt(nt / (nchan * std::sqrt((double)M)));
+  const double most = std::min({256.0, finalise, partials, nt / 16.0});
   const int s = (int)std::max(1.0, std::min<double>((256 + groups - 1) / groups, most));
   if (s >= 3) return (s + 1) / 4 * 4;
-  return s == 2 && nt < 8LL * M ? 1 : s;
+  return s == 2 && nt < 4LL * M ? 1 : s;
 }
 
 // the largest |X| of an F-stage of L points is L times the largest sample

@@ -1,8 +1,9 @@
 """What gxc_config.xsplits and xtile still vary.
 
-xsplits: the streaming X-stage with one split, odd counts and as many splits as
-FFTs (fewer than a stage each), FP32 against 64-bit sums of the handle's own
-spectra and 16-bit against one split of the same spectra.  The bound is that of
+xsplits: one split, odd counts and as many splits as FFTs (fewer than a stage
+each), FP32 against 64-bit sums of the handle's own spectra and 16-bit against
+one split of the same spectra (up to 16 inputs the streaming X-stage, above, at
+these sizes, the general one; test_gpu_xsplit_wide.py has the streaming one).  The bound is that of
 test_gpu_xsplit.py, 15 * 2^-24 of sqrt(V_aa V_bb): at most 7 K-steps of 16 FFTs
 (13 of 8) per split, splits summed with compensation.
 xtile: FP8, and FP16 and BF16 at 33 and more inputs, where it chooses among

@@ -15,10 +15,10 @@ def splits(mode, M, nchan, nt):
 
 @pytest.mark.parametrize("mode,M,nchan,nt,want", [
     (F32, 12, 1024, 62500, 8), (F32, 32, 4096, 15625, 2), (F32, 64, 1024, 6000, 4), (F32, 8, 128, 12500, 64),
-    (F16, 20, 2048, 5001, 8), (F16, 16, 32768, 1000, 1), (F32, 60, 256, 64, 1), (F32, 60, 256, 500, 8),
-    (F32, 32, 128, 500, 12), (F16, 32, 128, 500, 8), (F32, 6, 32, 5000, 84), (F32, 16, 256, 2000, 32),
+    (F16, 20, 2048, 5001, 8), (F16, 16, 32768, 1000, 1), (F32, 60, 256, 64, 4), (F32, 60, 256, 500, 8),
+    (F32, 32, 128, 500, 12), (F16, 32, 128, 500, 12), (F32, 6, 32, 5000, 84), (F32, 16, 256, 2000, 32),
     (F32, 24, 4096, 50, 1), (F32, 32, 2048, 60, 1), (F32, 2, 32, 1, 1), (F32, 2, 32, 17, 1), (F32, 6, 256, 64, 4),
-    (F16, 12, 1024, 200, 8), (F16, 32, 512, 200, 4), (F16, 16, 512, 200, 4), (F16, 24, 4096, 50, 1)])
+    (F16, 12, 1024, 200, 4), (F16, 32, 512, 200, 4), (F16, 16, 512, 200, 8), (F16, 24, 4096, 50, 1)])
 def test_choice(mode, M, nchan, nt, want):
     assert splits(mode, M, nchan, nt) == want
 

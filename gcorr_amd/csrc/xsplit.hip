@@ -19,13 +19,14 @@
 // 2-bit spectra are of rms sqrt(L) and more, scaled 54 and more, and lose
 // nothing by it.  Complex ones are of rms 1 where a window holds one sample of
 // one level: the loss is then 2^-25 / scale, and from 4096 points on (scale
-// below kLiftBelow) lo parts are kept times 2^11 (LIFT), their products summed
-// apart and taken down, which holds 24 bits down to 2^-4 of that weakest rms.
+// below kLiftBelow) lo parts are kept times 2^6 (LIFT), so that it is 2^-24 at
+// 32768 points.  A K-step's products with lo parts are taken down before they
+// join; where sums run on (64 inputs), the hi parts that meet lo parts are.
 // Errors of such visibilities against 64 bits with FP32 products, without LIFT
 // and with it: 2048 points 6.0e-7, 2.7e-7, -; 8192 points (10 stations) 8.0e-7,
 // 1.7e-6, 3.6e-7; 32768 points (8 stations) 8.8e-7, 7.6e-6, 4.1e-7.  X-stage in
 // the same order: 8 x 32768 x 1000 FFTs 0.78, 0.65, 0.66 ms; 12 x 16384 x 800
-// 0.68, 0.48, 0.54; 32 x 4096 x 1500 1.22, 0.61, 0.76.
+// 0.68, 0.48, 0.54; 32 x 4096 x 1500 1.22, 0.61, 0.70.
 // Spectra handed in by a caller have no such bound and take xengine.hip's FP32
 // products.
 //
@@ -68,8 +69,7 @@ constexpr int kNontemporal = 2;                               // cache policy of
 constexpr int kVmcnt(int n) { return 0x0f70 | (n & 15); }  // s_waitcnt vmcnt(n), n < 16
 
 
-// LIFT: lo parts times kLift (FP32 only).
-template <int ET, int MB, bool LIFT = false>
+template <int ET, int MB>
 struct XS {
   static constexpr bool F32 = ET == OUT_F32;
   static constexpr int CB = F32 ? 8 : 4;           // bytes of a complex value
@@ -82,10 +82,9 @@ struct XS {
   __device__ static constexpr int swz(int row) { return UPR == 8 ? (row >> 1) & 7 : row & 15; }
   static constexpr int SB = MB == 1 ? 8 : 4;   // FFTs per stage
   static constexpr int NU = SB / 4;            // a lane's units of an input and stage
-  // FFTs per MFMA: 16 (K = 32), or 8 (K = 16) where the running sums leave no
-  // registers for the operands of 16 (16-bit, 32 inputs: 96 sums of four
-  // channels; LIFT, 64 inputs: 80 and the sums of the lo parts)
-  static constexpr int KF = (!F32 && MB == 2) || (LIFT && MB == 4) ? 8 : 16, KD = KF / 4;
+  // FFTs per MFMA: 16 (K = 32), or 8 (K = 16) where the 96 running sums of four
+  // channels leave no registers for the operands of 16
+  static constexpr int KF = !F32 && MB == 2 ? 8 : 16, KD = KF / 4;
   static constexpr int NST = KF / SB;          // stages per MFMA K-step
   static constexpr int RING = 5;               // stages in LDS: 160 KiB at 16, 32 and 64 inputs
   static constexpr int NTILE = MB * (MB + 1) / 2;
@@ -121,8 +120,8 @@ __device__ __forceinline__ floatx4 mfma(const Op<2> &a, const Op<2> &b, floatx4 
 }
 
 // (re, im) * scale as an f16 pair and the f16 pair of the remainder (LIFT: times
-// kLift; at most half a unit of f16's largest values, 16, so 2^15)
-constexpr float kLift = 2048.f, kUnlift = 1.f / kLift;
+// kLift; at most half a unit of f16's largest values, 16, so 2^10)
+constexpr float kLift = 64.f, kUnlift = 1.f / kLift;
 constexpr float kLiftBelow = 0.125f;  // p.scale; real input has 0.5 and more
 template <bool LIFT>
 __device__ __forceinline__ void split(float re, float im, float scale, uint32_t &hi, uint32_t &lo) {
@@ -133,6 +132,17 @@ __device__ __forceinline__ void split(float re, float im, float scale, uint32_t 
   if constexpr (LIFT) d = {d.x * kLift, d.y * kLift};
   hi = __builtin_bit_cast(uint32_t, h);
   lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(d, half2v));
+}
+
+// an operand of hi parts for a product with lifted lo parts (and lo parts taken
+// down)
+template <int KD>
+__device__ __forceinline__ Op<KD> unlift(const Op<KD> &v) {
+  Op<KD> w;
+#pragma unroll
+  for (int i = 0; i < KD; i++)
+    w.d[i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(half2v, v.d[i]) * (half2v){(_Float16)kUnlift, (_Float16)kUnlift});
+  return w;
 }
 
 // [a, b] -> [-b, a]
@@ -177,7 +187,7 @@ __device__ __forceinline__ void read_blocks(floatx2 &a, floatx2 &b, floatx2 &c, 
 template <int ET, int MB, bool LIFT = false>
 __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int unit_split, unsigned char *lds) {
   const int group = __builtin_amdgcn_readfirstlane(group_), split_ = __builtin_amdgcn_readfirstlane(unit_split);
-  using X = XS<ET, MB, LIFT>;
+  using X = XS<ET, MB>;
   static_assert(X::F32 || !LIFT, "lo parts");
   constexpr int CPW = X::CPW, SB = X::SB, KD = X::KD;
   static_assert(X::F32 || X::ROWB == 256, "read_blocks");
@@ -293,43 +303,31 @@ __device__ __forceinline__ void xsplit_item(const XMParams &p, int group_, int u
           r[bi] = OWN ? floatx4{0, 0, 0, 0} : sr[bi];
           q[bi] = OWN ? floatx4{0, 0, 0, 0} : sq[bi];
         }
-        if constexpr (LIFT && !OWN) {
-          // the lo parts' products of one block, then the next: their sum is
-          // taken down by kLift before it joins the running sums
-          const Op<KD> wl = turn(L[c][bj]), wh = turn(H[c][bj]);
-#pragma unroll
-          for (int bi = 0; bi <= bj; bi++) {
-            floatx4 lr = {0, 0, 0, 0};
-            if (bi == bj) lr = mfma<ET>(L[c][bj], L[c][bj], lr) * kUnlift;
-            lr = mfma<ET>(L[c][bi], H[c][bj], mfma<ET>(H[c][bi], L[c][bj], lr));
-            floatx4 lq = mfma<ET>(L[c][bi], wh, mfma<ET>(H[c][bi], wl, floatx4{0, 0, 0, 0}));
-            sr[bi] = mfma<ET>(H[c][bi], H[c][bj], sr[bi]) + lr * kUnlift;
-            sq[bi] = mfma<ET>(H[c][bi], wh, sq[bi]) + lq * kUnlift;
-          }
-          __builtin_amdgcn_sched_barrier(0);
-          continue;
-        }
         if constexpr (X::F32) {
-          r[bj] = mfma<ET>(L[c][bj], L[c][bj], r[bj]);
-          if constexpr (LIFT) r[bj] *= kUnlift;
+          // LIFT: a K-step's own sums are taken down before the hi products
+          // join; running sums take lifted lo parts times hi parts taken down
+          constexpr bool DOWN = LIFT && !OWN;
+          const Op<KD> l = DOWN ? unlift(L[c][bj]) : L[c][bj];
+          r[bj] = mfma<ET>(l, l, r[bj]);
+          if constexpr (LIFT && OWN) r[bj] *= kUnlift;
           const Op<KD> w = turn(L[c][bj]);
 #pragma unroll
           for (int bi = 0; bi <= bj; bi++) {
-            r[bi] = mfma<ET>(H[c][bi], L[c][bj], r[bi]);
-            q[bi] = mfma<ET>(H[c][bi], w, q[bi]);
+            const Op<KD> h = DOWN ? unlift(H[c][bi]) : H[c][bi];
+            r[bi] = mfma<ET>(h, L[c][bj], r[bi]);
+            q[bi] = mfma<ET>(h, w, q[bi]);
           }
-        }
-        const Op<KD> w = turn(H[c][bj]);
-        if constexpr (X::F32) {
+          const Op<KD> h = DOWN ? unlift(H[c][bj]) : H[c][bj], wh = turn(h);
 #pragma unroll
           for (int bi = 0; bi <= bj; bi++) {
-            r[bi] = mfma<ET>(L[c][bi], H[c][bj], r[bi]);
-            q[bi] = mfma<ET>(L[c][bi], w, q[bi]);
+            r[bi] = mfma<ET>(L[c][bi], h, r[bi]);
+            q[bi] = mfma<ET>(L[c][bi], wh, q[bi]);
           }
-          if constexpr (LIFT)
+          if constexpr (LIFT && OWN)
 #pragma unroll
             for (int bi = 0; bi <= bj; bi++) r[bi] *= kUnlift, q[bi] *= kUnlift;
         }
+        const Op<KD> w = turn(H[c][bj]);
 #pragma unroll
         for (int bi = 0; bi <= bj; bi++) {
           r[bi] = mfma<ET>(H[c][bi], H[c][bj], r[bi]);

@@ -1,6 +1,7 @@
 // Device helpers shared by the F-stage kernels: fstage16.hpp (16 points per
-// thread, L = 64..1024), fstage_big.hpp (32 points per thread, L =
-// 2048..32768) and fstage_mfma.hip (all passes on the matrix cores).
+// thread, L = 64..1024), fstage_1k.hip (a wave per FFT pair, 1024 real points),
+// fstage_big.hpp (32 points per thread, L = 2048..32768) and fstage_mfma.hip
+// (all passes on the matrix cores).
 #pragma once
 
 #include "gxc_internal.hpp"
@@ -99,11 +100,6 @@ __device__ __forceinline__ void dft4(float2 &a0, float2 &a1, float2 &a2, float2 
   a2 = csub(t0, t2);
   a1 = cadd(t1, t3);
   a3 = csub(t1, t3);
-}
-
-template <int K>
-__device__ __forceinline__ float2 tw32(float2 a) {
-  return twc<32, K>(a);
 }
 
 // v[q] = e[q] + W32^q o[q], v[q + 16] = e[q] - W32^q o[q] for q = Q .. 15
@@ -464,7 +460,6 @@ __device__ __forceinline__ FParams segment_params(const FSeg *__restrict__ segs,
 // Global-address-space view of the packed station buffers: the loads then
 // use the global rather than the flat address path.
 typedef const __attribute__((address_space(1))) uint8_t gbyte;
-typedef const __attribute__((address_space(1))) int gint;
 
 }  // namespace fs
 }  // namespace gxc

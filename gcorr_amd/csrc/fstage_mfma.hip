@@ -2,8 +2,10 @@
 // (and the power pass) at FFT lengths 2048..8192, FP32 spectra at
 // 2048..4096.
 //
-// The FP32 F-stage issues about one VALU wave-instruction per sample and is
-// bound by that.  Here the radix passes run as MFMA products: a radix-R
+// The F-stage of fstage_big.hpp issues 0.68 VALU wave-instructions per sample
+// and is bound by them and by LDS.  Here all radix passes run as MFMA products
+// (0.36; its FP32 form, which carries hi and lo, is slower than that kernel: 1.77
+// against 1.13 ms at 2048 points, 3.89 against 2.07 at 4096): a radix-R
 // pass over columns b is Y[r'][b] = sum_r W_R^(r r') X[r][b], a real 16x16x32
 // f16 MFMA per 16 columns with the complex data interleaved along K (re, im
 // of 16 points), accumulated in FP32:
@@ -116,9 +118,12 @@ struct Split {
   int offset, valid;
 };
 // The item's tables of the reduced-precision forms, as fill_tables but with the
-// hardware's sine and cosine of FP32 radians: reduced arguments, within 5e-7 of
-// the exact values, against 2^-12 of the rounding to f16 that follows (16
-// stations x 4096 channels: F-stage 4.38 ms with fill_tables, 4.25 with this).
+// hardware's sine and cosine of FP32 radians.  The fringe phases are reduced to
+// one turn, the fractional-sample ones lie within one (frac within two samples):
+// rounding an angle to FP32 adds up to 2.4e-7, its conversion to turns up to
+// 3.7e-7, to the unit's own error, against 2^-12 (2.4e-4) of the rounding to f16
+// that follows (16 stations x 4096 channels: F-stage 4.38 ms with fill_tables,
+// 4.25 with this).
 template <int L>
 __device__ __forceinline__ void fill_tables_f16(const FParams &p, double frac, double a, double b, float2 *tab, int e0,
                                                 int estep) {

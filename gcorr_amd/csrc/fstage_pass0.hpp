@@ -1,6 +1,6 @@
 // First pass of the F-stage: packed samples to the outputs of one radix-32
-// pass on the matrix cores (FFT lengths of 2048 and more) or of one radix-16
-// pass on the VALU, and the twiddles of the later passes.
+// pass on the matrix cores (FFT lengths of 2048 and more, and 1024 real points)
+// or of one radix-16 pass on the VALU, and the twiddles of the later passes.
 #pragma once
 
 #include "fstage_common.hpp"

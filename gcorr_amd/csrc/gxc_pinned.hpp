@@ -32,9 +32,11 @@ struct Mailbox {
 };
 
 // Device-to-host copies into pageable memory through two pinned chunks: the
-// device fills one while the host empties the other (10 stations x 2048
-// channels, 3.6 MB of BF16 products, whole pass: 1070 -> 984 us; the runtime's
-// own staging fills and empties in turn).
+// device fills one while the host empties the other (the runtime's own staging
+// fills and empties in turn).  Visibilities of any size take them: the runtime's
+// copy -> this, into memory written before: 0.05 MB 28 -> 15 us, 0.33 MB (one
+// chunk, in turn here too) 23 -> 25, 3.6 MB 204 -> 131, 18 MB 1.04 -> 0.59 ms, 71 MB
+// 4.06 -> 3.64, 277 MB 15.7 -> 15.0; into fresh pages 277 MB 27 -> 20.
 class HostOut {
  public:
   static size_t bytes(size_t largest);  // of pinned memory for copies up to `largest` bytes

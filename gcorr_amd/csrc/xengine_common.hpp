@@ -1,5 +1,6 @@
-// Device helpers shared by the X-stage kernels: xengine.hip (spectra of any
-// format) and xsplit.hip (FP32 spectra of this build's own F-stage).
+// Device helpers shared by the X-stage kernels: xengine.hip (the general form)
+// and xsplit.hip (the streaming form: FP16 and BF16 spectra of up to 32 inputs,
+// FP32 spectra of the F-stage).
 #pragma once
 
 #include "gxc_xengine.hpp"

@@ -20,7 +20,7 @@
 // component plane at a time: 64 registers and 4.5 bytes of LDS per point, 8
 // waves per SIMD.  Against one thread per 16 points of both polarisations (3-4
 // waves): 32 stations x 1024 complex channels 1.15 -> 0.79 ms, 5 stations x 512
-// channels 0.42 -> 0.27 ms (before fstage_1k.hip took real input of 1024 points).
+// channels 0.42 -> 0.27 ms (before fstage_1k.hpp took real input of 1024 points).
 #pragma once
 
 #include "fstage_pass0.hpp"

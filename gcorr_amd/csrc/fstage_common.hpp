@@ -1,5 +1,5 @@
 // Device helpers shared by the F-stage kernels: fstage16.hpp (16 points per
-// thread, L = 64..1024), fstage_1k.hip (a wave per FFT pair, 1024 real points),
+// thread, L = 64..1024), fstage_1k.hpp (a wave per FFT pair, 1024 real points),
 // fstage_big.hpp (32 points per thread, L = 2048..32768) and fstage_mfma.hip
 // (all passes on the matrix cores).
 #pragma once

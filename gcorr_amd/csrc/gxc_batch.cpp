@@ -1,13 +1,13 @@
 // Multi-subband batch (include/gxcorr.h, gxc_batch_*): every subband of a
-// subintegration, the F-stage in a launch per FFT length, the other stages in one
-// launch for all.
+// subintegration, the F-stage in a launch per FFT length (one for all of short
+// subbands), the other stages in one launch for all.
 //
 // Device work of one subintegration:
 //   [H2D copies of host input, per subband]
 //   [reduced precision: power pass over 64 sampled FFTs of every subband
-//    (a launch each), power-of-two scales (one launch)]
+//    (launches as below), power-of-two scales (one launch)]
 //   for each chunk c (1/chunks of every subband's FFTs):
-//     F-stage (a launch per FFT length) -> spectra buffer c % 2
+//     F-stage (a launch per FFT length or one) -> spectra buffer c % 2
 //     X-stage of all subbands (one launch), accumulating split partials
 //   row counts (one launch), finalise (one launch)
 // The launches for all subbands read segment tables built once at gxc_batch_create: one
@@ -83,9 +83,9 @@ struct gxc_batch {
   int2 *d_rowmap = nullptr;
   void *d_spec[2] = {nullptr, nullptr};
   // segment tables and unit totals
-  struct FLaunch {  // F launch of one subband (count 1) or several of one length
+  struct FLaunch {  // F launch of one subband (count 1) or several
     gxc::FParams p;   // of the first
-    int L, count;
+    int L, count;     // L 0: several lengths
     size_t first;     // in d_fseg
     long long units;
   };
@@ -213,28 +213,43 @@ int chunk_begin(const Sub &u, int c, int nchunks) {
 }
 
 // F launches of subbands (parameters, FFT length), their segments appended to
-// `all`: one per length in the order of the subbands, or, matrix, one per subband
-// of the lengths that the matrix-core F-stage covers.
+// `all`: one per length in the order of the subbands, or one for all of them where
+// they are short together, and, matrix, one per subband of the lengths that the
+// matrix-core F-stage covers.
 std::vector<gxc_batch::FLaunch> f_launches(const gxc_batch *b, const std::vector<std::pair<gxc::FParams, int>> &subs,
                                            bool matrix, std::vector<gxc::FSeg> *all) {
-  std::vector<gxc_batch::FLaunch> out;
+  const auto own = [&](int L) { return matrix && gxc::fstage_mfma_supported(L, false, b->out_mode == gxc::OUT_F32); };
+  const auto units = [](const std::pair<gxc::FParams, int> &s) {
+    return gxc::fstage_units(s.second, (long long)s.first.nant * s.first.nt);
+  };
   std::vector<int> lengths;
-  for (const auto &s : subs)
-    if (std::find(lengths.begin(), lengths.end(), s.second) == lengths.end()) lengths.push_back(s.second);
+  int shared = 0;  // lengths without launches of their own
+  long long total = 0;
+  for (const auto &s : subs) {
+    if (!own(s.second)) total += units(s);
+    if (std::find(lengths.begin(), lengths.end(), s.second) != lengths.end()) continue;
+    lengths.push_back(s.second);
+    shared += !own(s.second);
+  }
+  const bool mixed = shared > 1 && total <= (long long)gxc::kFMixedUnits * (shared - 1);
+  if (mixed)
+    std::sort(lengths.begin(), lengths.end(),
+              [&](int x, int y) { return own(x) != own(y) ? own(y) : x > y; });
+  std::vector<gxc_batch::FLaunch> out;
   for (int L : lengths) {
-    const bool own = matrix && gxc::fstage_mfma_supported(L, false, b->out_mode == gxc::OUT_F32);
-    long long ffts = 0;  // of the open launch
+    long long ffts = 0;  // of the length's open launch
     for (const auto &s : subs) {
       if (s.second != L) continue;
-      const bool open = ffts > 0 && !own && ffts + s.first.nt <= gxc::fstage_most_ffts(L, s.first.nant);
+      const bool open = !own(L) && (mixed ? !out.empty()
+                                          : ffts > 0 && ffts + s.first.nt <= gxc::fstage_most_ffts(L, s.first.nant));
       if (!open) {
-        out.push_back({s.first, L, 0, all->size(), 0});
+        out.push_back({s.first, own(L) || !mixed ? L : 0, 0, all->size(), 0});
         ffts = 0;
       }
       gxc_batch::FLaunch &f = out.back();
-      all->push_back({s.first, f.units});
+      all->push_back({s.first, f.units, L});
       f.count++;
-      f.units += gxc::fstage_units(L, (long long)s.first.nant * s.first.nt);
+      f.units += units(s);
       ffts += s.first.nt;
     }
   }
@@ -259,7 +274,8 @@ gxc_status build_tables(gxc_batch *b) {
   // apart 5.83, all apart 5.53), and a launch per subband costs 5 us and leaves
   // a short subband's workgroups alone on the chip (4 stations, whole pass: 64
   // subbands of 128 channels x 40 FFTs 0.42 ms apart, 0.12 together, FP8 0.76 and
-  // 0.16; 8 of 256 x 100 0.092 and 0.051; subbands of 4000 FFTs the same).
+  // 0.16; 8 of 256 x 100 0.092 and 0.051; subbands of 4000 FFTs the same).  Short
+  // subbands of several lengths do share one launch (fstage_mixed.hip).
   // fstage_mfma 1 runs them with f16 operands in every pass where that form
   // covers the length, a subband a launch.
   const bool matrix = b->cfg.fstage_mfma == 1;
@@ -354,6 +370,7 @@ gxc_status build_tables(gxc_batch *b) {
 hipError_t launch_f(const gxc_batch *b, const gxc_batch::FLaunch &f, bool matrix, hipStream_t s) {
   if (matrix && gxc::fstage_mfma_supported(f.L, false, b->out_mode == gxc::OUT_F32))
     return gxc::launch_fstage_mfma(f.p, f.L, s);
+  if (f.L == 0) return gxc::launch_fstage_mixed(b->d_fseg + f.first, f.count, f.units, f.p.out_mode, s);
   if (f.count == 1) return gxc::launch_fstage(f.p, f.L, false, 0, s);
   return gxc::launch_fstage_group(b->d_fseg + f.first, f.count, f.units, f.L, f.p.out_mode, s);
 }

@@ -64,7 +64,7 @@ constexpr int f_tw_off(int L, int p) {
 }
 constexpr int f_tw_size(int L) { return f_tw_off(L, f_npass(L)); }
 // Real input of 1024 points: a wave per (station, FFT), radices 32 * 32
-// (fstage_1k.hip); its W_32 and W_1024 follow the length's other tables.
+// (fstage_1k.hpp); its W_32 and W_1024 follow the length's other tables.
 constexpr bool fstage_one_wave(int L, bool real) { return L == 1024 && real; }
 
 // What the F-stage writes per (station, FFT): FP32 spectra, scaled
@@ -111,9 +111,10 @@ struct CountParams {
 
 // One subband's share of a multi-subband launch (units of segment k are
 // unit0[k] .. unit0[k+1]-1, segments in increasing unit0).
-struct FSeg {  // subbands of one FFT length; units = fstage_units
+struct FSeg {  // units = fstage_units
   FParams p;
   long long unit0;
+  int L;
 };
 struct CountSeg {  // units = nrows
   CountParams p;
@@ -152,6 +153,10 @@ long long fstage_units(int L, long long items);
 hipError_t launch_fstage_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s);
 hipError_t launch_fstage_big_group(const FSeg *segs, int nseg, long long units, int L, int out_mode, hipStream_t s);
 hipError_t launch_fstage_1k_group(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s);
+// Subbands of several of these lengths in one launch, longest first
+// (fstage_mixed.hip): taken up to kFMixedUnits units per launch that it saves.
+constexpr int kFMixedUnits = 1500;
+hipError_t launch_fstage_mixed(const FSeg *segs, int nseg, long long units, int out_mode, hipStream_t s);
 // F-stage with the FFT passes on the matrix cores (fstage_mfma.hip): real
 // input; reduced-precision outputs (and the power pass) at L = 2048..8192,
 // FP32 spectra (operands as f16 hi + lo) at L = 2048..4096.

@@ -1,4 +1,5 @@
-"""Subbands of one FFT length share an F-stage launch.  The batch must give what a
+"""Subbands of one FFT length share an F-stage launch, and short ones of several
+lengths as well.  The batch must give what a
 batch of each subband alone gives, whose F-stage is a launch with one subband's
 parameters, bit for bit: FFT counts below 64 leave one X split either way.
 
@@ -60,5 +61,29 @@ def test_chunks_and_kernels(gpu, kw):
     got = correlate(3, subs, **kw)
     for i, s in enumerate(subs):
         (v, c), = correlate(3, [s], **kw)
+        assert np.array_equal(got[i][1], c)
+        assert np.array_equal(got[i][0].view(np.uint32), v.view(np.uint32)), s[0]
+
+
+@pytest.mark.parametrize("precision", ["fp32", "fp16", "fp8"])
+@pytest.mark.parametrize("nchan", [128, 256, 512, 1024, 2048, 4096])
+def test_one_length(gpu, precision, nchan):
+    """Subbands of one length only: the launch of that length."""
+    subs = inputs(5, [(nchan, 7), (nchan, 1), (nchan, 45), (nchan, 2)])
+    got = correlate(5, subs, precision=precision)
+    for i, s in enumerate(subs):
+        (v, c), = correlate(5, [s], precision=precision)
+        assert np.array_equal(got[i][1], c)
+        assert np.array_equal(got[i][0].view(np.uint32), v.view(np.uint32)), s[0]
+
+
+@pytest.mark.parametrize("nfft,kw", [(25, {}), (25, {"precision": "bf16"}), (26, {}), (26, {"graph": False})])
+def test_launch_limit(gpu, nfft, kw):
+    """Two lengths on both sides of 1500 units: 17 stations x (25 or 26 FFTs of
+    2048 points and 63 of 1024)."""
+    subs = inputs(17, [(1024, nfft), (512, 63)])
+    got = correlate(17, subs, **kw)
+    for i, s in enumerate(subs):
+        (v, c), = correlate(17, [s], **kw)
         assert np.array_equal(got[i][1], c)
         assert np.array_equal(got[i][0].view(np.uint32), v.view(np.uint32)), s[0]
